@@ -4,28 +4,31 @@
 // segment x + irep*N), SORT-Seq.cpp:31-42 (std::sort), SORT-Hip.cpp:35-43
 // (RAJA::sort on the device; the suite has no hand-written GPU sort).
 //
-// MI355X design: least-significant-digit radix sort over 8 passes of 8-bit
-// digits of an order-preserving 64-bit image of the double (sign bit set for
-// non-negative values, all bits flipped for negative ones), so unsigned order
-// is numeric order with -0.0 before +0.0.  Every segment is cut into tiles of
-// 2048 keys; each pass is three launches over all tiles of all segments:
-//   hist:    per-tile digit counts (LDS atomics) -> counts[seg][tile][digit]
-//   offsets: one workgroup per segment scans its counts digit-major, giving
-//            every (digit, tile) its output offset inside the segment (the
-//            tile-major layout makes each step's 256 loads one coalesced row)
-//   scatter: per tile, a stable rank of each key among equal digits (the
-//            lanes of a row with equal digits found through a per-wavefront
-//            LDS mask table, row by row, then a prefix over the wavefronts);
-//            the tile is first reordered by digit in LDS, then written out so
-//            that the keys of one digit go to consecutive addresses from
-//            consecutive work-items.
-// A wavefront owns 512 consecutive keys of its tile and reads them as 8
-// coalesced rows of 64, which keeps the ranking order equal to the tile order
-// (LSD stability).  2048-key tiles (22.5 KB of LDS, seven wavefronts per
-// SIMD), the mask table in place of 8 ballots per row, and a write-out that
-// reads all of a work-item's slots first took 256 ragged segments (35.8 M
-// keys) from 2.32 to 2.20 ms together; alone, each gained 1-2%.  Pass 0 converts doubles to keys on load; pass 7 converts
-// back on store.  The passes ping-pong between x and a scratch copy.
+// Keys are ordered by the 64-bit image of the double (sign bit set for
+// non-negative values, all bits flipped for negative ones), whose unsigned
+// order is numeric order with -0.0 before +0.0 and NaNs at the ends.  Equal
+// images are equal bit patterns, so the sort need not be stable.
+//
+// MI355X design: a sample sort.  A bucket of up to 4096 keys is sorted in
+// registers and LDS by one workgroup (bucket_kernel); a longer segment is
+// first cut into buckets of about 3000 keys by splitters taken from a sorted
+// random sample of it:
+//   sample:  one workgroup per segment sorts a sample, writes the splitters;
+//   hist:    every key's bucket (search over the splitters in LDS), kept as
+//            16 bits, and the bucket counts of each row of 4096-key tiles;
+//   colscan: each bucket's counts, scanned over the segment's rows;
+//   scatter: keys to their buckets, each tile grouped by bucket in LDS first;
+//   bucket:  every bucket (and every short segment) sorted.
+// So a key moves twice and is read once more, where a least-significant-digit
+// radix sort of 8-bit digits, which this replaces, moves it eight times and
+// reads it eight times more: 41.6 M keys in 256 ragged segments 2.30 -> 0.83
+// ms, one segment of 10^6 keys (24 launches then, 6 now) 0.30 -> 0.12 ms.
+// Segments above kOneLevel keys are cut twice, first into about
+// sqrt(n / 3072) parts.  Keys equal to a repeated splitter go round robin to
+// the buckets between its copies, which hold nothing else and are not sorted,
+// so equal keys cannot overfill a bucket.  A bucket that is overfull by bad
+// luck in the sample is sorted by big_kernel, of any length.
+#include <algorithm>
 #include <vector>
 
 #include "rpx_common.hpp"
@@ -34,91 +37,346 @@ using namespace rpx;
 
 namespace {
 
-constexpr int kBS = 256;
-constexpr int kRows = 8;
-constexpr int kTile = kBS * kRows;  // 2048 keys
-constexpr int kRadix = 256;
-constexpr int kPasses = 8;
-
 typedef unsigned long long u64;
 
-struct TileInfo {
-  long long seg_x;       // first key of the tile's segment in x
-  long long seg_alt;     // first key of the segment in the packed scratch copy
-  long long count_base;  // first counter of the segment
-  int len;               // keys in the tile
-  int local;             // tile index inside the segment
-  int ntiles;            // tiles of the segment
-  int seg_len;           // keys in the segment
+constexpr int kBS = 256;
+constexpr int kRows = 16;
+constexpr int kTile = kBS * kRows;  // 4096 keys per tile of hist and scatter
+constexpr int kBucket = 4096;       // keys bucket_kernel sorts
+constexpr int kAim = 3072;          // mean keys per bucket
+constexpr int kMaxK = 1024;         // buckets per segment and level
+constexpr int kCol = 64;            // buckets per workgroup of colscan
+constexpr int kBig = 8192;          // keys big_kernel sorts in one piece
+// Longest segment cut in one level: 512 buckets leave runs of 8 keys (64
+// bytes) per tile and bucket to write.
+constexpr long long kOneLevel = 512ll * kAim;
+
+// A segment at one level: keys [base, base + len) of x (src = 0) or of the
+// scratch copy (src = 1; both are indexed alike), cut into k buckets that
+// go to the other of the two.  k = 1: left where it is.
+struct Seg {
+  long long base, count_base;  // first key; first entry in the count table
+  int len, k, rows, first_row, first_bucket, first_col;
+  int src, pure;  // pure: all keys equal
 };
 
-struct SegInfo {
-  long long count_base;
-  int ntiles;
-  int pad;
+// Number of rows, buckets and column groups of a level whose segments were
+// found on the device, and the list of overfull buckets.
+struct Header {
+  int rows, buckets, cols, nbig;
 };
 
-// One per non-empty segment of a ragged layout, built on the host (O(nseg))
-// and expanded on the device into the per-tile TileInfo table.
-struct SegDesc {
-  long long seg_x, seg_alt, count_base;
-  int first_tile, ntiles, seg_len, pad;
+// One level.  segs = null: nseg segments of equal length from x[0], all
+// alike (`one` describes the first).
+struct Level {
+  const Seg* segs;
+  Seg one;
+  int nseg;
+  int chunk;  // tiles per row
+  const Header* bound;  // device counts, or null where the grid is exact
+  int* row_seg;
+  int* col_seg;
+  int* bucket_seg;   // null where every segment is one bucket
+  int* dup;          // per segment: a splitter is repeated
+  u64* splitters;    // [first_bucket + j], j < k - 1, ascending
+  unsigned* counts;  // [count_base + row * k + bucket]
+  unsigned* totals;  // [first_bucket + bucket]
+  unsigned* starts;  // first key of the bucket in its segment; top bit: pure
+  unsigned short* ids;
+  Header* header;
+  int* big;
 };
-
-// Uniform segmentation (equal lengths), or an explicit table in scratch.
-struct Plan {
-  const TileInfo* tiles;  // null => uniform
-  const SegInfo* segs;
-  long long seg_len;
-  int tiles_per_seg;
-};
-
-__device__ __forceinline__ TileInfo get_tile(const Plan& p, int t) {
-  if (p.tiles) return p.tiles[t];
-  TileInfo ti;
-  const int seg = t / p.tiles_per_seg;
-  ti.local = t % p.tiles_per_seg;
-  ti.ntiles = p.tiles_per_seg;
-  ti.seg_x = (long long)seg * p.seg_len;
-  ti.seg_alt = ti.seg_x;
-  const long long rem = p.seg_len - (long long)ti.local * kTile;
-  ti.len = int(rem < kTile ? rem : kTile);
-  ti.count_base = (long long)seg * p.tiles_per_seg * kRadix;
-  ti.seg_len = int(p.seg_len);
-  return ti;
-}
 
 __device__ __forceinline__ u64 to_key(u64 b) { return (b >> 63) ? ~b : (b | 0x8000000000000000ull); }
 __device__ __forceinline__ u64 from_key(u64 u) { return (u >> 63) ? (u & 0x7FFFFFFFFFFFFFFFull) : ~u; }
 
-__device__ __forceinline__ int tile_pos(int wave, int r, int lane) { return wave * (kRows * kWave) + r * kWave + lane; }
+__device__ __forceinline__ Seg get_seg(const Level& l, int s) {
+  if (l.segs) return l.segs[s];
+  Seg g = l.one;
+  g.base = (long long)s * g.len;
+  g.count_base = (long long)s * g.rows * g.k;
+  g.first_row = s * g.rows;
+  g.first_bucket = s * g.k;
+  g.first_col = s * ((g.k + kCol - 1) / kCol);
+  return g;
+}
 
-// Per-wavefront sub-histograms: a digit shared by many keys (the top byte
-// of doubles of one sign and binade) then contends within one wavefront only.
-__global__ __launch_bounds__(kBS) void hist_kernel(const u64* __restrict__ src, unsigned* __restrict__ counts, Plan plan,
-                                                   int shift, int convert, int src_is_x) {
-  __shared__ unsigned h[kBS / kWave][kRadix];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const TileInfo ti = get_tile(plan, xcd_major(blockIdx.x, gridDim.x));
-  const long long sbase = (src_is_x ? ti.seg_x : ti.seg_alt) + (long long)ti.local * kTile;
-#pragma unroll
-  for (int w = 0; w < kBS / kWave; ++w) h[w][tid] = 0u;
-  __syncthreads();
-  u64 k[kRows];
-#pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    const int p = tile_pos(wave, r, lane);
-    k[r] = p < ti.len ? src[sbase + p] : 0ull;
+__host__ __device__ inline int buckets_for(long long len, bool whole) {
+  if (len <= kBucket) return 1;
+  if (whole || len <= kOneLevel) {
+    const long long k = (len + kAim - 1) / kAim;
+    return int(k < kMaxK ? k : kMaxK);
   }
+  // Two levels: about sqrt(len / kAim) parts each.
+  int k = 2;
+  while ((long long)k * k * kAim < len && k < kMaxK) ++k;
+  return k;
+}
+
+// ---- sorting network in registers and LDS ------------------------------------
+//
+// 256 work-items sort N = 2^M = 256 R keys (M = 8 + RB, R = 2^RB per
+// work-item) with a bitonic network whose merges begin with the mirrored
+// comparison (i with i ^ (2^k - 1)), so every comparison is ascending.  A
+// work-item holds the R keys whose indexes differ in bits [LO, LO + RB) and
+// runs up to RB strides on registers before the keys change places through
+// LDS; element i lives at LDS slot i + i/R, which spreads every layout over
+// the banks.  A work-item writes only slots that it has itself just read, so
+// one barrier per exchange is enough, and none (an in-order LDS queue) while
+// the merged runs lie within one wavefront's 64 R keys.
+//
+// What bounds it: 1 VALU operation per key and stage (78 stages for 4096
+// keys) and 2 ceil(k/RB) LDS accesses per key and merge.  Keys are compared as
+// doubles, with one v_min_f64 and one v_max_f64 per pair where the integer
+// images would take a 64-bit compare and four selects: a negative double's
+// bit pattern is incremented first, which keeps the order, takes -0.0 away
+// from +0.0, and leaves out only NaNs and -inf.  A workgroup that
+// holds one of those sorts the images instead.  (The instructions are written
+// out because fmin/fmax quieten each operand with an extra v_max_f64 when it
+// comes from LDS.)
+struct AsDouble {
+  typedef double T;
+  static __device__ __forceinline__ void order(double& a, double& b) {
+    double lo, hi;
+    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+    a = lo;
+    b = hi;
+  }
+  static __device__ __forceinline__ double enter(u64 b) { return __longlong_as_double((long long)(b + (b >> 63))); }
+  static __device__ __forceinline__ u64 leave(double d) {
+    const u64 b = (u64)__double_as_longlong(d);
+    return b - (b >> 63);
+  }
+  static __device__ __forceinline__ double last() { return __longlong_as_double(0x7FF0000000000000ll); }
+};
+struct AsImage {
+  typedef u64 T;
+  static __device__ __forceinline__ void order(u64& a, u64& b) {
+    const bool swap = b < a;
+    const u64 lo = swap ? b : a, hi = swap ? a : b;
+    a = lo;
+    b = hi;
+  }
+  static __device__ __forceinline__ u64 enter(u64 b) { return to_key(b); }
+  static __device__ __forceinline__ u64 leave(u64 u) { return from_key(u); }
+  static __device__ __forceinline__ u64 last() { return ~0ull; }
+};
+// A bit pattern that AsDouble cannot order: NaN or -inf.
+__device__ __forceinline__ bool unordered(u64 b) { return b >= 0xFFF0000000000000ull || (b << 1) > (0x7FF0000000000000ull << 1); }
+
+template <class C, int RB>
+struct Net {
+  typedef typename C::T T;
+  static constexpr int R = 1 << RB, M = 8 + RB, N = 1 << M;
+  static constexpr int kSlots = N + N / R;
+
+  // LDS slot of element (hi, r, lo) of layout LO is base + offset(r).
+  template <int LO>
+  static __device__ __forceinline__ int base(int t, bool flip) {
+    const int mask = (1 << LO) - 1;
+    const int lo = (flip ? ~t : t) & mask;
+    const int i = ((t >> LO) << (LO + RB)) | lo;
+    return i + (i >> RB);
+  }
+  template <int LO>
+  static __device__ __forceinline__ constexpr int offset(int r) {
+    return (r << LO) + ((r << LO) >> RB);
+  }
+  // In layout LO > 0 of a merge's first exchange the upper half of the
+  // registers holds elements whose low index bits are complemented.
+  template <int LO, bool FLIP>
+  static __device__ __forceinline__ void get(T (&v)[R], const T* lds, int t) {
+    const int b0 = base<LO>(t, false), b1 = FLIP ? base<LO>(t, true) : b0;
 #pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    if (tile_pos(wave, r, lane) < ti.len) {
-      const u64 key = convert ? to_key(k[r]) : k[r];
-      atomicAdd(&h[wave][(key >> shift) & 0xFF], 1u);
+    for (int r = 0; r < R; ++r) v[r] = lds[(r < R / 2 ? b0 : b1) + offset<LO>(r)];
+  }
+  template <int LO, bool FLIP>
+  static __device__ __forceinline__ void put(const T (&v)[R], T* lds, int t) {
+    const int b0 = base<LO>(t, false), b1 = FLIP ? base<LO>(t, true) : b0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) lds[(r < R / 2 ? b0 : b1) + offset<LO>(r)] = v[r];
+  }
+  // Strides 2^S .. 1 of the register index.
+  template <int S>
+  static __device__ __forceinline__ void strides(T (&v)[R]) {
+    if constexpr (S >= 0) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if ((r & (1 << S)) == 0) C::order(v[r], v[r | (1 << S)]);
+      strides<S - 1>(v);
     }
   }
+  template <int K>
+  static __device__ __forceinline__ void mirror(T (&v)[R]) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if ((r & (1 << (K - 1))) == 0) C::order(v[r], v[r ^ ((1 << K) - 1)]);
+  }
+  template <int K>
+  static __device__ __forceinline__ void exchange_sync() {
+    if constexpr (K > 6 + RB) __syncthreads();
+    else {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+  }
+  // The strides of merge K below layout HI's, down to layout 0.
+  template <int K, int HI>
+  static __device__ __forceinline__ void descend(T (&v)[R], T* lds, int t) {
+    if constexpr (HI > 0) {
+      constexpr int LO = HI > RB ? HI - RB : 0;
+      exchange_sync<K>();
+      get<LO, false>(v, lds, t);
+      strides<HI - 1 - LO>(v);
+      if constexpr (LO > 0) put<LO, false>(v, lds, t);
+      descend<K, LO>(v, lds, t);
+    }
+  }
+  template <int K>
+  static __device__ __forceinline__ void merges(T (&v)[R], T* lds, int t) {
+    if constexpr (K <= RB) {
+      mirror<K>(v);
+      strides<K - 2>(v);
+      merges<K + 1>(v, lds, t);
+    } else if constexpr (K <= M) {
+      constexpr int LO = K - RB;
+      put<0, false>(v, lds, t);
+      exchange_sync<K>();
+      get<LO, true>(v, lds, t);
+      mirror<RB>(v);
+      strides<RB - 2>(v);
+      put<LO, true>(v, lds, t);
+      descend<K, LO>(v, lds, t);
+      merges<K + 1>(v, lds, t);
+    }
+  }
+  // v in any order -> v[r] = element R t + r of the sorted sequence; lds
+  // (kSlots values) is overwritten.
+  static __device__ __forceinline__ void sort(T (&v)[R], T* lds, int t) { merges<1>(v, lds, t); }
+
+  // Sorts src[0..len) into dst (which may be src), len <= N.
+  static __device__ __forceinline__ void sort_keys(const u64 (&b)[R], u64* dst, int len, void* mem, int t) {
+    T* lds = reinterpret_cast<T*>(mem);
+    T v[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = (r * kBS + t < len) ? C::enter(b[r]) : C::last();
+    sort(v, lds, t);
+    put<0, false>(v, lds, t);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = r * kBS + t;
+      if (i < len) dst[i] = C::leave(lds[i + (i >> RB)]);
+    }
+  }
+};
+
+constexpr int kBucketSlots = Net<AsDouble, 4>::kSlots;
+constexpr int kBigSlots = Net<AsDouble, 5>::kSlots;
+static_assert(Net<AsDouble, 4>::N == kBucket && Net<AsDouble, 5>::N == kBig, "network sizes");
+
+template <int RB>
+__device__ __forceinline__ bool load_keys(u64 (&b)[1 << RB], const u64* src, int len, int t) {
+  bool special = false;
+#pragma unroll
+  for (int r = 0; r < (1 << RB); ++r) {
+    const int i = r * kBS + t;
+    b[r] = i < len ? src[i] : 0ull;
+  }
+#pragma unroll
+  for (int r = 0; r < (1 << RB); ++r) special |= unordered(b[r]);
+  return special;
+}
+
+// src[0..len) -> dst sorted, len <= 256 << RB, with the images if need be.
+template <int RB>
+__device__ __forceinline__ void sort_piece(const u64* src, u64* dst, int len, void* mem, int t) {
+  u64 b[1 << RB];
+  const bool special = load_keys<RB>(b, src, len, t);
+  if (__syncthreads_or(special)) Net<AsImage, RB>::sort_keys(b, dst, len, mem, t);
+  else Net<AsDouble, RB>::sort_keys(b, dst, len, mem, t);
+}
+
+// ---- splitters -----------------------------------------------------------------
+
+// Sample of segment s, sorted, and every k-quantile of it as a splitter.
+// S = 2^M keys from S equal strata at pseudo-random places in them; at least
+// 16 per bucket for the most buckets, 32 and more otherwise (the spread of the
+// bucket sizes is 1/sqrt of that).
+template <class C, int RB>
+__device__ __forceinline__ void make_splitters(const u64 (&b)[1 << RB], const Seg& g, u64* splitters, int* dup,
+                                               void* mem, int t) {
+  typedef Net<C, RB> W;
+  typename C::T* lds = reinterpret_cast<typename C::T*>(mem);
+  typename C::T v[W::R];
+#pragma unroll
+  for (int r = 0; r < W::R; ++r) v[r] = C::enter(b[r]);
+  W::sort(v, lds, t);
+  W::template put<0, false>(v, lds, t);
   __syncthreads();
-  counts[ti.count_base + (long long)ti.local * kRadix + tid] = h[0][tid] + h[1][tid] + h[2][tid] + h[3][tid];
+  bool d = false;
+  for (int j = t + 1; j < g.k; j += kBS) {
+    auto quantile = [&](int q) {
+      const int i = q * W::N / g.k;  // q < 1024
+      return to_key(C::leave(lds[i + (i >> RB)]));
+    };
+    const u64 s = quantile(j);
+    splitters[j - 1] = s;
+    d |= j > 1 && s == quantile(j - 1);
+  }
+  const int any = __syncthreads_or(d);
+  if (t == 0) *dup = any;
+}
+
+template <int RB>
+__device__ __forceinline__ void sample_segment(const u64* src, const Seg& g, u64* splitters, int* dup, void* mem,
+                                               int t) {
+  constexpr int R = 1 << RB, S = 256 << RB;
+  u64 b[R];
+  bool special = false;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const u64 i = u64(r * kBS + t);
+    const u64 jitter = mix64(i * kGamma + u64(g.len)) >> 48;
+    b[r] = src[(i << 16 | jitter) * u64(g.len) >> (16 + 8 + RB)];  // (i + jitter 2^-16) len / S
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) special |= unordered(b[r]);
+  static_assert(S <= kBig, "sample fits the LDS");
+  if (__syncthreads_or(special)) make_splitters<AsImage, RB>(b, g, splitters, dup, mem, t);
+  else make_splitters<AsDouble, RB>(b, g, splitters, dup, mem, t);
+}
+
+// One workgroup per segment: its entries of the row, column and bucket maps,
+// and its splitters.
+__global__ __launch_bounds__(kBS) void sample_kernel(const u64* x, const u64* alt, Level l) {
+  __shared__ u64 mem[kBigSlots];
+  const int t = threadIdx.x, s = blockIdx.x;
+  if (s == 0 && t == 0) l.header->nbig = 0;
+  const Seg g = get_seg(l, s);
+  if (l.segs) {
+    for (int i = t; i < g.k; i += kBS) l.bucket_seg[g.first_bucket + i] = s;
+    if (g.k > 1) {
+      for (int i = t; i < g.rows; i += kBS) l.row_seg[g.first_row + i] = s;
+      for (int i = t; i < (g.k + kCol - 1) / kCol; i += kBS) l.col_seg[g.first_col + i] = s;
+    }
+  }
+  if (g.k <= 1) return;
+  const u64* src = (g.src ? alt : x) + g.base;
+  u64* sp = l.splitters + g.first_bucket;
+  // 2048 samples for up to 64 buckets, 8192 above.
+  if (g.k <= 64) sample_segment<3>(src, g, sp, l.dup + s, mem, t);
+  else sample_segment<5>(src, g, sp, l.dup + s, mem, t);
+}
+
+// ---- partition -----------------------------------------------------------------
+
+// Segment of row, column group or bucket i.
+__device__ __forceinline__ int seg_of(const Level& l, const int* map, int i, int per_seg) {
+  if (!l.segs) return i / per_seg;
+  return map ? map[i] : i;
 }
 
 // Exclusive scan over the 256 work-items of a workgroup (one value each).
@@ -137,257 +395,510 @@ __device__ __forceinline__ unsigned block_exclusive_scan(unsigned v, unsigned* w
   return run;
 }
 
-// One workgroup per segment: exclusive scan of counts in digit-major order.
-// kWalkers work-items share each digit: walker w of digit d visits the
-// segment's tiles [w*q, (w+1)*q), q = ceil(nt / kWalkers), in batches of
-// kBatch coalesced loads.  The largest segment's workgroup sets the kernel's
-// time, and its walk is kWalkers times shorter than with one work-item per
-// digit.  The walkers' sums give each digit's total (scanned over the
-// digits) and each walker's starting offset; the walkers then write their
-// tiles' offsets.
-constexpr int kBatch = 32;
-constexpr int kWalkers = 4;
-constexpr int kOffThreads = kWalkers * kRadix;
-__global__ __launch_bounds__(kOffThreads) void offsets_kernel(unsigned* __restrict__ counts, Plan plan) {
-  __shared__ unsigned part[kWalkers][kRadix];
-  __shared__ unsigned wsum[kRadix / kWave];
-  long long base;
-  int nt;
-  if (plan.segs) {
-    base = plan.segs[blockIdx.x].count_base;
-    nt = plan.segs[blockIdx.x].ntiles;
-  } else {
-    base = (long long)blockIdx.x * plan.tiles_per_seg * kRadix;
-    nt = plan.tiles_per_seg;
+// A row is `chunk` tiles.  The search runs over the splitters as a complete
+// binary tree in breadth-first order (missing ones above every key): a
+// level's nodes lie together, so the top five levels are free of bank
+// conflicts.
+__global__ __launch_bounds__(kBS) void hist_kernel(const u64* x, const u64* alt, Level l) {
+  __shared__ u64 tree[kMaxK];
+  __shared__ u64 sorted[kMaxK];
+  __shared__ unsigned cnt[kMaxK];
+  const int t = threadIdx.x;
+  const int row = int(xcd_major(blockIdx.x, gridDim.x));
+  if (l.bound && row >= l.bound->rows) return;
+  const int s = seg_of(l, l.row_seg, row, l.one.rows);
+  const Seg g = get_seg(l, s);
+  int depth = 1;
+  while ((1 << depth) < g.k) ++depth;
+  const u64* sp = l.splitters + g.first_bucket;
+  for (int j = t; j < (1 << depth); j += kBS) {
+    const u64 v = j < g.k - 1 ? sp[j] : ~0ull;
+    sorted[j] = v;
+    cnt[j] = 0u;
+    const int z = __ffs(j + 1) - 1;  // node of rank j: 2^z divides j + 1
+    if (j + 1 < (1 << depth)) tree[(1 << (depth - 1 - z)) - 1 + ((j + 1) >> (z + 1))] = v;
   }
-  const int d = threadIdx.x % kRadix, w = threadIdx.x / kRadix;  // w is wavefront-uniform
-  const int q = (nt + kWalkers - 1) / kWalkers;
-  const int t0 = w * q < nt ? w * q : nt;
-  const int t1 = (w + 1) * q < nt ? (w + 1) * q : nt;
-  unsigned* col = counts + base + d;  // col[t * kRadix]: digit d of tile t
-  unsigned s = 0;
-  int t = t0;
-  for (; t + kBatch <= t1; t += kBatch) {
+  const bool dup = l.dup[s] != 0;
+  __syncthreads();
+  const long long local0 = (long long)(row - g.first_row) * l.chunk * kTile;
+  const u64* src = (g.src ? alt : x) + g.base;
+  unsigned short* ids = l.ids + g.base;
+  for (int c = 0; c < l.chunk; ++c) {
+    const long long first = local0 + (long long)c * kTile;
+    if (first >= g.len) break;
+    const int n = int(g.len - first < kTile ? g.len - first : kTile);
+    u64 k[kRows];
+    int node[kRows];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      const int i = r * kBS + t;
+      k[r] = i < n ? to_key(src[first + i]) : 0ull;
+      node[r] = 0;
+    }
+    for (int d = 0; d < depth; ++d) {
+#pragma unroll
+      for (int r = 0; r < kRows; ++r) node[r] = 2 * node[r] + 1 + (tree[node[r]] < k[r] ? 1 : 0);
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      const int i = r * kBS + t;
+      int b = node[r] - ((1 << depth) - 1);  // splitters below the key: at most k - 1
+      if (dup && b < g.k - 1 && sorted[b] == k[r]) {
+        // Equal to splitters b .. b + run - 1: any bucket b .. b + run will
+        // do; between two copies it holds this value only.
+        int lo = b + 1, hi = g.k - 1;  // the first splitter above the key
+        while (lo < hi) {
+          const int m = (lo + hi) >> 1;
+          if (sorted[m] == k[r]) lo = m + 1;
+          else hi = m;
+        }
+        const int run = lo - b;
+        const unsigned h = unsigned(mix64(u64(first + i) * kGamma) >> 32);
+        b += run == 1 ? int(h & 1u) : 1 + int((u64(h) * unsigned(run - 1)) >> 32);
+      }
+      if (i < n) {
+        atomicAdd(&cnt[b], 1u);
+        ids[first + i] = (unsigned short)b;
+      }
+    }
+  }
+  __syncthreads();
+  unsigned* out = l.counts + g.count_base + (long long)(row - g.first_row) * g.k;
+  for (int j = t; j < g.k; j += kBS) out[j] = cnt[j];
+}
+
+// kCol buckets of one segment: exclusive scan of their counts over the rows
+// (16 walkers per bucket, each over a sixteenth of the rows), and totals.
+constexpr int kWalkers = 16;
+__global__ __launch_bounds__(kCol* kWalkers) void colscan_kernel(Level l) {
+  __shared__ unsigned part[kWalkers][kCol];
+  const int col = blockIdx.x;
+  if (l.bound && col >= l.bound->cols) return;
+  const int s = seg_of(l, l.col_seg, col, (l.one.k + kCol - 1) / kCol);
+  const Seg g = get_seg(l, s);
+  const int lane = threadIdx.x % kCol, w = threadIdx.x / kCol;
+  const int b = (col - g.first_col) * kCol + lane;
+  const bool live = b < g.k;
+  const int q = (g.rows + kWalkers - 1) / kWalkers;
+  const int r0 = w * q < g.rows ? w * q : g.rows;
+  const int r1 = (w + 1) * q < g.rows ? (w + 1) * q : g.rows;
+  unsigned* at = l.counts + g.count_base + b;
+  constexpr int kBatch = 16;
+  unsigned sum = 0;
+  if (live) {
+    int r = r0;
+    for (; r + kBatch <= r1; r += kBatch) {
+      unsigned v[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) v[u] = at[(long long)(r + u) * g.k];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) sum += v[u];
+    }
+    for (; r < r1; ++r) sum += at[(long long)r * g.k];
+  }
+  part[w][lane] = sum;
+  __syncthreads();
+  unsigned run = 0, total = 0;
+#pragma unroll
+  for (int i = 0; i < kWalkers; ++i) {
+    const unsigned p = part[i][lane];
+    if (i < w) run += p;
+    total += p;
+  }
+  if (!live) return;
+  if (w == 0) l.totals[g.first_bucket + b] = total;
+  int r = r0;
+  for (; r + kBatch <= r1; r += kBatch) {
     unsigned v[kBatch];
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) v[u] = col[(long long)(t + u) * kRadix];
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) s += v[u];
-  }
-  for (; t < t1; ++t) s += col[(long long)t * kRadix];
-  part[w][d] = s;
-  __syncthreads();
-  // Walker 0's wavefronts: digit totals, scanned over the 256 digits.
-  unsigned run = 0;
-  if (w == 0) {
-    unsigned total = 0;
-#pragma unroll
-    for (int k = 0; k < kWalkers; ++k) total += part[k][d];
-    const int lane = d & (kWave - 1), wave = d / kWave;
-    unsigned incl = total;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const unsigned o = __shfl_up(incl, off, kWave);
-      if (lane >= off) incl += o;
-    }
-    if (lane == kWave - 1) wsum[wave] = incl;
-    run = incl - total;
-  }
-  __syncthreads();
-  if (w == 0) {
-    for (int k = 0; k < d / kWave; ++k) run += wsum[k];
-#pragma unroll
-    for (int k = 0; k < kWalkers; ++k) {  // each walker's first offset
-      const unsigned c = part[k][d];
-      part[k][d] = run;
-      run += c;
-    }
-  }
-  __syncthreads();
-  run = part[w][d];
-  for (t = t0; t + kBatch <= t1; t += kBatch) {
-    unsigned v[kBatch];
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) v[u] = col[(long long)(t + u) * kRadix];
+    for (int u = 0; u < kBatch; ++u) v[u] = at[(long long)(r + u) * g.k];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
-      col[(long long)(t + u) * kRadix] = run;
+      at[(long long)(r + u) * g.k] = run;
       run += v[u];
     }
   }
-  for (; t < t1; ++t) {
-    const unsigned c = col[(long long)t * kRadix];
-    col[(long long)t * kRadix] = run;
-    run += c;
+  for (; r < r1; ++r) {
+    const unsigned v = at[(long long)r * g.k];
+    at[(long long)r * g.k] = run;
+    run += v;
   }
 }
 
-// Tiles are numbered XCD-major (each XCD takes a contiguous range of a
-// segment's tiles): the partial 128-byte lines at the ends of adjacent tiles'
-// digit runs are then written from one L2, close together in time.  Tile
-// order does not change the result (every position comes from the offsets);
-// measured 2.47 -> 2.33 ms on 256 ragged segments (35.8 M keys).
-__global__ __launch_bounds__(kBS) void scatter_kernel(const u64* __restrict__ src, u64* __restrict__ dst,
-                                                      const unsigned* __restrict__ counts, Plan plan, int shift,
-                                                      int convert_in, int convert_out, int src_is_x) {
-  __shared__ unsigned cnt[kBS / kWave][kRadix];
-  __shared__ unsigned goff[kRadix];
-  __shared__ unsigned dstart[kRadix];  // first LDS slot of each digit in the reordered tile
+// Keys of a row to their buckets.  Within a tile a key's slot is its
+// bucket's first slot plus the old value of an LDS counter; the tile then
+// leaves in slot order, so that each bucket's keys go to consecutive
+// addresses from consecutive work-items.  Rows are numbered XCD-major: the
+// partial lines at the ends of adjacent rows' runs are written from one L2.
+__global__ __launch_bounds__(kBS) void scatter_kernel(u64* x, u64* alt, Level l) {
+  __shared__ u64 keys[kTile];
+  __shared__ unsigned short slot_id[kTile];
+  __shared__ unsigned cnt[kMaxK];
+  __shared__ unsigned next[kMaxK];   // where the row's next key of the bucket goes
+  __shared__ unsigned delta[kMaxK];  // next - first slot
   __shared__ unsigned wsum[kBS / kWave];
-  __shared__ u64 sorted[kTile];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const TileInfo ti = get_tile(plan, xcd_major(blockIdx.x, gridDim.x));
-  const long long sbase = (src_is_x ? ti.seg_x : ti.seg_alt) + (long long)ti.local * kTile;
-  const long long dbase = src_is_x ? ti.seg_alt : ti.seg_x;
+  const int t = threadIdx.x;
+  const int row = int(xcd_major(blockIdx.x, gridDim.x));
+  if (l.bound && row >= l.bound->rows) return;
+  const int s = seg_of(l, l.row_seg, row, l.one.rows);
+  const Seg g = get_seg(l, s);
+  const int lrow = row - g.first_row;
+  constexpr int kPer = kMaxK / kBS;
+  const unsigned* before = l.counts + g.count_base + (long long)lrow * g.k;
+  // First key of each bucket in the segment.
+  {
+    unsigned tot[kPer], sum = 0;
 #pragma unroll
-  for (int w = 0; w < kBS / kWave; ++w) cnt[w][tid] = 0u;
-  goff[tid] = counts[ti.count_base + (long long)ti.local * kRadix + tid];
-  // Match masks of the ranking, one per wavefront and digit, in the part of
-  // the reorder buffer that is not written before the ranking ends.
-  static_assert(kTile >= (kBS / kWave) * kRadix, "match masks fit in the reorder buffer");
-  u64(*match)[kRadix] = reinterpret_cast<u64(*)[kRadix]>(sorted);
-#pragma unroll
-  for (int w = 0; w < kBS / kWave; ++w) match[w][tid] = 0ull;
-  __syncthreads();
-
-  u64 key[kRows];
-  unsigned rank[kRows];
-  const u64 lane_below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-#pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    const int p = tile_pos(wave, r, lane);
-    const bool valid = p < ti.len;
-    u64 k = 0;
-    if (valid) {
-      k = src[sbase + p];
-      if (convert_in) k = to_key(k);
+    for (int j = 0; j < kPer; ++j) {
+      const int b = t * kPer + j;
+      tot[j] = b < g.k ? l.totals[g.first_bucket + b] : 0u;
+      sum += tot[j];
     }
-    key[r] = k;
-    const unsigned d = unsigned(k >> shift) & 0xFFu;
-    // The row's lanes of digit d: each valid lane ORs its bit into the
-    // wavefront's mask of d and reads the mask back.  One wavefront's LDS
-    // operations complete in issue order, each over all its lanes, so the
-    // read sees every lane's bit, and the group's highest lane clears the
-    // mask after its read, before the next row's ORs.
-    u64 m = 0;
-    if (valid) {
-      atomicOr(&match[wave][d], 1ull << lane);
-      m = match[wave][d];
-    }
-    unsigned base = 0;
-    if (valid) base = cnt[wave][d];
-    rank[r] = base + unsigned(__popcll(m & lane_below));
-    // highest lane of the group advances the wavefront's digit counter
-    if (valid && (m >> lane) == 1ull) {
-      cnt[wave][d] = base + unsigned(__popcll(m));
-      match[wave][d] = 0ull;
+    unsigned run = block_exclusive_scan(sum, wsum);
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const int b = t * kPer + j;
+      if (b < g.k) {
+        next[b] = run + before[b];
+        if (lrow == 0) {
+          const u64* sp = l.splitters + g.first_bucket;
+          const bool pure = b > 0 && b < g.k - 1 && sp[b - 1] == sp[b];
+          l.starts[g.first_bucket + b] = run | (pure ? 0x80000000u : 0u);
+        }
+      }
+      run += tot[j];
     }
   }
-  __syncthreads();
-  // Prefix over wavefronts for every digit (thread = digit), then over the
-  // digits: each key's slot in the tile reordered by digit.
-  unsigned total = 0;
-#pragma unroll
-  for (int w = 0; w < kBS / kWave; ++w) {
-    const unsigned c = cnt[w][tid];
-    cnt[w][tid] = total;
-    total += c;
-  }
-  dstart[tid] = block_exclusive_scan(total, wsum);
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    const int p = tile_pos(wave, r, lane);
-    if (p < ti.len) {
-      const unsigned d = unsigned(key[r] >> shift) & 0xFFu;
-      sorted[dstart[d] + cnt[wave][d] + rank[r]] = key[r];
-    }
-  }
-  __syncthreads();
-  // Slot i holds the (i - dstart[d])-th key of digit d in the tile, which
-  // goes to goff[d] + i - dstart[d]: runs of one digit are contiguous.
-  if (ti.len == kTile) {
-    // Full tile: all of the work-item's slots are read before any is
-    // written out, so the LDS reads overlap instead of waiting in turn.
-    u64 kk[kRows];
-#pragma unroll
-    for (int r = 0; r < kRows; ++r) kk[r] = sorted[tid + r * kBS];
+  const u64* src = (g.src ? alt : x) + g.base;
+  u64* dst = (g.src ? x : alt) + g.base;
+  const unsigned short* ids = l.ids + g.base;
+  const long long local0 = (long long)lrow * l.chunk * kTile;
+  for (int c = 0; c < l.chunk; ++c) {
+    const long long first = local0 + (long long)c * kTile;
+    if (first >= g.len) break;
+    const int n = int(g.len - first < kTile ? g.len - first : kTile);
+    u64 k[kRows];
+    unsigned id[kRows], rank[kRows];
 #pragma unroll
     for (int r = 0; r < kRows; ++r) {
-      const int i = tid + r * kBS;
-      const unsigned d = unsigned(kk[r] >> shift) & 0xFFu;
-      const long long pos = (long long)goff[d] + (i - dstart[d]);
-      if (pos < ti.seg_len) dst[dbase + pos] = convert_out ? from_key(kk[r]) : kk[r];
+      const int i = r * kBS + t;
+      id[r] = i < n ? ids[first + i] : 0u;
+      k[r] = i < n ? src[first + i] : 0ull;
     }
-  } else {
-    for (int i = tid; i < ti.len; i += kBS) {
-      const u64 k = sorted[i];
-      const unsigned d = unsigned(k >> shift) & 0xFFu;
-      const long long pos = (long long)goff[d] + (i - dstart[d]);
-      if (pos < ti.seg_len) dst[dbase + pos] = convert_out ? from_key(k) : k;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) cnt[t + j * kBS] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kRows; ++r)
+      if (r * kBS + t < n) rank[r] = atomicAdd(&cnt[id[r]], 1u);
+    __syncthreads();
+    {
+      unsigned cc[kPer], sum = 0;
+#pragma unroll
+      for (int j = 0; j < kPer; ++j) {
+        cc[j] = cnt[t * kPer + j];
+        sum += cc[j];
+      }
+      unsigned run = block_exclusive_scan(sum, wsum);
+#pragma unroll
+      for (int j = 0; j < kPer; ++j) {
+        const int b = t * kPer + j;
+        cnt[b] = run;  // first slot
+        if (b < g.k) {
+          delta[b] = next[b] - run;
+          next[b] += cc[j];
+        }
+        run += cc[j];
+      }
     }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kRows; ++r)
+      if (r * kBS + t < n) {
+        const unsigned at = cnt[id[r]] + rank[r];
+        keys[at] = k[r];
+        slot_id[at] = (unsigned short)id[r];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      const int i = r * kBS + t;
+      if (i < n) dst[delta[slot_id[i]] + unsigned(i)] = keys[i];
+    }
+    __syncthreads();
   }
 }
 
-// The ragged layout's tables from the per-segment descriptors: work-item t
-// writes TileInfo t (its segment found by binary search over the
-// descriptors' first tiles) and, for t < nsd, SegInfo t.
-__global__ __launch_bounds__(256) void tile_table_kernel(const SegDesc* __restrict__ d, int nsd,
-                                                         TileInfo* __restrict__ tiles, SegInfo* __restrict__ segs,
-                                                         int total_tiles) {
-  const int t = int(blockIdx.x) * 256 + int(threadIdx.x);
-  if (t < nsd) segs[t] = SegInfo{d[t].count_base, d[t].ntiles, 0};
-  if (t >= total_tiles) return;
-  int lo = 0, hi = nsd - 1;  // the last descriptor whose first tile is <= t
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (d[mid].first_tile <= t) lo = mid;
-    else hi = mid - 1;
+// ---- buckets -------------------------------------------------------------------
+
+struct Piece {
+  long long base;
+  int len, src;
+  bool pure;
+};
+
+// Bucket i of a level (a whole segment where k = 1), and where it lies.
+__device__ __forceinline__ Piece get_piece(const Level& l, int i) {
+  const int s = seg_of(l, l.bucket_seg, i, l.one.k);
+  const Seg g = get_seg(l, s);
+  if (g.k <= 1) return Piece{g.base, g.len, g.src, g.pure != 0};
+  const unsigned st = l.starts[i];
+  return Piece{g.base + (long long)(st & 0x7FFFFFFFu), int(l.totals[i]), 1 - g.src, (st >> 31) != 0};
+}
+
+// Every bucket of up to kBucket keys, by the smallest network that holds it.
+// Longer ones go on the list for big_kernel.
+__global__ __launch_bounds__(kBS) void bucket_kernel(u64* x, const u64* alt, Level l) {
+  __shared__ u64 mem[kBucketSlots];
+  const int t = threadIdx.x, i = blockIdx.x;
+  if (l.bound && i >= l.bound->buckets) return;
+  const Piece p = get_piece(l, i);
+  const u64* src = (p.src ? alt : x) + p.base;
+  u64* dst = x + p.base;
+  if (p.pure) {
+    if (p.src)
+      for (int j = t; j < p.len; j += kBS) dst[j] = src[j];
+    return;
   }
-  const SegDesc sd = d[lo];
-  TileInfo ti;
-  ti.seg_x = sd.seg_x;
-  ti.seg_alt = sd.seg_alt;
-  ti.count_base = sd.count_base;
-  ti.local = t - sd.first_tile;
-  ti.ntiles = sd.ntiles;
-  ti.seg_len = sd.seg_len;
-  const int rem = sd.seg_len - ti.local * kTile;
-  ti.len = rem < kTile ? rem : kTile;
-  tiles[t] = ti;
+  if (p.len > kBucket) {
+    if (t == 0) l.big[atomicAdd(&l.header->nbig, 1)] = i;
+    return;
+  }
+  if (p.len <= 1 && !p.src) return;
+  if (p.len <= 1024) sort_piece<2>(src, dst, p.len, mem, t);
+  else if (p.len <= 2048) sort_piece<3>(src, dst, p.len, mem, t);
+  else sort_piece<4>(src, dst, p.len, mem, t);
+}
+
+// Any length: pieces of kBig keys, then merges of ever longer runs, every
+// key finding its place by a search in the other run.  The pieces start in x
+// or alt so that the last merge ends in x.
+__device__ void sort_any(u64* x, u64* alt, const Piece& p, void* mem, int t) {
+  u64* at[2] = {x + p.base, alt + p.base};
+  const u64* src = at[p.src];
+  int rounds = 0;
+  while (((long long)kBig << rounds) < p.len) ++rounds;
+  int cur = rounds & 1;
+  for (long long o = 0; o < p.len; o += kBig) {
+    const int n = int(p.len - o < kBig ? p.len - o : kBig);
+    sort_piece<5>(src + o, at[cur] + o, n, mem, t);
+    __syncthreads();
+  }
+  for (long long w = kBig; w < p.len; w *= 2) {
+    const u64* a = at[cur];
+    u64* d = at[cur ^ 1];
+    for (long long i = t; i < p.len; i += kBS) {
+      const long long lo = i / (2 * w) * (2 * w);
+      const long long mid = lo + w < p.len ? lo + w : p.len;
+      const long long hi = lo + 2 * w < p.len ? lo + 2 * w : p.len;
+      const bool left = i < mid;
+      const u64 raw = a[i], key = to_key(raw);
+      long long b = left ? mid : lo, e = left ? hi : mid;
+      const long long b0 = b;
+      while (b < e) {
+        const long long m = (b + e) >> 1;
+        const u64 o = to_key(a[m]);
+        if (left ? o < key : o <= key) b = m + 1;
+        else e = m;
+      }
+      d[lo + (left ? i - lo : i - mid) + (b - b0)] = raw;
+    }
+    __syncthreads();
+    cur ^= 1;
+  }
+}
+
+__global__ __launch_bounds__(kBS) void big_kernel(u64* x, u64* alt, Level l) {
+  __shared__ u64 mem[kBigSlots];
+  const int n = l.header->nbig;
+  for (int i = blockIdx.x; i < n; i += gridDim.x) {
+    sort_any(x, alt, get_piece(l, l.big[i]), mem, threadIdx.x);
+    __syncthreads();
+  }
+}
+
+// The second level's segments are the first level's buckets: one workgroup
+// numbers their rows, buckets, column groups and count entries.
+__global__ __launch_bounds__(1024) void second_level_kernel(Level l, int nbuckets, Seg* out, Header* bound, int chunk) {
+  __shared__ long long sums[1024 / kWave][4];
+  __shared__ long long carry[4];
+  const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+  if (t < 4) carry[t] = 0;
+  __syncthreads();
+  for (int i0 = 0; i0 < nbuckets; i0 += 1024) {
+    const int i = i0 + t;
+    Piece p{0, 0, 0, false};
+    if (i < nbuckets) p = get_piece(l, i);
+    Seg g;
+    g.base = p.base;
+    g.len = p.len;
+    g.src = p.src;
+    g.pure = p.pure;
+    g.k = p.pure ? 1 : buckets_for(p.len, true);
+    g.rows = g.k > 1 ? int((p.len + (long long)chunk * kTile - 1) / ((long long)chunk * kTile)) : 0;
+    const int cols = g.k > 1 ? (g.k + kCol - 1) / kCol : 0;
+    if (i >= nbuckets) g.k = 0;
+    long long v[4] = {g.rows, g.k, cols, (long long)g.rows * g.k}, incl[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      incl[c] = v[c];
+      for (int off = 1; off < kWave; off <<= 1) {
+        const long long o = __shfl_up(incl[c], off, kWave);
+        if (lane >= off) incl[c] += o;
+      }
+      if (lane == kWave - 1) sums[wave][c] = incl[c];
+    }
+    __syncthreads();
+    long long first[4], total[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      first[c] = carry[c] + incl[c] - v[c];
+      total[c] = carry[c];
+      for (int w = 0; w < 1024 / kWave; ++w) {
+        if (w < wave) first[c] += sums[w][c];
+        total[c] += sums[w][c];
+      }
+    }
+    if (i < nbuckets) {
+      g.first_row = int(first[0]);
+      g.first_bucket = int(first[1]);
+      g.first_col = int(first[2]);
+      g.count_base = first[3];
+      out[i] = g;
+    }
+    __syncthreads();
+    if (t == 0)
+      for (int c = 0; c < 4; ++c) carry[c] = total[c];
+    __syncthreads();
+  }
+  if (t == 0) {
+    bound->rows = int(carry[0]);
+    bound->buckets = int(carry[1]);
+    bound->cols = int(carry[2]);
+  }
 }
 
 inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
-struct Sizes {
-  long long total_keys = 0, total_tiles = 0;
-  bool uniform = true;
-  long long seg_len = 0;
+// Sizes of one level's tables, for exact counts (first level) or bounds.
+struct LevelSize {
+  long long segs = 0, rows = 0, buckets = 0, cols = 0, counts = 0;
 };
+struct Sizes {
+  long long keys = 0, longest = 0, base = 0;
+  int64_t nseg = 0;  // non-empty segments
+  bool uniform = true, small = true, two_levels = false;
+  int chunk = 1;
+  LevelSize l1, l2;
+};
+
+// Tiles per row: one, and more where that would make over 4096 rows.
+int chunk_for(long long keys) {
+  const long long c = keys / (4096ll * kTile);
+  return int(c < 1 ? 1 : c > 64 ? 64 : c);
+}
+
+Seg describe(long long base, long long len, int chunk) {
+  Seg g{};
+  g.base = base;
+  g.len = int(len);
+  g.k = buckets_for(len, false);
+  g.rows = g.k > 1 ? int(ceil_div(len, (long long)chunk * kTile)) : 0;
+  return g;
+}
 
 Sizes measure(const int64_t* off, int64_t nseg) {
   Sizes s;
+  if (nseg <= 0) return s;
+  s.base = off[0];
+  s.keys = off[nseg] - off[0];
+  s.chunk = chunk_for(s.keys);
+  s.uniform = off[0] == 0 && s.keys > 0;
   for (int64_t i = 0; i < nseg; ++i) {
     const long long len = off[i + 1] - off[i];
-    s.total_keys += len;
-    s.total_tiles += (len + kTile - 1) / kTile;
-    if (i == 0) s.seg_len = len;
-    else if (len != s.seg_len) s.uniform = false;
+    if (len != off[1] - off[0]) s.uniform = false;
+    if (len <= 0) continue;
+    ++s.nseg;
+    s.longest = std::max(s.longest, len);
+    const Seg g = describe(0, len, s.chunk);
+    s.l1.rows += g.rows;
+    s.l1.buckets += g.k;
+    if (g.k > 1) {
+      s.l1.cols += ceil_div(g.k, kCol);
+      s.l1.counts += (long long)g.rows * g.k;
+    }
   }
-  if (nseg > 0 && off[0] != 0) s.uniform = false;
-  if (s.uniform && s.seg_len == 0) s.uniform = false;
+  s.l1.segs = s.nseg;
+  s.small = s.longest <= kBucket;
+  s.two_levels = s.longest > kOneLevel;
+  if (s.two_levels) {
+    s.l2.segs = s.l1.buckets;
+    s.l2.rows = s.keys / ((long long)s.chunk * kTile) + s.l2.segs;
+    s.l2.buckets = s.keys / kAim + s.l2.segs;
+    s.l2.cols = s.l2.buckets / kCol + s.l2.segs;
+    s.l2.counts = s.l2.rows * buckets_for(s.longest, true);
+  }
   return s;
 }
 
-size_t scratch_for(const Sizes& s, int64_t nseg) {
-  size_t b = align256(size_t(s.total_keys) * 8);                      // ping-pong keys
-  b += align256(size_t(s.total_tiles) * kRadix * sizeof(unsigned));  // counters
-  if (!s.uniform) {
-    b += align256(size_t(s.total_tiles) * sizeof(TileInfo));
-    b += align256(size_t(nseg) * sizeof(SegInfo));
-    b += align256(size_t(nseg) * sizeof(SegDesc));
+// Hands out the scratch in 256-byte pieces.
+struct Arena {
+  char* base;
+  size_t used = 0;
+  template <typename T>
+  T* take(long long n) {
+    T* p = base ? reinterpret_cast<T*>(base + used) : nullptr;
+    used += align256(size_t(n) * sizeof(T));
+    return p;
   }
-  return b;
+};
+
+struct Layout {
+  u64* alt;
+  Seg *segs1, *segs2;
+  Header* bound;
+  Level level[2];
+  size_t total;
+};
+
+Layout lay_out(const Sizes& s, void* scratch) {
+  Arena a{reinterpret_cast<char*>(scratch)};
+  Layout o{};
+  o.alt = a.take<u64>(s.keys);
+  unsigned short* ids = a.take<unsigned short>(s.keys);
+  Header* headers = a.take<Header>(2);  // overfull buckets; bounds of the second level
+  o.bound = headers + 1;
+  o.segs1 = a.take<Seg>(s.nseg);
+  o.segs2 = a.take<Seg>(s.l2.segs);
+  int* big = a.take<int>(std::max(s.l1.buckets, s.l2.buckets));
+  for (int i = 0; i < 2; ++i) {
+    const LevelSize& z = i ? s.l2 : s.l1;
+    Level& l = o.level[i];
+    l.chunk = s.chunk;
+    l.row_seg = a.take<int>(z.rows);
+    l.col_seg = a.take<int>(z.cols);
+    l.bucket_seg = a.take<int>(z.buckets);
+    l.dup = a.take<int>(z.segs);
+    l.splitters = a.take<u64>(z.buckets);
+    l.counts = a.take<unsigned>(z.counts);
+    l.totals = a.take<unsigned>(z.buckets);
+    l.starts = a.take<unsigned>(z.buckets);
+    l.ids = ids;
+    l.header = headers;
+    l.big = big;
+  }
+  o.total = a.used;
+  return o;
+}
+
+int partition(u64* x, u64* alt, const Level& l, const LevelSize& z, hipStream_t st) {
+  sample_kernel<<<dim3(unsigned(l.nseg)), dim3(kBS), 0, st>>>(x, alt, l);
+  if (z.rows > 0) {
+    hist_kernel<<<dim3(unsigned(z.rows)), dim3(kBS), 0, st>>>(x, alt, l);
+    colscan_kernel<<<dim3(unsigned(z.cols)), dim3(kCol * kWalkers), 0, st>>>(l);
+    scatter_kernel<<<dim3(unsigned(z.rows)), dim3(kBS), 0, st>>>(x, alt, l);
+  }
+  return launch_status();
 }
 
 }  // namespace
@@ -396,7 +907,8 @@ extern "C" {
 
 size_t rpx_sort_segmented_scratch_bytes(const int64_t* offsets_host, int64_t nseg) {
   if (!offsets_host || nseg < 0) return 0;
-  return scratch_for(measure(offsets_host, nseg), nseg);
+  const Sizes s = measure(offsets_host, nseg);
+  return s.keys > 0 ? lay_out(s, nullptr).total : 0;
 }
 
 int rpx_sort_segmented_f64(double* x, const int64_t* offsets_host, int64_t nseg, void* scratch, size_t scratch_bytes,
@@ -407,69 +919,63 @@ int rpx_sort_segmented_f64(double* x, const int64_t* offsets_host, int64_t nseg,
     if (offsets_host[i] < 0 || len < 0 || len > INT32_MAX) return RPX_ERR_INVALID_ARGUMENT;
   }
   const Sizes s = measure(offsets_host, nseg);
-  if (s.total_keys == 0) return RPX_SUCCESS;
+  if (s.keys == 0) return RPX_SUCCESS;
   if (!x || !scratch) return RPX_ERR_INVALID_ARGUMENT;
-  if (scratch_bytes < scratch_for(s, nseg)) return RPX_ERR_SCRATCH_TOO_SMALL;
-  if (s.total_tiles > INT32_MAX || nseg > INT32_MAX) return RPX_ERR_UNSUPPORTED;
+  Layout o = lay_out(s, scratch);
+  if (scratch_bytes < o.total) return RPX_ERR_SCRATCH_TOO_SMALL;
+  if (s.nseg > INT32_MAX || s.l1.buckets > INT32_MAX || s.l2.buckets > INT32_MAX) return RPX_ERR_UNSUPPORTED;
   hipStream_t st = as_stream(stream);
+  // x and the scratch copies are indexed alike, from the first segment's key.
+  u64* xs = reinterpret_cast<u64*>(x) + s.base;
 
-  // Segments with no keys contribute no tiles; non-uniform layouts (and
-  // segments not starting at x[0]) use an explicit tile table.
-  char* base = reinterpret_cast<char*>(scratch);
-  u64* alt = reinterpret_cast<u64*>(base);
-  size_t off = align256(size_t(s.total_keys) * 8);
-  unsigned* counts = reinterpret_cast<unsigned*>(base + off);
-  off += align256(size_t(s.total_tiles) * kRadix * sizeof(unsigned));
-
-  Plan plan{nullptr, nullptr, s.seg_len, int((s.seg_len + kTile - 1) / kTile)};
-  int64_t nseg_launch = nseg;
-  if (!s.uniform) {
-    // Ragged layout: explicit tile and segment tables.  Segments keep their
-    // positions in x; in the scratch copy they are packed back to back.  The
-    // host describes each non-empty segment; a kernel expands the
-    // descriptors into one TileInfo per tile.
-    std::vector<SegDesc> desc;
-    desc.reserve(size_t(nseg));
-    long long cbase = 0, packed = 0;
-    int first = 0;
+  Level* l = &o.level[0];
+  l->nseg = int(s.nseg);
+  if (s.uniform) {
+    l->one = describe(0, s.longest, s.chunk);
+  } else {
+    std::vector<Seg> segs;
+    segs.reserve(size_t(s.nseg));
+    Seg next{};
     for (int64_t i = 0; i < nseg; ++i) {
       const long long len = offsets_host[i + 1] - offsets_host[i];
-      const int nt = int((len + kTile - 1) / kTile);
-      if (nt == 0) continue;
-      desc.push_back(SegDesc{offsets_host[i], packed, cbase, first, nt, int(len), 0});
-      cbase += (long long)nt * kRadix;
-      packed += len;
-      first += nt;
+      if (len == 0) continue;
+      Seg g = describe(offsets_host[i] - s.base, len, s.chunk);
+      g.first_row = next.first_row;
+      g.first_bucket = next.first_bucket;
+      g.first_col = next.first_col;
+      g.count_base = next.count_base;
+      next.first_row += g.rows;
+      next.first_bucket += g.k;
+      next.first_col += g.k > 1 ? int(ceil_div(g.k, kCol)) : 0;
+      next.count_base += (long long)g.rows * g.k;
+      segs.push_back(g);
     }
-    TileInfo* dt = reinterpret_cast<TileInfo*>(base + off);
-    off += align256(size_t(s.total_tiles) * sizeof(TileInfo));
-    SegInfo* ds = reinterpret_cast<SegInfo*>(base + off);
-    off += align256(size_t(nseg) * sizeof(SegInfo));
-    SegDesc* dd = reinterpret_cast<SegDesc*>(base + off);
-    const HostChunk table{dd, desc.data(), desc.size() * sizeof(SegDesc)};
+    const HostChunk table{o.segs1, segs.data(), segs.size() * sizeof(Seg)};
     if (const int rc = upload_async(&table, 1, st); rc != RPX_SUCCESS) return rc;
-    tile_table_kernel<<<dim3(unsigned(ceil_div(s.total_tiles, 256))), dim3(256), 0, st>>>(
-        dd, int(desc.size()), dt, ds, int(s.total_tiles));
-    if (const int rc = launch_status(); rc != RPX_SUCCESS) return rc;
-    plan.tiles = dt;
-    plan.segs = ds;
-    nseg_launch = int64_t(desc.size());
+    l->segs = o.segs1;
   }
-
-  u64* xs = reinterpret_cast<u64*>(x);
-  for (int pass = 0; pass < kPasses; ++pass) {
-    const u64* src = (pass % 2 == 0) ? xs : alt;
-    u64* dst = (pass % 2 == 0) ? alt : xs;
-    const int shift = 8 * pass;
-    const int src_is_x = (pass % 2 == 0);
-    hist_kernel<<<dim3(unsigned(s.total_tiles)), dim3(kBS), 0, st>>>(src, counts, plan, shift, pass == 0, src_is_x);
-    offsets_kernel<<<dim3(unsigned(nseg_launch)), dim3(kOffThreads), 0, st>>>(counts, plan);
-    scatter_kernel<<<dim3(unsigned(s.total_tiles)), dim3(kBS), 0, st>>>(src, dst, counts, plan, shift, pass == 0,
-                                                                        pass == kPasses - 1, src_is_x);
-    const int rc = launch_status();
-    if (rc != RPX_SUCCESS) return rc;
+  LevelSize z = s.l1;
+  if (s.small) {
+    l->bucket_seg = nullptr;
+  } else {
+    if (const int rc = partition(xs, o.alt, *l, z, st); rc != RPX_SUCCESS) return rc;
   }
-  return RPX_SUCCESS;
+  if (s.two_levels) {
+    Level* l2 = &o.level[1];
+    second_level_kernel<<<dim3(1), dim3(1024), 0, st>>>(*l, int(s.l1.buckets), o.segs2, o.bound, s.chunk);
+    l2->segs = o.segs2;
+    l2->nseg = int(s.l2.segs);
+    l2->bound = o.bound;
+    l = l2;
+    z = s.l2;
+    if (const int rc = partition(xs, o.alt, *l, z, st); rc != RPX_SUCCESS) return rc;
+  }
+  bucket_kernel<<<dim3(unsigned(z.buckets)), dim3(kBS), 0, st>>>(xs, o.alt, *l);
+  if (!s.small) {
+    const unsigned grid = unsigned(z.buckets < 512 ? z.buckets : 512);
+    big_kernel<<<dim3(grid), dim3(kBS), 0, st>>>(xs, o.alt, *l);
+  }
+  return launch_status();
 }
 
 }  // extern "C"
