@@ -266,14 +266,16 @@ int rpx_jacobi2d_sweep_f64(double* dst, const double* src, int64_t N,
  * (POLYBENCH_JACOBI_2D-Seq.cpp:30-54, -Hip.cpp:27-114). */
 int rpx_jacobi2d_f64(double* A, double* B, int64_t N, int64_t tsteps,
                      const rpx_tuning* tune, void* stream);
-/* Same result with temporal blocking: each launch runs `depth` whole time
- * steps (2*depth sweeps, tune->depth: 1..4, default 3) on register-resident
- * tiles or chunks,
- * reading A once and writing only the final B and the new A, the new A going
- * to `scratch` (an N x N grid) and back, so no launch overwrites values a
- * neighbouring tile still reads.  Ends with the result in A and B, bit-equal
- * to rpx_jacobi2d_f64.  Falls back to the two-sweep path for odd N,
- * N > 2^22 or pointers that are not 16-byte aligned. */
+/* Same result with temporal blocking: each launch runs several whole time
+ * steps on register-resident tiles, reading A once and writing only the final
+ * B and the new A, the new A going to `scratch` (an N x N grid) and back, so
+ * no launch overwrites values a neighbouring tile still reads.  Ends with the
+ * result in A and B, bit-equal to rpx_jacobi2d_f64.  Without a requested shape
+ * tile and depth are chosen by N and tsteps, for odd N too.  With
+ * tune->items_per_thread or tune->depth (1..4, default 3) it runs
+ * rpx_jacobi2d_fused_launch_f64's launches of that shape, and the two-sweep
+ * path for odd N or pointers that are not 16-byte aligned.  The two-sweep
+ * path also takes N > 2^22, and odd N > 128 without a usable scratch. */
 size_t rpx_jacobi2d_fused_scratch_bytes(int64_t N);
 /* The building block of rpx_jacobi2d_fused_f64: one launch advancing `depth`
  * time steps (1..4) from Ain into Aout, writing the final B (unless
