@@ -1,7 +1,6 @@
 // GEMM (polybench): C[i][j] = sum_k (alpha*A[i][k]) * B[k][j].  With
 // RPX_TUNE_GEMM_BETA the textbook form C = alpha*A*B + beta*C instead (the
-// old C read once; the MFMA kernel starts its sums at beta*C, the
-// comparator adds beta*C to its sum).
+// old C read once and beta*C added to the finished sum).
 //
 // Reference: src/polybench/POLYBENCH_GEMM.hpp:12-50 (C *= beta, then C is
 // overwritten by the dot, so beta never reaches the result),
@@ -11,12 +10,11 @@
 // Two FP64 paths:
 //  * gemm_naive_kernel: the one-thread-per-element shape of the suite's
 //    Base_HIP variant, kept as the "plain FP64 GPU" comparator;
-//  * gemm_mfma_f64_kernel: 128x128 workgroup tiles, four wavefronts of 64x64,
-//    each a 4x4 grid of v_mfma_f64_16x16x4f64 accumulators; A (pre-scaled by
-//    alpha, as the suite rounds alpha*A[i][k]) and B staged through LDS in
-//    16-deep K slabs with the next slab's global loads in flight during the
-//    current slab's MFMAs.  Tiles are mapped XCD-major so neighbouring tiles
-//    that share A rows / B columns run on the same XCD's L2.
+//  * gemm_mfma_f64_kernel: v_mfma_f64_16x16x4f64 on workgroup tiles from
+//    128 x 128 to 16 x 16, by size; tiles are mapped XCD-major so neighbouring
+//    tiles that share A rows / B columns run on the same XCD's L2.
+#include <type_traits>
+
 #include "rpx_common.hpp"
 
 using namespace rpx;
@@ -40,186 +38,271 @@ __global__ __launch_bounds__(256) void gemm_naive_kernel(double* __restrict__ C,
 
 // ---- FP64 MFMA ---------------------------------------------------------------
 //
-// 128x128 output tile per workgroup of four wavefronts (64x64 each, a 4x4
-// grid of v_mfma_f64_16x16x4f64 tiles), K in slabs of 16, double-buffered
-// in LDS.  Both operands sit in LDS k-contiguous ([m][k] for A, [n][k] for
-// B, rows padded by two doubles), and in each pair of MFMA steps lane (r, q)
-// of a fragment takes the adjacent k = 8h + 2q and 8h + 2q + 1, so one
-// 16-byte LDS read feeds two MFMAs.  The k order inside a slab is thereby
-// permuted; the result is the same sum in another association.  Interior
-// tiles load full slabs with unconditional 16-byte loads (A rows as they
-// are, B as 2x4 blocks transposed in registers); edge tiles, partial slabs
-// and odd shapes take guarded 8-byte loads.
-constexpr int kTM = 128, kTN = 128, kTK = 16;
-constexpr int kThreads = 256;
-constexpr int kLdsRow = kTK + 2;  // doubles per LDS row of either operand
+// A workgroup computes a tile of C with WM x WN x WK wavefronts: each owns
+// MF x NF tiles of v_mfma_f64_16x16x4f64 and, of every K slab, the WK-th part
+// of TK deep (partial sums of the WK groups meet in LDS at the end, added in
+// a fixed order).  Slabs are double-buffered in LDS, both operands
+// k-contiguous ([m][k] for A, [n][k] for B, rows padded by two doubles); in
+// each pair of MFMA steps lane (r, q) of a fragment takes the adjacent
+// k = 8h + 2q and 8h + 2q + 1, so one 16-byte LDS read feeds two MFMAs.  The
+// k order inside a slab is thereby permuted; the result is the same sum in
+// another association.  The next slab's global loads are in flight during the
+// current slab's MFMAs and nothing reads them before those are issued: A is
+// scaled by alpha, as the suite rounds alpha*A[i][k], on its way to LDS.
+// Rows and columns outside C are loaded from its last ones (their products are
+// never stored); only the K remainder is zeroed.
+typedef v2d v2d_u __attribute__((aligned(8)));
 
-// BETA: the textbook C = beta*C + the products (a separate kernel; the
-// suite's form reads no C).
-template <bool BETA>
-__device__ __forceinline__ void gemm_mfma_f64_tile(double* __restrict__ C, const double* __restrict__ A,
-                                                   const double* __restrict__ B, double alpha, double beta,
-                                                   int64_t ni, int64_t nj, int64_t nk, int tiles_n, int vec) {
-  __shared__ __attribute__((aligned(16))) double As[2][kTM * kLdsRow];  // As[m][k]
-  __shared__ __attribute__((aligned(16))) double Bs[2][kTN * kLdsRow];  // Bs[n][k]
+template <int MF_, int NF_, int WM_, int WN_, int WK_, int TK_, int FB_>
+struct Shape {
+  static constexpr int FB = FB_;  // fragment sets: 2 where the registers allow reading a step ahead
+  static constexpr int MF = MF_, NF = NF_, WM = WM_, WN = WN_, WK = WK_, TK = TK_;
+  static constexpr int TM = 16 * MF * WM, TN = 16 * NF * WN, KS = TK * WK, T = kWave * WM * WN * WK;
+  static constexpr int LR = KS + 2;              // doubles per LDS row of either operand
+  static constexpr int PA = TM * KS / 2 / T;     // 16-byte pairs of A per work-item and slab
+  static constexpr int PB = TN * KS / 4 / T;     // 2x2 blocks of B
+  static constexpr int kSlabs = 2 * (TM + TN) * LR, kSums = WK > 1 ? WK * TM * TN : 0;
+  static constexpr int kLds = kSlabs > kSums ? kSlabs : kSums;
+  static_assert(PA * T * 2 == TM * KS && PB * T * 4 == TN * KS, "whole pairs and blocks");
+  static_assert(TK % 8 == 0, "whole steps");
+};
+
+template <typename S>
+__global__ __launch_bounds__(S::T, 2) void gemm_mfma_f64_kernel(double* __restrict__ C, const double* __restrict__ A,
+                                                             const double* __restrict__ B, double alpha, double beta,
+                                                             int use_beta, int64_t ni, int64_t nj, int64_t nk,
+                                                             int tiles_n) {
+  __shared__ __attribute__((aligned(16))) double lds[S::kLds];
+  auto As = [&](int buf) { return lds + buf * S::TM * S::LR; };
+  auto Bs = [&](int buf) { return lds + 2 * S::TM * S::LR + buf * S::TN * S::LR; };
 
   const unsigned tile = xcd_major(blockIdx.x, gridDim.x);
-  const int64_t m0 = int64_t(tile / unsigned(tiles_n)) * kTM;
-  const int64_t n0 = int64_t(tile % unsigned(tiles_n)) * kTN;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = (wave >> 1) * 64;  // wave's row offset in the tile
-  const int wn = (wave & 1) * 64;   // wave's column offset
-  const bool interior = vec && m0 + kTM <= ni && n0 + kTN <= nj;
+  const int64_t m0 = int64_t(tile / unsigned(tiles_n)) * S::TM;
+  const int64_t n0 = int64_t(tile % unsigned(tiles_n)) * S::TN;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wn = wave % S::WN * 16 * S::NF, wm = wave / S::WN % S::WM * 16 * S::MF, wk = wave / (S::WN * S::WM);
+  const bool n_inside = n0 + S::TN <= nj;
 
-  // Loader mapping.  A: row a_m, k a_k .. a_k+7.  B: k rows b_k, b_k+1,
-  // columns b_n .. b_n+3.
-  const int a_m = tid >> 1, a_k = (tid & 1) * 8;
-  const int b_k = (tid >> 5) * 2, b_n = (tid & 31) * 4;
-
-  double ra[8], rb[8];  // rb[c*2 + t]: B(k = b_k + t, n = b_n + c)
+  const double* pa[S::PA];  // this work-item's row of A, at its k
+  int ka[S::PA];
+  const double* pb[S::PB];  // its first row of B, first column
+  int kb[S::PB], nb[S::PB], odd[S::PB];
+#pragma unroll
+  for (int u = 0; u < S::PA; ++u) {
+    const int at = tid + u * S::T;
+    const int64_t row = m0 + at / (S::KS / 2);
+    ka[u] = 2 * (at % (S::KS / 2));
+    pa[u] = A + (row < ni ? row : ni - 1) * nk + ka[u];
+  }
+#pragma unroll
+  for (int u = 0; u < S::PB; ++u) {
+    const int at = tid + u * S::T;
+    nb[u] = 2 * (at % (S::TN / 2));
+    kb[u] = 2 * (at / (S::TN / 2));
+    const int64_t c = n0 + nb[u];
+    odd[u] = c + 1 < nj;  // the second column exists
+    pb[u] = B + kb[u] * nj + (c < nj ? c : nj - 1);
+  }
+  v2d ra[S::PA], rb[S::PB][2];
   auto load_slab = [&](int64_t k0) {
-    if (interior && k0 + kTK <= nk) {
-      const double* pa = A + (m0 + a_m) * nk + k0 + a_k;
+    if (k0 + S::KS <= nk) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const v2d x = *reinterpret_cast<const v2d*>(pa + 2 * u);
-        ra[2 * u] = alpha * x.x;
-        ra[2 * u + 1] = alpha * x.y;
+      for (int u = 0; u < S::PA; ++u) ra[u] = *reinterpret_cast<const v2d_u*>(pa[u] + k0);
+      if (n_inside) {
+#pragma unroll
+        for (int u = 0; u < S::PB; ++u)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) rb[u][t] = *reinterpret_cast<const v2d_u*>(pb[u] + (k0 + t) * nj);
+      } else {
+#pragma unroll
+        for (int u = 0; u < S::PB; ++u)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            rb[u][t].x = pb[u][(k0 + t) * nj];
+            rb[u][t].y = pb[u][(k0 + t) * nj + odd[u]];
+          }
       }
-      const double* pb = B + (k0 + b_k) * nj + n0 + b_n;
+    } else {  // the K remainder
+      const int left = int(nk - k0);
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const v2d x0 = *reinterpret_cast<const v2d*>(pb + t * nj);
-        const v2d x1 = *reinterpret_cast<const v2d*>(pb + t * nj + 2);
-        rb[0 * 2 + t] = x0.x;
-        rb[1 * 2 + t] = x0.y;
-        rb[2 * 2 + t] = x1.x;
-        rb[3 * 2 + t] = x1.y;
-      }
-    } else {
-      const int64_t gi = m0 + a_m;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int64_t gk = k0 + a_k + u;
-        ra[u] = (gi < ni && gk < nk) ? alpha * A[gi * nk + gk] : 0.0;
+      for (int u = 0; u < S::PA; ++u) {
+        ra[u].x = ka[u] < left ? pa[u][k0] : 0.0;
+        ra[u].y = ka[u] + 1 < left ? pa[u][k0 + 1] : 0.0;
       }
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int u = 0; u < S::PB; ++u)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int64_t gk = k0 + b_k + t, gj = n0 + b_n + c;
-          rb[c * 2 + t] = (gk < nk && gj < nj) ? B[gk * nj + gj] : 0.0;
+        for (int t = 0; t < 2; ++t) {
+          rb[u][t].x = kb[u] + t < left ? pb[u][(k0 + t) * nj] : 0.0;
+          rb[u][t].y = kb[u] + t < left ? pb[u][(k0 + t) * nj + odd[u]] : 0.0;
         }
     }
   };
   auto store_slab = [&](int buf) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-      *reinterpret_cast<v2d*>(&As[buf][a_m * kLdsRow + a_k + 2 * u]) = v2d{ra[2 * u], ra[2 * u + 1]};
+    for (int u = 0; u < S::PA; ++u)
+      *reinterpret_cast<v2d*>(As(buf) + (tid + u * S::T) / (S::KS / 2) * S::LR + ka[u]) = alpha * ra[u];
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-      *reinterpret_cast<v2d*>(&Bs[buf][(b_n + c) * kLdsRow + b_k]) = v2d{rb[c * 2], rb[c * 2 + 1]};
+    for (int u = 0; u < S::PB; ++u) {
+      *reinterpret_cast<v2d*>(Bs(buf) + nb[u] * S::LR + kb[u]) = v2d{rb[u][0].x, rb[u][1].x};
+      *reinterpret_cast<v2d*>(Bs(buf) + (nb[u] + 1) * S::LR + kb[u]) = v2d{rb[u][0].y, rb[u][1].y};
+    }
   };
 
-  // With BETA the accumulators start at beta*C (the old C read once, before
-  // the K loop), so the result is beta*C plus the products; otherwise at 0.
-  // The C reads go one fragment row at a time (the empty asm statement keeps
-  // the compiler from issuing all 64 together, which took 100 more VGPRs
-  // and a wavefront per SIMD).
-  v4d acc[4][4];
+  v4d acc[S::MF][S::NF];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < S::MF; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if constexpr (BETA) {
-        if (j == 0) asm volatile("" ::: "memory");
-      }
-      acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
-      if constexpr (BETA) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int64_t gi = m0 + wm + i * 16 + 4 * r + (lane >> 4);
-          const int64_t gj = n0 + wn + j * 16 + (lane & 15);
-          // Clamped into C: the accumulators of rows or columns outside C
-          // are never stored, so what they start from does not matter.
-          const int64_t ci = gi < ni ? gi : ni - 1, cj = gj < nj ? gj : nj - 1;
-          acc[i][j][r] = beta * C[ci * nj + cj];
-        }
-      }
-    }
+    for (int j = 0; j < S::NF; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
 
-  const int64_t nslabs = (nk + kTK - 1) / kTK;
-  load_slab(0);
-  store_slab(0);
-  __syncthreads();
   const int fr = lane & 15;  // fragment row (A) / column (B)
-  const int fq = lane >> 4;  // k pair within an 8-deep half slab
-  for (int64_t s = 0; s < nslabs; ++s) {
-    const int buf = int(s & 1);
-    if (s + 1 < nslabs) load_slab((s + 1) * kTK);
+  const int fk = wk * S::TK + 2 * (lane >> 4);
+  v2d af[S::FB][S::MF], bf[S::FB][S::NF];
+  auto read_frags = [&](int buf, int h, int to) {
 #pragma unroll
-    for (int h = 0; h < kTK / 8; ++h) {
-      v2d af[4], bf[4];
+    for (int i = 0; i < S::MF; ++i)
+      af[to][i] = *reinterpret_cast<const v2d*>(As(buf) + (wm + i * 16 + fr) * S::LR + 8 * h + fk);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        af[i] = *reinterpret_cast<const v2d*>(&As[buf][(wm + i * 16 + fr) * kLdsRow + 8 * h + 2 * fq]);
+    for (int j = 0; j < S::NF; ++j)
+      bf[to][j] = *reinterpret_cast<const v2d*>(Bs(buf) + (wn + j * 16 + fr) * S::LR + 8 * h + fk);
+  };
+  // A step is two halves, the first k of every lane and the second, so each
+  // accumulator's two MFMAs are apart.  With two fragment sets the next step's
+  // are read between the halves; the slab's last step then runs behind the
+  // barrier, over the first reads of the next slab.
+  constexpr int kSteps = S::TK / 8;
+  static_assert(S::FB == 1 || kSteps % 2 == 0, "a slab begins with set 0");
+  if (nk > 0) {
+    load_slab(0);
+    store_slab(0);
+    __syncthreads();
+    if (S::FB == 2) read_frags(0, 0, 0);
+  }
+  int buf = 0;
+  for (int64_t k0 = 0; k0 < nk; k0 += S::KS) {
+    const bool more = k0 + S::KS < nk;
+    if (more) load_slab(k0 + S::KS);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        bf[j] = *reinterpret_cast<const v2d*>(&Bs[buf][(wn + j * 16 + fr) * kLdsRow + 8 * h + 2 * fq]);
-      // All 16 tiles take their first k before any takes its second, so
-      // each accumulator's two MFMAs are 16 instructions apart.
+    for (int h = 0; h < kSteps; ++h) {
+      const int cur = S::FB == 2 ? h % 2 : 0, nxt = S::FB == 2 ? cur ^ 1 : 0;
+      if (S::FB == 1) read_frags(buf, h, 0);
+      __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < S::MF; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i].x, bf[j].x, acc[i][j], 0, 0, 0);
+        for (int j = 0; j < S::NF; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[cur][i].x, bf[cur][j].x, acc[i][j], 0, 0, 0);
+      if (S::FB == 2 && h + 1 < kSteps) read_frags(buf, h + 1, nxt);
+      if (S::FB == 2 && h + 1 == kSteps && more) {
+        store_slab(buf ^ 1);
+        __syncthreads();
+        read_frags(buf ^ 1, 0, nxt);
+      }
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < S::MF; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i].y, bf[j].y, acc[i][j], 0, 0, 0);
-      // The backend's LDS-read/MFMA interleave for small GEMM loops: 2.228
-      // against 2.248 ms at 4096^3 (strategy 1 was slower, 2.305 ms).
-      __builtin_amdgcn_iglp_opt(0);
+        for (int j = 0; j < S::NF; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[cur][i].y, bf[cur][j].y, acc[i][j], 0, 0, 0);
     }
-    if (s + 1 < nslabs) {
+    __builtin_amdgcn_s_setprio(0);
+    if (S::FB == 1 && more) {
       store_slab(buf ^ 1);
       __syncthreads();
     }
+    buf ^= 1;
   }
 
+  auto put = [&](int64_t gi, int64_t gj, double v) {
+    if (gi < ni && gj < nj) {
+      double* c = C + gi * nj + gj;
+      *c = use_beta ? fma(beta, *c, v) : v;
+    }
+  };
   // v_mfma_f64_16x16x4f64 accumulator layout (measured on gfx950): element r
   // of lane l is row 4*r + l/16, column l%16.
+  if constexpr (S::WK == 1) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < S::MF; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < S::NF; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t gi = m0 + wm + i * 16 + 4 * r + (lane >> 4);
-        const int64_t gj = n0 + wn + j * 16 + (lane & 15);
-        if (gi < ni && gj < nj) C[gi * nj + gj] = acc[i][j][r];
-      }
+        for (int r = 0; r < 4; ++r)
+          put(m0 + wm + i * 16 + 4 * r + (lane >> 4), n0 + wn + j * 16 + fr, acc[i][j][r]);
+  } else {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < S::MF; ++i)
+#pragma unroll
+      for (int j = 0; j < S::NF; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          lds[(wk * S::TM + wm + i * 16 + 4 * r + (lane >> 4)) * S::TN + wn + j * 16 + fr] = acc[i][j][r];
+    __syncthreads();
+    for (int e = tid; e < S::TM * S::TN; e += S::T) {
+      double v = lds[e];
+#pragma unroll
+      for (int k = 1; k < S::WK; ++k) v += lds[k * S::TM * S::TN + e];
+      put(m0 + e / S::TN, n0 + e % S::TN, v);
+    }
   }
 }
 
-__global__ __launch_bounds__(kThreads) void gemm_mfma_f64_kernel(double* __restrict__ C,
-                                                                 const double* __restrict__ A,
-                                                                 const double* __restrict__ B, double alpha,
-                                                                 int64_t ni, int64_t nj, int64_t nk, int tiles_n,
-                                                                 int vec) {
-  gemm_mfma_f64_tile<false>(C, A, B, alpha, 0.0, ni, nj, nk, tiles_n, vec);
+template <typename S>
+int launch_mfma(double* C, const double* A, const double* B, double alpha, double beta, int use_beta, int64_t ni,
+                int64_t nj, int64_t nk, hipStream_t s) {
+  const int64_t tm = ceil_div(ni, S::TM), tn = ceil_div(nj, S::TN);
+  if (tm * tn > INT32_MAX || tn > INT32_MAX) return RPX_ERR_UNSUPPORTED;
+  gemm_mfma_f64_kernel<S><<<dim3(unsigned(tm * tn)), dim3(S::T), 0, s>>>(C, A, B, alpha, beta, use_beta, ni, nj, nk,
+                                                                       int(tn));
+  return launch_status();
 }
 
-// The textbook form.  Left to itself the compiler gives this instance 256
-// VGPRs and 148 AGPRs (one wavefront per SIMD, 1.6x the time); capped at
-// two wavefronts per SIMD it spills 20 bytes per work-item.
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_mfma_f64_beta_kernel(
-    double* __restrict__ C, const double* __restrict__ A, const double* __restrict__ B, double alpha, double beta,
-    int64_t ni, int64_t nj, int64_t nk, int tiles_n, int vec) {
-  gemm_mfma_f64_tile<true>(C, A, B, alpha, beta, ni, nj, nk, tiles_n, vec);
+// The shapes, largest tile first.  A large tile moves the least data per
+// product, but C has to hold 256 tiles before every CU has one; small tiles
+// split K over their wavefronts instead, so that few of them still fill the
+// matrix cores.
+//
+// What bounds them: FP64 MFMA issue, 64 clocks each (77 TF/s, measured).
+// 4096^3 runs at 65 TF/s (2.10 ms; 2.24 ms when A was scaled, and so waited
+// for, as it was loaded), its matrix cores busy 86% of the time; the rest is
+// LDS writes and the barrier between slabs.  1000 x 1000 x 1200 took 261 us as
+// 64 tiles of 128 x 128 on 256 CUs and takes 58 us as 256 tiles of 64 x 64
+// (31 us of MFMAs, 10 us of launch, first loads and epilogue, 8 us of LDS
+// writes, 6 us of loads).
+using Big = Shape<4, 4, 2, 2, 1, 16, 1>;     // 128 x 128, four wavefronts
+using Mid = Shape<2, 2, 2, 2, 2, 16, 2>;     // 64 x 64, K in two, two workgroups per CU
+using MidDeep = Shape<2, 2, 2, 2, 2, 32, 2>; // 64 x 64, K in two, one workgroup per CU
+using Small = Shape<2, 2, 1, 1, 4, 8, 1>;    // 32 x 32, K in four
+using SmallDeep = Shape<2, 2, 1, 1, 8, 8, 1>;// 32 x 32, K in eight
+using Tiny = Shape<1, 1, 1, 1, 8, 16, 1>;    // 16 x 16, K in eight
+
+// Time of a product without the launch, in microseconds: a tile alone on a CU
+// takes `alone` per unit of K, a CU's n-th tile `shared` (both fitted to 12
+// sizes from 64^3 to 4096^3, within about 15%).
+template <typename S>
+double mfma_us(int64_t ni, int64_t nj, int64_t nk, double alone, double shared) {
+  const double n = double(ceil_div(ni, S::TM)) * double(ceil_div(nj, S::TN)) / 256.0;
+  const double per_k = shared * (n < 8 ? double(ceil_div(int64_t(n * 256.0), 256)) : n + 0.5);
+  return double(ceil_div(nk, S::KS) * S::KS) * (per_k > alone ? per_k : alone);
+}
+
+int gemm_mfma(double* C, const double* A, const double* B, double alpha, double beta, int use_beta, int64_t ni,
+              int64_t nj, int64_t nk, hipStream_t s) {
+  const double us[] = {mfma_us<Big>(ni, nj, nk, 0.145, 0.131),        mfma_us<Mid>(ni, nj, nk, 0.0435, 0.0365),
+                       mfma_us<MidDeep>(ni, nj, nk, 0.041, 0.041),    mfma_us<Small>(ni, nj, nk, 0.0163, 0.0122),
+                       mfma_us<SmallDeep>(ni, nj, nk, 0.0138, 0.0122), mfma_us<Tiny>(ni, nj, nk, 0.0049, 0.0047)};
+  int best = 0;
+  for (int i = 1; i < 6; ++i)
+    if (us[i] < us[best]) best = i;
+  switch (best) {
+    case 0: return launch_mfma<Big>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
+    case 1: return launch_mfma<Mid>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
+    case 2: return launch_mfma<MidDeep>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
+    case 3: return launch_mfma<Small>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
+    case 4: return launch_mfma<SmallDeep>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
+    default: return launch_mfma<Tiny>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
+  }
 }
 
 }  // namespace
@@ -240,16 +323,7 @@ int rpx_gemm_f64(double* C, const double* A, const double* B, double alpha, doub
                                                                               nj, nk);
     return launch_status();
   }
-  const int64_t tm = ceil_div(ni, kTM), tn = ceil_div(nj, kTN);
-  if (tm * tn > INT32_MAX || tn > INT32_MAX) return RPX_ERR_UNSUPPORTED;
-  const int vec = (nk % 2 == 0) && (nj % 2 == 0) && aligned16(A) && aligned16(B);
-  if (use_beta)
-    gemm_mfma_f64_beta_kernel<<<dim3(unsigned(tm * tn)), dim3(kThreads), 0, s>>>(C, A, B, alpha, beta, ni, nj, nk,
-                                                                                int(tn), vec);
-  else
-    gemm_mfma_f64_kernel<<<dim3(unsigned(tm * tn)), dim3(kThreads), 0, s>>>(C, A, B, alpha, ni, nj, nk, int(tn),
-                                                                           vec);
-  return launch_status();
+  return gemm_mfma(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
 }
 
 }  // extern "C"
