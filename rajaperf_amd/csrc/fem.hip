@@ -40,21 +40,9 @@ namespace {
 constexpr int kBS = 256;
 constexpr int kLdsBudget = 48 * 1024;
 
-// MASS3DPA's LDS bytes per workgroup by order, which sets its elements per
-// workgroup: below 48 KB a CU holds four workgroups where the registers
-// allow it.  Timed with 24, 32, 36, 40 and 48 KB at NE = 262144 (65536 for
-// D1D >= 5): 24 KB is ~10% faster at D1D = 3, 36 KB 2-6% at 4, 40 KB ~6% at
-// 5; D1D = 2 and >= 6 show no gain.
-constexpr int mass_lds_budget(int D) {
-  return D == 3 ? 24 * 1024 : D == 4 ? 36 * 1024 : D == 5 ? 40 * 1024 : kLdsBudget;
-}
-
-// A compiler barrier at the top of each pencil iteration (orders D1D >= 7):
-// the basis values are then re-read from LDS (a wavefront-uniform
-// broadcast) for every pencil instead of all D*Q of them being hoisted into
-// registers, which at these orders cost more VGPRs than the rest of the
-// kernel together (246 against 164 at (8,9)).  Lower orders keep them in
-// registers: re-reading cost 27% at (4,5).
+// A compiler barrier at the top of each pencil iteration of DIFFUSION3DPA: the
+// basis values are then re-read from LDS (a wavefront-uniform broadcast) for
+// every pencil instead of all of them being hoisted into registers.
 __device__ __forceinline__ void reload_basis() { asm volatile("" ::: "memory"); }
 
 // Global-memory pointers: with the address space in the type, accesses are
@@ -62,222 +50,183 @@ __device__ __forceinline__ void reload_basis() { asm volatile("" ::: "memory"); 
 typedef const __attribute__((address_space(1))) double gcdouble;
 typedef __attribute__((address_space(1))) double gdouble;
 
-// Doubles of D a work-item may hold in registers from the start of the
-// element code to its third stage (measured at (4,5): 0.150 -> 0.137 ms).
-constexpr int kMassPrefetch = 24;
+// Basis tables are read through the scalar cache into SGPRs, which a multiply
+// takes as its uniform operand: they cost no LDS bandwidth and no VGPRs.  (A
+// broadcast LDS read of a basis value costs as much LDS time as one of 64
+// different values; re-read per pencil they were 80% of the LDS traffic at
+// (8,9).)  The pointer is made opaque where a stage begins, so that a table
+// is loaded for one stage and not kept over all of them.
+typedef const __attribute__((address_space(4))) double cdouble;
+__device__ __forceinline__ cdouble* table(gcdouble* p) {
+  const uint64_t a = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(a));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(uint32_t(a >> 32));
+  return reinterpret_cast<cdouble*>(uint64_t(hi) << 32 | lo);
+}
+__device__ __forceinline__ cdouble* opaque(cdouble* p) {
+  asm volatile("" : "+s"(p));
+  return p;
+}
+// u[q] = sum_d v[d] B(q,d), B(q,d) = T[q + Q*d].
+template <int D, int Q>
+__device__ __forceinline__ void to_quad(const double (&v)[D], cdouble* T, double (&u)[Q]) {
+#pragma unroll
+  for (int q = 0; q < Q; ++q) u[q] = 0.0;
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) u[q] += v[d] * T[q + Q * d];
+}
 
+// u[d] = sum_q v[q] Bt'(d,q), Bt'(d,q) = T[q + D*d].
+template <int D, int Q>
+__device__ __forceinline__ void to_dofs(const double (&v)[Q], cdouble* T, double (&u)[D]) {
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    u[d] = 0.0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) u[d] += v[q] * T[q + D * d];
+  }
+}
+
+// E elements per workgroup, so that no stage has more pencils than there are
+// work-items: the Q^2 of the widest stage fill them as far as they go.  What
+// bounds the operator is then the memory it moves: at NE = 185185 / 116618 /
+// 78125 of D1D = 6 / 7 / 8 it takes 264 / 260 / 269 us (0.80-0.85 of the time
+// of its bytes at 6.5 TB/s).  With as many elements as 24 to 48 KB of LDS hold
+// a stage took two passes, the second nearly empty, and fewer workgroups fit
+// on a CU: 278 / 312 / 317 us; with the basis in LDS as well 324 / 396 / 388 us.
 template <int D, int Q>
 struct MassShape {
   static constexpr int kA = Q * Q * Q;  // DDQ / QQQ / QDD per element
   static constexpr int kB = D * Q * Q;  // DQQ / QQD per element
-  static constexpr int kBytes = 8 * (kA + kB);
-  static constexpr int E0 = mass_lds_budget(D) / kBytes;
-  static constexpr int E = E0 < 1 ? 1 : (E0 > 64 ? 64 : E0);
-  static constexpr int kLds = E * (kA + kB) + 2 * Q * D;  // doubles of LDS
+  static constexpr int E = kBS / (Q * Q);
+  static constexpr int kLds = E * (kA + kB);  // doubles of LDS
 };
 
 // Elements [e0, e0+ne) of one operator application, ne <= MassShape::E, by
-// the whole workgroup, with four disjoint LDS buffers: bufA [E][kA],
-// bufB [E][kB], sB[q*D + d] = B(q,d) and sBt[d*Q + q] = Bt'(d,q) =
-// Bt[q + D*d] (Q*D each).  They are separate restrict parameters so the
-// compiler may reorder accesses between them.  Ends with the workgroup's
-// last LDS reads still pending: a caller that reuses the buffers must
-// synchronise first.
+// the whole workgroup, with two disjoint LDS buffers, bufA [E][kA] and
+// bufB [E][kB].  They are separate restrict parameters so the compiler may
+// reorder accesses between them.  Ends with the workgroup's last LDS reads
+// still pending: a caller that reuses the buffers must synchronise first.
 template <int D, int Q, bool kEarlyXY = true>
 __device__ __forceinline__ void mass3dpa_elements(gcdouble* __restrict__ Bg, gcdouble* __restrict__ Btg,
                                                   gcdouble* __restrict__ Dg, gcdouble* __restrict__ Xg,
                                                   gdouble* __restrict__ Yg, int64_t e0, int ne,
-                                                  double* __restrict__ bufA, double* __restrict__ bufB,
-                                                  double* __restrict__ sB, double* __restrict__ sBt) {
+                                                  double* __restrict__ bufA, double* __restrict__ bufB) {
   using S = MassShape<D, Q>;
   constexpr int D2 = D * D, D3 = D * D * D, Q2 = Q * Q, Q3 = Q * Q * Q;
-  const int tid = threadIdx.x;
+  const int w = threadIdx.x;  // the pencil of every stage
+  cdouble* const Bc = table(Bg);
+  cdouble* const Btc = table(Btg);
 
-  for (int t = tid; t < Q * D; t += kBS) {
-    const int q = t / D, d = t % D;
-    sB[t] = Bg[q + Q * d];
-    const int d2 = t / Q, q2 = t % Q;
-    sBt[t] = Btg[q2 + D * d2];
+  // D (P3), X (P1) and Y (P6) pencils go to registers early: D and X before
+  // P1, Y at the start of P4 (when D's registers are free), so none of these
+  // loads waits at the head of its stage.  X and Y only for D1D up to 8, and
+  // not at Q = D + 2 from D = 5 nor in the persistent loops (the single-launch
+  // batch kernel and the per-order loop), where the extra live registers cost
+  // a wavefront per SIMD.
+  constexpr bool kPreXY = kEarlyXY && D <= 8 && !(D >= 5 && Q >= D + 2);
+  gcdouble* const xp = Xg + (e0 + w / D2) * D3 + w % D2 * D;  // X[e][dz][dy][:]
+  gdouble* const yp = Yg + (e0 + w / D2) * D3 + w % D2;       // Y[e][:][dy][dx]
+  double x[D], y[D], dq[Q];
+  auto load_x = [&] {
+#pragma unroll
+    for (int dx = 0; dx < D; ++dx) x[dx] = xp[dx];
+  };
+  // All of the pencil's Y values are loaded before the first store: where the
+  // Y pointer comes from memory the compiler otherwise keeps each load behind
+  // the previous store and waits on it D times per pencil.
+  auto load_y = [&] {
+#pragma unroll
+    for (int dz = 0; dz < D; ++dz) y[dz] = yp[dz * D2];
+  };
+  if (kPreXY && w < ne * D2) load_x();
+  if (w < ne * Q2) {
+    gcdouble* dp = Dg + (e0 + w / Q2) * Q3 + w % Q2;
+#pragma unroll
+    for (int qz = 0; qz < Q; ++qz) dq[qz] = dp[qz * Q2];
   }
-  constexpr int kIt3 = (S::E * Q2 + kBS - 1) / kBS;  // P3 pencils per work-item
-  constexpr bool kPre = kIt3 * Q <= kMassPrefetch;
-  double dpre[kPre ? kIt3 : 1][Q];
-  // X (P1) and Y (P6) pencils go to registers early where they fit in eight
-  // doubles: X before the first barrier, Y at the start of P4 (when D's
-  // registers are free), so neither load waits at the head of its stage.
-  // Not at Q = D + 2 from D = 5, and not in the persistent loops (the
-  // single-launch batch kernel and the per-order loop), where the extra live
-  // registers cost a wavefront per SIMD.
-  constexpr int kIt1 = (S::E * D2 + kBS - 1) / kBS;  // P1 and P6 pencils per work-item
-  constexpr bool kPreXY = kEarlyXY && kIt1 * D <= 8 && !(D >= 5 && Q >= D + 2);
-  double xpre[kPreXY ? kIt1 : 1][D];
-  if constexpr (kPreXY) {
-#pragma unroll
-    for (int it = 0; it < kIt1; ++it) {
-      const int w = tid + it * kBS;
-      if (w < ne * D2) {
-        gcdouble* xp = Xg + (e0 + w / D2) * D3 + (w % D2) * D;  // X[e][dz][dy][:]
-#pragma unroll
-        for (int dx = 0; dx < D; ++dx) xpre[it][dx] = xp[dx];
-      }
-    }
-  }
-  if constexpr (kPre) {
-#pragma unroll
-    for (int it = 0; it < kIt3; ++it) {
-      const int w = tid + it * kBS;
-      if (w < ne * Q2) {
-        const int e = w / Q2, r = w % Q2;
-#pragma unroll
-        for (int qz = 0; qz < Q; ++qz) dpre[it][qz] = Dg[(e0 + e) * Q3 + r + qz * Q2];
-      }
-    }
-  }
-  __syncthreads();
 
   // P1: x-contraction of X pencils.
-  for (int w = tid, it = 0; w < ne * D2; w += kBS, ++it) {
-    if constexpr (D >= 7) reload_basis();
-    const int e = w / D2, r = w % D2, dz = r / D, dy = r % D;
-    double x[D];
-    if constexpr (kPreXY) {
+  cdouble* T = opaque(Bc);
+  if (w < ne * D2) {
+    if constexpr (!kPreXY) load_x();
+    double u[Q];
+    to_quad<D, Q>(x, T, u);
+    double* out = bufA + w / D2 * S::kA + w % D2 * Q;  // DDQ[dz][dy][qx]
 #pragma unroll
-      for (int dx = 0; dx < D; ++dx) x[dx] = xpre[it][dx];
-    } else {
-      gcdouble* xp = Xg + (e0 + e) * D3 + dz * D2 + dy * D;
-#pragma unroll
-      for (int dx = 0; dx < D; ++dx) x[dx] = xp[dx];
-    }
-    double* out = bufA + e * S::kA + (dz * D + dy) * Q;
-#pragma unroll
-    for (int qx = 0; qx < Q; ++qx) {
-      double u = 0.0;
-#pragma unroll
-      for (int dx = 0; dx < D; ++dx) u += x[dx] * sB[qx * D + dx];
-      out[qx] = u;
-    }
+    for (int qx = 0; qx < Q; ++qx) out[qx] = u[qx];
   }
   __syncthreads();
   // P2: y-contraction.
-  for (int w = tid; w < ne * D * Q; w += kBS) {
-    if constexpr (D >= 7) reload_basis();
+  T = opaque(Bc);
+  if (w < ne * D * Q) {
     const int e = w / (D * Q), r = w % (D * Q), dz = r / Q, qx = r % Q;
     const double* in = bufA + e * S::kA + dz * D * Q + qx;  // DDQ[dz][dy][qx], stride Q in dy
-    double v[D];
+    double v[D], u[Q];
 #pragma unroll
     for (int dy = 0; dy < D; ++dy) v[dy] = in[dy * Q];
+    to_quad<D, Q>(v, T, u);
     double* out = bufB + e * S::kB + dz * Q2 + qx;  // DQQ[dz][qy][qx], stride Q in qy
 #pragma unroll
-    for (int qy = 0; qy < Q; ++qy) {
-      double u = 0.0;
-#pragma unroll
-      for (int dy = 0; dy < D; ++dy) u += v[dy] * sB[qy * D + dy];
-      out[qy * Q] = u;
-    }
+    for (int qy = 0; qy < Q; ++qy) out[qy * Q] = u[qy];
   }
   __syncthreads();
-  // P3: z-contraction and the quadrature-point scaling.  The D values were
-  // loaded before P1 when they fit in a few registers (kPre), so their
-  // latency overlaps the first two stages.
+  // P3: z-contraction and the quadrature-point scaling.
+  T = opaque(Bc);
+  if (w < ne * Q2) {
+    const int e = w / Q2, r = w % Q2;         // r = qy*Q + qx
+    const double* in = bufB + e * S::kB + r;  // DQQ[dz][qy][qx], stride Q2 in dz
+    double v[D], u[Q];
 #pragma unroll
-  for (int it = 0; it < kIt3; ++it) {
-    const int w = tid + it * kBS;
-    if (w < ne * Q2) {
-      if constexpr (D >= 7) reload_basis();
-      const int e = w / Q2, r = w % Q2;  // r = qy*Q + qx
-      const double* in = bufB + e * S::kB + r;  // DQQ[dz][qy][qx], stride Q2 in dz
-      double v[D];
+    for (int dz = 0; dz < D; ++dz) v[dz] = in[dz * Q2];
+    to_quad<D, Q>(v, T, u);
+    double* out = bufA + e * S::kA + r;  // QQQ[qz][qy][qx], stride Q2 in qz
 #pragma unroll
-      for (int dz = 0; dz < D; ++dz) v[dz] = in[dz * Q2];
-      double* out = bufA + e * S::kA + r;  // QQQ[qz][qy][qx], stride Q2 in qz
-#pragma unroll
-      for (int qz = 0; qz < Q; ++qz) {
-        double u = 0.0;
-#pragma unroll
-        for (int dz = 0; dz < D; ++dz) u += v[dz] * sB[qz * D + dz];
-        if constexpr (kPre)
-          out[qz * Q2] = u * dpre[it][qz];
-        else
-          out[qz * Q2] = u * Dg[(e0 + e) * Q3 + r + qz * Q2];
-      }
-    }
+    for (int qz = 0; qz < Q; ++qz) out[qz * Q2] = u[qz] * dq[qz];
   }
   __syncthreads();
-  double ypre[kPreXY ? kIt1 : 1][D];
-  if constexpr (kPreXY) {
-#pragma unroll
-    for (int it = 0; it < kIt1; ++it) {
-      const int w = tid + it * kBS;
-      if (w < ne * D2) {
-        gcdouble* yp = Yg + (e0 + w / D2) * D3 + w % D2;  // Y[e][:][dy][dx]
-#pragma unroll
-        for (int dz = 0; dz < D; ++dz) ypre[it][dz] = yp[dz * D2];
-      }
-    }
-  }
+  if (kPreXY && w < ne * D2) load_y();
   // P4: backward x-contraction.
-  for (int w = tid; w < ne * Q2; w += kBS) {
-    if constexpr (D >= 7) reload_basis();
-    const int e = w / Q2, r = w % Q2;  // r = qz*Q + qy
+  T = opaque(Btc);
+  if (w < ne * Q2) {
+    const int e = w / Q2, r = w % Q2;             // r = qz*Q + qy
     const double* in = bufA + e * S::kA + r * Q;  // QQQ[qz][qy][qx], contiguous in qx
-    double v[Q];
+    double v[Q], u[D];
 #pragma unroll
     for (int qx = 0; qx < Q; ++qx) v[qx] = in[qx];
+    to_dofs<D, Q>(v, T, u);
     double* out = bufB + e * S::kB + r * D;  // QQD[qz][qy][dx]
 #pragma unroll
-    for (int dx = 0; dx < D; ++dx) {
-      double u = 0.0;
-#pragma unroll
-      for (int qx = 0; qx < Q; ++qx) u += v[qx] * sBt[dx * Q + qx];
-      out[dx] = u;
-    }
+    for (int dx = 0; dx < D; ++dx) out[dx] = u[dx];
   }
   __syncthreads();
   // P5: backward y-contraction.
-  for (int w = tid; w < ne * Q * D; w += kBS) {
-    if constexpr (D >= 7) reload_basis();
+  T = opaque(Btc);
+  if (w < ne * Q * D) {
     const int e = w / (Q * D), r = w % (Q * D), qz = r / D, dx = r % D;
     const double* in = bufB + e * S::kB + qz * Q * D + dx;  // QQD[qz][qy][dx], stride D in qy
-    double v[Q];
+    double v[Q], u[D];
 #pragma unroll
     for (int qy = 0; qy < Q; ++qy) v[qy] = in[qy * D];
+    to_dofs<D, Q>(v, T, u);
     double* out = bufA + e * S::kA + qz * D2 + dx;  // QDD[qz][dy][dx], stride D in dy
 #pragma unroll
-    for (int dy = 0; dy < D; ++dy) {
-      double u = 0.0;
-#pragma unroll
-      for (int qy = 0; qy < Q; ++qy) u += v[qy] * sBt[dy * Q + qy];
-      out[dy * D] = u;
-    }
+    for (int dy = 0; dy < D; ++dy) out[dy * D] = u[dy];
   }
   __syncthreads();
   // P6: backward z-contraction, accumulate into Y.
-  for (int w = tid, it = 0; w < ne * D2; w += kBS, ++it) {
-    if constexpr (D >= 7) reload_basis();
-    const int e = w / D2, r = w % D2;  // r = dy*D + dx
-    const double* in = bufA + e * S::kA + r;  // QDD[qz][dy][dx], stride D2 in qz
-    double v[Q];
+  T = opaque(Btc);
+  if (w < ne * D2) {
+    const double* in = bufA + w / D2 * S::kA + w % D2;  // QDD[qz][dy][dx], stride D2 in qz
+    double v[Q], u[D];
 #pragma unroll
     for (int qz = 0; qz < Q; ++qz) v[qz] = in[qz * D2];
-    gdouble* yp = Yg + (e0 + e) * D3 + r;
-    // All of the pencil's Y values are loaded before the first store: where
-    // the Y pointer comes from memory the compiler otherwise keeps each
-    // load behind the previous store and waits on it D times per pencil.
-    double y[D];
-    if constexpr (kPreXY) {
+    if constexpr (!kPreXY) load_y();
+    to_dofs<D, Q>(v, T, u);
 #pragma unroll
-      for (int dz = 0; dz < D; ++dz) y[dz] = ypre[it][dz];
-    } else {
-#pragma unroll
-      for (int dz = 0; dz < D; ++dz) y[dz] = yp[dz * D2];
-    }
-#pragma unroll
-    for (int dz = 0; dz < D; ++dz) {
-      double u = 0.0;
-#pragma unroll
-      for (int qz = 0; qz < Q; ++qz) u += v[qz] * sBt[dz * Q + qz];
-      yp[dz * D2] = y[dz] + u;
-    }
+    for (int dz = 0; dz < D; ++dz) yp[dz * D2] = y[dz] + u[dz];
   }
 }
 
@@ -290,12 +239,9 @@ __global__ __launch_bounds__(kBS) void mass3dpa_kernel(const double* __restrict_
   using S = MassShape<D, Q>;
   __shared__ double bufA[S::E * S::kA];
   __shared__ double bufB[S::E * S::kB];
-  __shared__ double sB[Q * D];
-  __shared__ double sBt[D * Q];
   const int64_t e0 = int64_t(blockIdx.x) * S::E;
   const int ne = int((NE - e0) < S::E ? (NE - e0) : S::E);
-  mass3dpa_elements<D, Q>((gcdouble*)Bg, (gcdouble*)Btg, (gcdouble*)Dg, (gcdouble*)Xg, (gdouble*)Yg, e0, ne, bufA, bufB,
-                          sB, sBt);
+  mass3dpa_elements<D, Q>((gcdouble*)Bg, (gcdouble*)Btg, (gcdouble*)Dg, (gcdouble*)Xg, (gdouble*)Yg, e0, ne, bufA, bufB);
 }
 
 // ---- ragged batches, one persistent launch ----------------------------------
@@ -306,7 +252,7 @@ __global__ __launch_bounds__(kBS) void mass3dpa_kernel(const double* __restrict_
 // chunk0[batch].  A grid of a few workgroups per CU strides over the chunks;
 // each chunk dispatches on its batch's order to the same element code as the
 // single-order kernel, so results are bit-identical to it.
-constexpr int kBatchLds = kLdsBudget / 8 + 2 * 9 * 8;  // doubles: the largest kLds over the orders
+constexpr int kBatchLds = MassShape<8, 9>::kLds > MassShape<7, 8>::kLds ? MassShape<8, 9>::kLds : MassShape<7, 8>::kLds;  // doubles: the largest kLds over the orders
 
 typedef __attribute__((address_space(3))) double lds_double;
 
@@ -324,11 +270,10 @@ __device__ __attribute__((noinline)) void mass_batch_chunk(rpx_mass_batch b, int
   const int ne = int((b.ne - e0) < S::E ? (b.ne - e0) : S::E);
   double* bufA = (double*)lds;
   double* bufB = bufA + S::E * S::kA;
-  double* sB = bufB + S::E * S::kB;
   // The descriptors' pointers are global memory: typed so, the element code
   // issues global (not FLAT) accesses, which do not hold up its LDS waits.
   mass3dpa_elements<D, D + 1, false>((gcdouble*)b.B, (gcdouble*)b.Bt, (gcdouble*)b.D, (gcdouble*)b.X, (gdouble*)b.Y, e0, ne,
-                              bufA, bufB, sB, sB + (D + 1) * D);
+                              bufA, bufB);
 }
 
 // Elements per chunk of a batch of order d1d (Q1D = d1d + 1).
@@ -413,8 +358,6 @@ __global__ __launch_bounds__(kBS) void mass3dpa_order_kernel(const char* __restr
   using S = MassShape<D, D + 1>;
   __shared__ double bufA[S::E * S::kA];
   __shared__ double bufB[S::E * S::kB];
-  __shared__ double sB[(D + 1) * D];
-  __shared__ double sBt[D * (D + 1)];
   const BatchHeader* hdr = reinterpret_cast<const BatchHeader*>(plan);
   const int64_t nchunks = hdr->nchunks, nbatch = hdr->nbatch;
   const int64_t begin = hdr->order_begin[D], end = hdr->order_end[D];
@@ -437,7 +380,7 @@ __global__ __launch_bounds__(kBS) void mass3dpa_order_kernel(const char* __restr
     const int64_t e0 = (c - cb) * S::E;
     const int ne = int((b.ne - e0) < S::E ? (b.ne - e0) : S::E);
     mass3dpa_elements<D, D + 1, false>((gcdouble*)b.B, (gcdouble*)b.Bt, (gcdouble*)b.D, (gcdouble*)b.X, (gdouble*)b.Y, e0,
-                                ne, bufA, bufB, sB, sBt);
+                                ne, bufA, bufB);
     __syncthreads();  // the next chunk rewrites the LDS
   }
 }
@@ -452,8 +395,6 @@ __global__ __launch_bounds__(kBS) void mass3dpa_order_chunk_kernel(const char* _
   using S = MassShape<D, D + 1>;
   __shared__ double bufA[S::E * S::kA];
   __shared__ double bufB[S::E * S::kB];
-  __shared__ double sB[(D + 1) * D];
-  __shared__ double sBt[D * (D + 1)];
   const BatchHeader* hdr = reinterpret_cast<const BatchHeader*>(plan);
   const int64_t nchunks = hdr->nchunks, nbatch = hdr->nbatch;
   const int64_t c = hdr->order_begin[D] + blockIdx.x;
@@ -466,7 +407,7 @@ __global__ __launch_bounds__(kBS) void mass3dpa_order_chunk_kernel(const char* _
   const int64_t e0 = (c - chunk0[bi]) * S::E;
   const int ne = int((b.ne - e0) < S::E ? (b.ne - e0) : S::E);
   mass3dpa_elements<D, D + 1>((gcdouble*)b.B, (gcdouble*)b.Bt, (gcdouble*)b.D, (gcdouble*)b.X, (gdouble*)b.Y, e0,
-                              ne, bufA, bufB, sB, sBt);
+                              ne, bufA, bufB);
 }
 
 template <int D>
