@@ -7,15 +7,17 @@
 // work-items with 8-9 barriers (MASS3DPA-Hip.cpp:25-111,
 // DIFFUSION3DPA-Hip.cpp:25-134).
 //
-// MI355X design: a workgroup of 256 work-items owns E elements.  Each of the
-// six contraction stages maps one work-item to one 1D "pencil" of one element
+// MI355X design: a workgroup of 256 work-items owns E elements, as many as have
+// a work-item for every pencil of the widest stage.  Each of the six
+// contraction stages maps one work-item to one 1D "pencil" of one element
 // (e.g. the x-contraction to the (e,dz,dy) pencils), keeps the pencil in
-// registers and writes the stage result to LDS; stages are separated by
-// workgroup barriers, so a workgroup takes 6 barriers per E elements.  X and
+// registers and replaces it in LDS by its result; stages are separated by
+// workgroup barriers, so a workgroup takes 5 barriers per E elements.  X and
 // the quadrature data are read once with coalesced pencil loads, Y is
-// updated in place.  The contraction order of every stage and the
-// association of every sum are those of the Base_Seq loops and no
-// multiply-add is fused, so results are bit-identical to Base_Seq.
+// updated in place, the basis tables come through the scalar cache.  The
+// contraction order of every stage and the association of every sum are those
+// of the Base_Seq loops and no multiply-add is fused, so results are
+// bit-identical to Base_Seq.
 //
 // Stage order (forward x, y, z; backward x, y, z):
 //   P1 (e,dz,dy): DDQ[dz][dy][qx] = sum_dx X[dz][dy][dx] B(qx,dx)
@@ -38,12 +40,6 @@ using namespace rpx;
 namespace {
 
 constexpr int kBS = 256;
-constexpr int kLdsBudget = 48 * 1024;
-
-// A compiler barrier at the top of each pencil iteration of DIFFUSION3DPA: the
-// basis values are then re-read from LDS (a wavefront-uniform broadcast) for
-// every pencil instead of all of them being hoisted into registers.
-__device__ __forceinline__ void reload_basis() { asm volatile("" ::: "memory"); }
 
 // Global-memory pointers: with the address space in the type, accesses are
 // global (not FLAT) instructions even where the pointer comes from memory.
@@ -96,25 +92,24 @@ __device__ __forceinline__ void to_dofs(const double (&v)[Q], cdouble* T, double
 // of its bytes at 6.5 TB/s).  With as many elements as 24 to 48 KB of LDS hold
 // a stage took two passes, the second nearly empty, and fewer workgroups fit
 // on a CU: 278 / 312 / 317 us; with the basis in LDS as well 324 / 396 / 388 us.
+// (4,5) at NE = 600000: 281 us, 234 at 6.5 TB/s.
 template <int D, int Q>
 struct MassShape {
-  static constexpr int kA = Q * Q * Q;  // DDQ / QQQ / QDD per element
-  static constexpr int kB = D * Q * Q;  // DQQ / QQD per element
+  static constexpr int Q3 = Q * Q * Q;  // doubles of LDS per element
   static constexpr int E = kBS / (Q * Q);
-  static constexpr int kLds = E * (kA + kB);  // doubles of LDS
+  static constexpr int kLds = E * Q3;
 };
 
 // Elements [e0, e0+ne) of one operator application, ne <= MassShape::E, by
-// the whole workgroup, with two disjoint LDS buffers, bufA [E][kA] and
-// bufB [E][kB].  They are separate restrict parameters so the compiler may
-// reorder accesses between them.  Ends with the workgroup's last LDS reads
-// still pending: a caller that reuses the buffers must synchronise first.
+// the whole workgroup, in an LDS grid [qz][qy][qx] per element: every stage
+// reads and writes the same rows or columns of it, one work-item each, and
+// only their lengths change.  Ends with the workgroup's last LDS reads still
+// pending: a caller that reuses the buffer must synchronise first.
 template <int D, int Q, bool kEarlyXY = true>
 __device__ __forceinline__ void mass3dpa_elements(gcdouble* __restrict__ Bg, gcdouble* __restrict__ Btg,
                                                   gcdouble* __restrict__ Dg, gcdouble* __restrict__ Xg,
                                                   gdouble* __restrict__ Yg, int64_t e0, int ne,
-                                                  double* __restrict__ bufA, double* __restrict__ bufB) {
-  using S = MassShape<D, Q>;
+                                                  double* __restrict__ buf) {
   constexpr int D2 = D * D, D3 = D * D * D, Q2 = Q * Q, Q3 = Q * Q * Q;
   const int w = threadIdx.x;  // the pencil of every stage
   cdouble* const Bc = table(Bg);
@@ -148,81 +143,75 @@ __device__ __forceinline__ void mass3dpa_elements(gcdouble* __restrict__ Bg, gcd
     for (int qz = 0; qz < Q; ++qz) dq[qz] = dp[qz * Q2];
   }
 
-  // P1: x-contraction of X pencils.
+  // P1: x-contraction of X pencils, to row dy of plane dz.
   cdouble* T = opaque(Bc);
   if (w < ne * D2) {
     if constexpr (!kPreXY) load_x();
     double u[Q];
     to_quad<D, Q>(x, T, u);
-    double* out = bufA + w / D2 * S::kA + w % D2 * Q;  // DDQ[dz][dy][qx]
+    double* out = buf + w / D2 * Q3 + w % D2 / D * Q2 + w % D * Q;
 #pragma unroll
     for (int qx = 0; qx < Q; ++qx) out[qx] = u[qx];
   }
   __syncthreads();
-  // P2: y-contraction.
+  // P2: y-contraction, column qx of plane dz.
   T = opaque(Bc);
   if (w < ne * D * Q) {
-    const int e = w / (D * Q), r = w % (D * Q), dz = r / Q, qx = r % Q;
-    const double* in = bufA + e * S::kA + dz * D * Q + qx;  // DDQ[dz][dy][qx], stride Q in dy
+    const int e = w / (D * Q), r = w % (D * Q);
+    double* col = buf + e * Q3 + r / Q * Q2 + r % Q;
     double v[D], u[Q];
 #pragma unroll
-    for (int dy = 0; dy < D; ++dy) v[dy] = in[dy * Q];
+    for (int dy = 0; dy < D; ++dy) v[dy] = col[dy * Q];
     to_quad<D, Q>(v, T, u);
-    double* out = bufB + e * S::kB + dz * Q2 + qx;  // DQQ[dz][qy][qx], stride Q in qy
 #pragma unroll
-    for (int qy = 0; qy < Q; ++qy) out[qy * Q] = u[qy];
+    for (int qy = 0; qy < Q; ++qy) col[qy * Q] = u[qy];
   }
   __syncthreads();
-  // P3: z-contraction and the quadrature-point scaling.
+  // P3: z-contraction and the quadrature-point scaling, column (qy, qx).
   T = opaque(Bc);
   if (w < ne * Q2) {
-    const int e = w / Q2, r = w % Q2;         // r = qy*Q + qx
-    const double* in = bufB + e * S::kB + r;  // DQQ[dz][qy][qx], stride Q2 in dz
+    double* col = buf + w / Q2 * Q3 + w % Q2;
     double v[D], u[Q];
 #pragma unroll
-    for (int dz = 0; dz < D; ++dz) v[dz] = in[dz * Q2];
+    for (int dz = 0; dz < D; ++dz) v[dz] = col[dz * Q2];
     to_quad<D, Q>(v, T, u);
-    double* out = bufA + e * S::kA + r;  // QQQ[qz][qy][qx], stride Q2 in qz
 #pragma unroll
-    for (int qz = 0; qz < Q; ++qz) out[qz * Q2] = u[qz] * dq[qz];
+    for (int qz = 0; qz < Q; ++qz) col[qz * Q2] = u[qz] * dq[qz];
   }
   __syncthreads();
   if (kPreXY && w < ne * D2) load_y();
-  // P4: backward x-contraction.
+  // P4: backward x-contraction, row (qz, qy).
   T = opaque(Btc);
   if (w < ne * Q2) {
-    const int e = w / Q2, r = w % Q2;             // r = qz*Q + qy
-    const double* in = bufA + e * S::kA + r * Q;  // QQQ[qz][qy][qx], contiguous in qx
+    double* row = buf + w * Q;
     double v[Q], u[D];
 #pragma unroll
-    for (int qx = 0; qx < Q; ++qx) v[qx] = in[qx];
+    for (int qx = 0; qx < Q; ++qx) v[qx] = row[qx];
     to_dofs<D, Q>(v, T, u);
-    double* out = bufB + e * S::kB + r * D;  // QQD[qz][qy][dx]
 #pragma unroll
-    for (int dx = 0; dx < D; ++dx) out[dx] = u[dx];
+    for (int dx = 0; dx < D; ++dx) row[dx] = u[dx];
   }
   __syncthreads();
-  // P5: backward y-contraction.
+  // P5: backward y-contraction, column dx of plane qz.
   T = opaque(Btc);
   if (w < ne * Q * D) {
-    const int e = w / (Q * D), r = w % (Q * D), qz = r / D, dx = r % D;
-    const double* in = bufB + e * S::kB + qz * Q * D + dx;  // QQD[qz][qy][dx], stride D in qy
+    const int e = w / (Q * D), r = w % (Q * D);
+    double* col = buf + e * Q3 + r / D * Q2 + r % D;
     double v[Q], u[D];
 #pragma unroll
-    for (int qy = 0; qy < Q; ++qy) v[qy] = in[qy * D];
+    for (int qy = 0; qy < Q; ++qy) v[qy] = col[qy * Q];
     to_dofs<D, Q>(v, T, u);
-    double* out = bufA + e * S::kA + qz * D2 + dx;  // QDD[qz][dy][dx], stride D in dy
 #pragma unroll
-    for (int dy = 0; dy < D; ++dy) out[dy * D] = u[dy];
+    for (int dy = 0; dy < D; ++dy) col[dy * Q] = u[dy];
   }
   __syncthreads();
-  // P6: backward z-contraction, accumulate into Y.
+  // P6: backward z-contraction of column (dy, dx), accumulate into Y.
   T = opaque(Btc);
   if (w < ne * D2) {
-    const double* in = bufA + w / D2 * S::kA + w % D2;  // QDD[qz][dy][dx], stride D2 in qz
+    const double* col = buf + w / D2 * Q3 + w % D2 / D * Q + w % D;
     double v[Q], u[D];
 #pragma unroll
-    for (int qz = 0; qz < Q; ++qz) v[qz] = in[qz * D2];
+    for (int qz = 0; qz < Q; ++qz) v[qz] = col[qz * Q2];
     if constexpr (!kPreXY) load_y();
     to_dofs<D, Q>(v, T, u);
 #pragma unroll
@@ -237,11 +226,10 @@ __global__ __launch_bounds__(kBS) void mass3dpa_kernel(const double* __restrict_
                                                        const double* __restrict__ Xg, double* __restrict__ Yg,
                                                        int64_t NE) {
   using S = MassShape<D, Q>;
-  __shared__ double bufA[S::E * S::kA];
-  __shared__ double bufB[S::E * S::kB];
+  __shared__ double buf[S::kLds];
   const int64_t e0 = int64_t(blockIdx.x) * S::E;
   const int ne = int((NE - e0) < S::E ? (NE - e0) : S::E);
-  mass3dpa_elements<D, Q>((gcdouble*)Bg, (gcdouble*)Btg, (gcdouble*)Dg, (gcdouble*)Xg, (gdouble*)Yg, e0, ne, bufA, bufB);
+  mass3dpa_elements<D, Q>((gcdouble*)Bg, (gcdouble*)Btg, (gcdouble*)Dg, (gcdouble*)Xg, (gdouble*)Yg, e0, ne, buf);
 }
 
 // ---- ragged batches, one persistent launch ----------------------------------
@@ -268,12 +256,10 @@ __device__ __attribute__((noinline)) void mass_batch_chunk(rpx_mass_batch b, int
   using S = MassShape<D, D + 1>;
   static_assert(S::kLds <= kBatchLds, "LDS budget");
   const int ne = int((b.ne - e0) < S::E ? (b.ne - e0) : S::E);
-  double* bufA = (double*)lds;
-  double* bufB = bufA + S::E * S::kA;
   // The descriptors' pointers are global memory: typed so, the element code
   // issues global (not FLAT) accesses, which do not hold up its LDS waits.
   mass3dpa_elements<D, D + 1, false>((gcdouble*)b.B, (gcdouble*)b.Bt, (gcdouble*)b.D, (gcdouble*)b.X, (gdouble*)b.Y, e0, ne,
-                              bufA, bufB);
+                                    (double*)lds);
 }
 
 // Elements per chunk of a batch of order d1d (Q1D = d1d + 1).
@@ -356,8 +342,7 @@ __global__ __launch_bounds__(kBS, 3) void mass3dpa_batched_kernel(const char* __
 template <int D>
 __global__ __launch_bounds__(kBS) void mass3dpa_order_kernel(const char* __restrict__ plan) {
   using S = MassShape<D, D + 1>;
-  __shared__ double bufA[S::E * S::kA];
-  __shared__ double bufB[S::E * S::kB];
+  __shared__ double buf[S::kLds];
   const BatchHeader* hdr = reinterpret_cast<const BatchHeader*>(plan);
   const int64_t nchunks = hdr->nchunks, nbatch = hdr->nbatch;
   const int64_t begin = hdr->order_begin[D], end = hdr->order_end[D];
@@ -380,7 +365,7 @@ __global__ __launch_bounds__(kBS) void mass3dpa_order_kernel(const char* __restr
     const int64_t e0 = (c - cb) * S::E;
     const int ne = int((b.ne - e0) < S::E ? (b.ne - e0) : S::E);
     mass3dpa_elements<D, D + 1, false>((gcdouble*)b.B, (gcdouble*)b.Bt, (gcdouble*)b.D, (gcdouble*)b.X, (gdouble*)b.Y, e0,
-                                ne, bufA, bufB);
+                                ne, buf);
     __syncthreads();  // the next chunk rewrites the LDS
   }
 }
@@ -393,8 +378,7 @@ __global__ __launch_bounds__(kBS) void mass3dpa_order_kernel(const char* __restr
 template <int D>
 __global__ __launch_bounds__(kBS) void mass3dpa_order_chunk_kernel(const char* __restrict__ plan) {
   using S = MassShape<D, D + 1>;
-  __shared__ double bufA[S::E * S::kA];
-  __shared__ double bufB[S::E * S::kB];
+  __shared__ double buf[S::kLds];
   const BatchHeader* hdr = reinterpret_cast<const BatchHeader*>(plan);
   const int64_t nchunks = hdr->nchunks, nbatch = hdr->nbatch;
   const int64_t c = hdr->order_begin[D] + blockIdx.x;
@@ -407,7 +391,7 @@ __global__ __launch_bounds__(kBS) void mass3dpa_order_chunk_kernel(const char* _
   const int64_t e0 = (c - chunk0[bi]) * S::E;
   const int ne = int((b.ne - e0) < S::E ? (b.ne - e0) : S::E);
   mass3dpa_elements<D, D + 1>((gcdouble*)b.B, (gcdouble*)b.Bt, (gcdouble*)b.D, (gcdouble*)b.X, (gdouble*)b.Y, e0,
-                              ne, bufA, bufB);
+                              ne, buf);
 }
 
 template <int D>
@@ -569,237 +553,224 @@ __global__ __launch_bounds__(Q* Q) void mass3dpa_naive_kernel(const double* __re
 
 // ---- DIFFUSION3DPA ----------------------------------------------------------
 
+// Compile-time form of diffusion_tables: where in b or g the effective B(q,d)
+// or G(q,d) sits, and G's sign.
 template <int D, int Q>
-struct DiffShape {
-  static constexpr int kA = 3 * Q * Q * Q;
-  static constexpr int kB = 3 * D * Q * Q;
-  static constexpr int kBytes = 8 * (kA + kB);
-  static constexpr int E0 = kLdsBudget / kBytes;
-  static constexpr int E = E0 < 1 ? 1 : (E0 > 64 ? 64 : E0);
+struct HalfTables {
+  static constexpr int key(int q, int d) { return d * Q + q; }
+  static constexpr int sgn(int q, int d) { return q <= d ? -1 : 1; }
+  static constexpr int b_at(int q, int d) {
+    const int i = q <= d ? q : Q - 1 - q, j = q <= d ? d : D - 1 - d;
+    const int mi = Q - 1 - i, mj = D - 1 - j;
+    return key(i, j) > key(mi, mj) ? i + Q * j : mi + Q * mj;
+  }
+  static constexpr int g_at(int q, int d) {
+    const int k = q <= d ? Q - 1 - q : q, l = q <= d ? D - 1 - d : d;
+    const int nk = Q - 1 - k, nl = D - 1 - l;
+    return key(k, l) > key(nk, nl) ? k + Q * l : nk + Q * nl;
+  }
+  static constexpr int g_sign(int q, int d) {
+    const int k = q <= d ? Q - 1 - q : q, l = q <= d ? D - 1 - d : d;
+    const int nk = Q - 1 - k, nl = D - 1 - l;
+    return (key(k, l) > key(nk, nl) ? sgn(k, l) : sgn(nk, nl)) * sgn(q, d);
+  }
+  cdouble* b;
+  cdouble* g;
+  __device__ __forceinline__ double B(int q, int d) const { return b[b_at(q, d)]; }
+  __device__ __forceinline__ double G(int q, int d) const { return g_sign(q, d) < 0 ? -g[g_at(q, d)] : g[g_at(q, d)]; }
+  __device__ __forceinline__ HalfTables fresh() const { return {opaque(b), opaque(g)}; }
 };
 
+// The stages of the head of this file for three components, in one LDS grid of
+// Q^3 per element and component: every stage reads and writes the same rows
+// or columns of it, one work-item each, and only their lengths change, so no
+// second buffer is needed and E elements fill the workgroup's lanes (as in
+// MassShape).  What bounds it is the memory it moves, six tensor components
+// per point: NE = 200000 of (4,5) takes 263 us, 232 at 6.5 TB/s; with two
+// buffers, as many elements as 48 KB held and the basis in LDS it took 317.
+// (8,9), NE = 26041: 317 us against 907.
 template <int D, int Q, bool SYMM>
 __global__ __launch_bounds__(kBS) void diffusion3dpa_kernel(const double* __restrict__ Bg,
                                                             const double* __restrict__ Gg,
                                                             const double* __restrict__ Dg,
                                                             const double* __restrict__ Xg,
                                                             double* __restrict__ Yg, int64_t NE) {
-  using S = DiffShape<D, Q>;
-  constexpr int E = S::E;
+  constexpr int E = kBS / (Q * Q);
   constexpr int D2 = D * D, D3 = D * D * D, Q2 = Q * Q, Q3 = Q * Q * Q;
   constexpr int NC = SYMM ? 6 : 9;
-  constexpr int A1 = Q3, B1 = D * Q2;  // per-component strides within an element
-  __shared__ double bufA[E * S::kA];
-  __shared__ double bufB[E * S::kB];
-  __shared__ double sB[Q * D];  // sB[q*D + d] = effective B(q,d)
-  __shared__ double sG[Q * D];  // sG[q*D + d] = effective G(q,d) with the reader's sign
+  constexpr int K = 3 * Q3;  // doubles of an element; a component's stage result takes Q3 of them
+  __shared__ double buf[E * K];
+  const HalfTables<D, Q> tables{table((gcdouble*)Bg), table((gcdouble*)Gg)};
 
-  const int tid = threadIdx.x;
+  const int w = threadIdx.x;  // the pencil of every stage
   const int64_t e0 = int64_t(blockIdx.x) * E;
   const int ne = int((NE - e0) < E ? (NE - e0) : E);
+  const bool in1 = w < ne * D2, in2 = w < ne * D * Q, in3 = w < ne * Q2;
 
-  for (int t = tid; t < Q * D; t += kBS) {
-    const int q = t / D, d = t % D;
-    double be, ge;
-    diffusion_tables(q, d, Q, D, Bg, Gg, &be, &ge);
-    sB[t] = be;
-    sG[t] = ge;
-  }
-  // Register budget.  Hoisting the 2*Q*D basis values out of the pencil
-  // loops costs more VGPRs than it saves LDS reads here (each basis read
-  // feeds three components), so every pencil iteration re-reads them from
-  // LDS (a wavefront-uniform broadcast); the registers go to the work-item's
-  // D values, loaded before P1 so that their latency overlaps two stages.
-  // Measured at NE = 262144 (65536 for D1D >= 5): (4,5) 0.447 -> 0.408 ms
-  // with uniform D, 0.49 -> 0.47 ms with the symmetric-tensor D of the
-  // roofline report (160 VGPRs, three wavefronts per SIMD; prefetching D
-  // alone took 232); (5,6) 0.404 -> 0.237 ms; (6,7) 0.651 -> 0.438 ms.  The
-  // non-symmetric (4,5) case, which has no prefetch, was 2% slower
-  // re-reading, so it keeps the hoist below D1D = 5.
-  constexpr bool kReload = SYMM || D >= 5;
-  constexpr bool kPreD = SYMM && E * Q2 <= kBS;  // one P3 pencil per work-item
-  double dpre[kPreD ? 6 : 1][Q];
-  if constexpr (kPreD) {
-    if (tid < ne * Q2) {
-      const int e = tid / Q2, r = tid % Q2;
-      const double* dp = Dg + (e0 + e) * (NC * Q3) + r;
-#pragma unroll
-      for (int c = 0; c < 6; ++c)
-#pragma unroll
-        for (int qz = 0; qz < Q; ++qz) dpre[c][qz] = dp[c * Q3 + qz * Q2];
-    }
-  }
-  __syncthreads();
-
-  // P1 (DIFFUSION3DPA_3): DDQ0 = sum X*B, DDQ1 = sum X*G over dx.
-  for (int w = tid; w < ne * D2; w += kBS) {
-    if constexpr (kReload) reload_basis();
-    const int e = w / D2, r = w % D2, dz = r / D, dy = r % D;
-    const double* xp = Xg + (e0 + e) * D3 + dz * D2 + dy * D;
-    double x[D];
+  // The point's tensor is loaded before P1 where it fits in the registers: (6,7)
+  // 298 -> 258 us at NE = 61728; (8,9) 317 -> 332 at NE = 26041.
+  constexpr bool kPreD = SYMM && Q <= 7;
+  // From D1D = 7 the tables overflow the SGPRs; they are then re-read per row.
+  constexpr bool kPerRow = D >= 7;
+  double x[D], y[D], o[kPreD ? 6 : 1][Q];
+  const double* const dp = Dg + (e0 + w / Q2) * (NC * Q3) + w % Q2;
+  if (in1) {
+    const double* xp = Xg + (e0 + w / D2) * D3 + w % D2 * D;
 #pragma unroll
     for (int dx = 0; dx < D; ++dx) x[dx] = xp[dx];
-    double* out = bufA + e * S::kA + (dz * D + dy) * Q;
+  }
+  if (kPreD && in3) {
 #pragma unroll
-    for (int qx = 0; qx < Q; ++qx) {
-      double u = 0.0, v = 0.0;
+    for (int c = 0; c < (kPreD ? 6 : 1); ++c)
 #pragma unroll
-      for (int dx = 0; dx < D; ++dx) {
-        u += x[dx] * sB[qx * D + dx];
-        v += x[dx] * sG[qx * D + dx];
+      for (int qz = 0; qz < Q; ++qz) o[c][qz] = dp[c * Q3 + qz * Q2];
+  }
+
+  // P1 (DIFFUSION3DPA_3): DDQ0 = sum X*B, DDQ1 = sum X*G over dx.
+  if (in1) {
+    auto T = tables.fresh();
+    double u[Q], v[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) u[q] = v[q] = 0.0;
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (kPerRow) T = tables.fresh();
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        u[q] += x[d] * T.B(q, d);
+        v[q] += x[d] * T.G(q, d);
       }
-      out[qx] = u;
-      out[A1 + qx] = v;
+    }
+    double* out = buf + w / D2 * K + w % D2 / D * Q2 + w % D * Q;  // rows dy of plane dz
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      out[q] = u[q];
+      out[Q3 + q] = v[q];
     }
   }
   __syncthreads();
   // P2 (DIFFUSION3DPA_4): DQQ0 = sum DDQ1*B, DQQ1 = sum DDQ0*G, DQQ2 = sum DDQ0*B over dy.
-  for (int w = tid; w < ne * D * Q; w += kBS) {
-    if constexpr (kReload) reload_basis();
-    const int e = w / (D * Q), r = w % (D * Q), dz = r / Q, qx = r % Q;
-    const double* in = bufA + e * S::kA + dz * D * Q + qx;
-    double a0[D], a1[D];
+  if (in2) {
+    const int e = w / (D * Q), r = w % (D * Q);
+    double* col = buf + e * K + r / Q * Q2 + r % Q;  // column qx of plane dz
+    double a0[D], a1[D], u[Q], v[Q], t[Q];
 #pragma unroll
-    for (int dy = 0; dy < D; ++dy) {
-      a0[dy] = in[dy * Q];
-      a1[dy] = in[A1 + dy * Q];
+    for (int d = 0; d < D; ++d) {
+      a0[d] = col[d * Q];
+      a1[d] = col[Q3 + d * Q];
     }
-    double* out = bufB + e * S::kB + dz * Q2 + qx;
+    auto T = tables.fresh();
 #pragma unroll
-    for (int qy = 0; qy < Q; ++qy) {
-      double u = 0.0, v = 0.0, ww = 0.0;
+    for (int q = 0; q < Q; ++q) u[q] = v[q] = t[q] = 0.0;
 #pragma unroll
-      for (int dy = 0; dy < D; ++dy) {
-        u += a1[dy] * sB[qy * D + dy];
-        v += a0[dy] * sG[qy * D + dy];
-        ww += a0[dy] * sB[qy * D + dy];
+    for (int d = 0; d < D; ++d) {
+      if (kPerRow) T = tables.fresh();
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        u[q] += a1[d] * T.B(q, d);
+        v[q] += a0[d] * T.G(q, d);
+        t[q] += a0[d] * T.B(q, d);
       }
-      out[qy * Q] = u;
-      out[B1 + qy * Q] = v;
-      out[2 * B1 + qy * Q] = ww;
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      col[q * Q] = u[q];
+      col[Q3 + q * Q] = v[q];
+      col[2 * Q3 + q * Q] = t[q];
     }
   }
   __syncthreads();
   // P3 (DIFFUSION3DPA_5): gradient at the point, times the symmetric tensor.
-  for (int w = tid; w < ne * Q2; w += kBS) {
-    if constexpr (kReload) reload_basis();
-    const int e = w / Q2, r = w % Q2;
-    const double* in = bufB + e * S::kB + r;
+  if (in3) {
+    double* col = buf + w / Q2 * K + w % Q2;
     double c0[D], c1[D], c2[D];
 #pragma unroll
-    for (int dz = 0; dz < D; ++dz) {
-      c0[dz] = in[dz * Q2];
-      c1[dz] = in[B1 + dz * Q2];
-      c2[dz] = in[2 * B1 + dz * Q2];
+    for (int d = 0; d < D; ++d) {
+      c0[d] = col[d * Q2];
+      c1[d] = col[Q3 + d * Q2];
+      c2[d] = col[2 * Q3 + d * Q2];
     }
-    const double* dp = Dg + (e0 + e) * (NC * Q3) + r;
-    double* out = bufA + e * S::kA + r;
+    auto T = tables.fresh();
 #pragma unroll
-    for (int qz = 0; qz < Q; ++qz) {
-      double u = 0.0, v = 0.0, ww = 0.0;
+    for (int q = 0; q < Q; ++q) {
+      if (kPerRow) T = tables.fresh();
+      double u = 0.0, v = 0.0, t = 0.0;
 #pragma unroll
-      for (int dz = 0; dz < D; ++dz) {
-        u += c0[dz] * sB[qz * D + dz];
-        v += c1[dz] * sB[qz * D + dz];
-        ww += c2[dz] * sG[qz * D + dz];
+      for (int d = 0; d < D; ++d) {
+        u += c0[d] * T.B(q, d);
+        v += c1[d] * T.B(q, d);
+        t += c2[d] * T.G(q, d);
       }
-      const double* o = dp + qz * Q2;
+      const double* op = dp + q * Q2;
       // Symmetric storage order (11, 12, 13, 22, 23, 33), DIFFUSION3DPA.hpp:384-392.
-      const double O11 = kPreD ? dpre[0][qz] : o[0];
-      const double O12 = kPreD ? dpre[1][qz] : o[Q3];
-      const double O13 = kPreD ? dpre[2][qz] : o[2 * Q3];
-      const double O21 = SYMM ? O12 : o[3 * Q3];
-      const double O22 = kPreD ? dpre[3][qz] : (SYMM ? o[3 * Q3] : o[4 * Q3]);
-      const double O23 = kPreD ? dpre[4][qz] : (SYMM ? o[4 * Q3] : o[5 * Q3]);
-      const double O31 = SYMM ? O13 : o[6 * Q3];
-      const double O32 = SYMM ? O23 : o[7 * Q3];
-      const double O33 = kPreD ? dpre[5][qz] : (SYMM ? o[5 * Q3] : o[8 * Q3]);
-      out[qz * Q2] = ((O11 * u) + (O12 * v)) + (O13 * ww);
-      out[A1 + qz * Q2] = ((O21 * u) + (O22 * v)) + (O23 * ww);
-      out[2 * A1 + qz * Q2] = ((O31 * u) + (O32 * v)) + (O33 * ww);
+      const double O11 = kPreD ? o[0][q] : op[0];
+      const double O12 = kPreD ? o[kPreD ? 1 : 0][q] : op[Q3];
+      const double O13 = kPreD ? o[kPreD ? 2 : 0][q] : op[2 * Q3];
+      const double O21 = SYMM ? O12 : op[3 * Q3];
+      const double O22 = kPreD ? o[kPreD ? 3 : 0][q] : (SYMM ? op[3 * Q3] : op[4 * Q3]);
+      const double O23 = kPreD ? o[kPreD ? 4 : 0][q] : (SYMM ? op[4 * Q3] : op[5 * Q3]);
+      const double O31 = SYMM ? O13 : op[6 * Q3];
+      const double O32 = SYMM ? O23 : op[7 * Q3];
+      const double O33 = kPreD ? o[kPreD ? 5 : 0][q] : (SYMM ? op[5 * Q3] : op[8 * Q3]);
+      col[q * Q2] = ((O11 * u) + (O12 * v)) + (O13 * t);
+      col[Q3 + q * Q2] = ((O21 * u) + (O22 * v)) + (O23 * t);
+      col[2 * Q3 + q * Q2] = ((O31 * u) + (O32 * v)) + (O33 * t);
     }
   }
   __syncthreads();
-  // P4 (DIFFUSION3DPA_7): QQD0 = sum QQQ0*Gt, QQD1 = sum QQQ1*Bt, QQD2 = sum QQQ2*Bt over qx.
-  for (int w = tid; w < ne * Q2; w += kBS) {
-    if constexpr (kReload) reload_basis();
-    const int e = w / Q2, r = w % Q2;  // r = qz*Q + qy
-    const double* in = bufA + e * S::kA + r * Q;
-    double c0[Q], c1[Q], c2[Q];
+  double* const yp = Yg + (e0 + w / D2) * D3 + w % D2;
+  if (in1) {
 #pragma unroll
-    for (int qx = 0; qx < Q; ++qx) {
-      c0[qx] = in[qx];
-      c1[qx] = in[A1 + qx];
-      c2[qx] = in[2 * A1 + qx];
+    for (int dz = 0; dz < D; ++dz) y[dz] = yp[dz * D2];
+  }
+  // Backward stages: component c's pencil times G where c == gc, B elsewhere.
+  auto back = [&](const double* in, int stride, int gc, double (&u)[3][D]) {
+    double c[3][Q];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int q = 0; q < Q; ++q) c[k][q] = in[k * Q3 + q * stride];
+    auto T = tables.fresh();
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (kPerRow) T = tables.fresh();
+      u[0][d] = u[1][d] = u[2][d] = 0.0;
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) u[k][d] += c[k][q] * (k == gc ? T.G(q, d) : T.B(q, d));
     }
-    double* out = bufB + e * S::kB + r * D;
+  };
+  double u[3][D];
+  // P4 (DIFFUSION3DPA_7): QQD0 = sum QQQ0*Gt, QQD1 = sum QQQ1*Bt, QQD2 = sum QQQ2*Bt
+  // over qx, row r = qz*Q + qy.
+  if (in3) {
+    double* row = buf + w / Q2 * K + w % Q2 * Q;
+    back(row, 1, 0, u);
 #pragma unroll
-    for (int dx = 0; dx < D; ++dx) {
-      double u = 0.0, v = 0.0, ww = 0.0;
+    for (int k = 0; k < 3; ++k)
 #pragma unroll
-      for (int qx = 0; qx < Q; ++qx) {
-        u += c0[qx] * sG[qx * D + dx];
-        v += c1[qx] * sB[qx * D + dx];
-        ww += c2[qx] * sB[qx * D + dx];
-      }
-      out[dx] = u;
-      out[B1 + dx] = v;
-      out[2 * B1 + dx] = ww;
-    }
+      for (int d = 0; d < D; ++d) row[k * Q3 + d] = u[k][d];
   }
   __syncthreads();
-  // P5 (DIFFUSION3DPA_8): QDD0 = sum QQD0*Bt, QDD1 = sum QQD1*Gt, QDD2 = sum QQD2*Bt over qy.
-  for (int w = tid; w < ne * Q * D; w += kBS) {
-    if constexpr (kReload) reload_basis();
+  // P5 (DIFFUSION3DPA_8): QDD0 = sum QQD0*Bt, QDD1 = sum QQD1*Gt, QDD2 = sum QQD2*Bt
+  // over qy, column dx of plane qz.
+  if (in2) {
     const int e = w / (Q * D), r = w % (Q * D), qz = r / D, dx = r % D;
-    const double* in = bufB + e * S::kB + qz * Q * D + dx;
-    double c0[Q], c1[Q], c2[Q];
+    double* col = buf + e * K + qz * Q2 + dx;
+    back(col, Q, 1, u);
 #pragma unroll
-    for (int qy = 0; qy < Q; ++qy) {
-      c0[qy] = in[qy * D];
-      c1[qy] = in[B1 + qy * D];
-      c2[qy] = in[2 * B1 + qy * D];
-    }
-    double* out = bufA + e * S::kA + qz * D2 + dx;
+    for (int k = 0; k < 3; ++k)
 #pragma unroll
-    for (int dy = 0; dy < D; ++dy) {
-      double u = 0.0, v = 0.0, ww = 0.0;
-#pragma unroll
-      for (int qy = 0; qy < Q; ++qy) {
-        u += c0[qy] * sB[qy * D + dy];
-        v += c1[qy] * sG[qy * D + dy];
-        ww += c2[qy] * sB[qy * D + dy];
-      }
-      out[dy * D] = u;
-      out[A1 + dy * D] = v;
-      out[2 * A1 + dy * D] = ww;
-    }
+      for (int d = 0; d < D; ++d) col[k * Q3 + d * Q] = u[k][d];
   }
   __syncthreads();
   // P6 (DIFFUSION3DPA_9): sum over qz, Y += (u + v) + w.
-  for (int w = tid; w < ne * D2; w += kBS) {
-    if constexpr (kReload) reload_basis();
-    const int e = w / D2, r = w % D2;
-    const double* in = bufA + e * S::kA + r;
-    double c0[Q], c1[Q], c2[Q];
+  if (in1) {
+    const int r = w % D2;
+    back(buf + w / D2 * K + r / D * Q + r % D, Q2, 2, u);
 #pragma unroll
-    for (int qz = 0; qz < Q; ++qz) {
-      c0[qz] = in[qz * D2];
-      c1[qz] = in[A1 + qz * D2];
-      c2[qz] = in[2 * A1 + qz * D2];
-    }
-    double* yp = Yg + (e0 + e) * D3 + r;
-#pragma unroll
-    for (int dz = 0; dz < D; ++dz) {
-      double u = 0.0, v = 0.0, ww = 0.0;
-#pragma unroll
-      for (int qz = 0; qz < Q; ++qz) {
-        u += c0[qz] * sB[qz * D + dz];
-        v += c1[qz] * sB[qz * D + dz];
-        ww += c2[qz] * sG[qz * D + dz];
-      }
-      yp[dz * D2] += (u + v) + ww;
-    }
+    for (int dz = 0; dz < D; ++dz) yp[dz * D2] = y[dz] + ((u[0][dz] + u[1][dz]) + u[2][dz]);
   }
 }
 
@@ -840,7 +811,7 @@ template <int D, bool SYMM>
 int launch_diff(const double* B, const double* G, const double* Dq, const double* X, double* Y, int64_t NE,
                 hipStream_t s) {
   constexpr int Q = D + 1;
-  const int64_t grid = ceil_div(NE, DiffShape<D, Q>::E);
+  const int64_t grid = ceil_div(NE, kBS / (Q * Q));
   if (grid > INT32_MAX) return RPX_ERR_UNSUPPORTED;
   diffusion3dpa_kernel<D, Q, SYMM><<<dim3(unsigned(grid)), dim3(kBS), 0, s>>>(B, G, Dq, X, Y, NE);
   return launch_status();
