@@ -22,12 +22,11 @@
 //    look-back always makes progress.  (A ticket counter taken with one
 //    atomic per tile serialises on its single address -- measured 5.5 ms
 //    against 0.8 ms for 2^28 doubles on MI355X.)
-//  * the look-back is done by one wavefront over windows of 64
-//    predecessors; flags carry a tag (header epoch + 1) so the scratch needs
-//    no clearing between calls.  The last tile advances the epoch after its
-//    look-back:
-//    by then every tile has published a flag, so every tile has read the
-//    epoch;
+//  * the look-back is done by the whole workgroup where there are few tiles
+//    and by one wavefront where there are many; a tile's words carry a tag (header epoch + 1) so the scratch
+//    needs no clearing between calls.  The last tile advances the epoch after
+//    its look-back: by then every tile has published, so every tile has read
+//    the epoch;
 //  * every spin is bounded; a wait that expires records RPX_ERR_WAIT_EXPIRED
 //    in the scratch header and the kernel still runs to completion.
 #include "rpx_common.hpp"
@@ -49,34 +48,73 @@ struct ScanHeader {
 constexpr size_t kHeaderBytes = 256;
 constexpr int kBS = 256;
 constexpr int kDefaultIPT = 64;
-constexpr int kDefaultScanBS = 256;  // work-items per tile (256 or 512)
 constexpr int kMinTile = kBS * 16;  // scratch is sized for the smallest tile
 constexpr unsigned kSpinLimit = 1u << 22;
+constexpr int64_t kWideTiles = 512;  // up to here the whole workgroup looks back
 
-// All look-back state (flags and values) moves through agent-scope atomic
-// loads and stores, which gfx950 performs coherently across the XCDs' L2s
-// (sc1).  Publishing a value before its flag therefore needs only the value
-// store to have completed (s_waitcnt vmcnt(0)) -- not the L2 write-back that
-// an agent-scope release fence would issue, which would also flush every
-// dirty output line of the XCD.  On the reading side the value load is only
-// issued after the flag load has returned and been tested.
-__device__ __forceinline__ unsigned long long load_flag(const unsigned long long* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// A tile's look-back state is three 64-bit words.  All move through
+// agent-scope atomic loads and stores, which gfx950 performs coherently across
+// the XCDs' L2s (sc1), and carry a 42-bit tag (epoch and status) in their top
+// bits.
+//
+// Many tiles: word 0 is a flag, the tag alone, words 1 and 2 the aggregate and
+// the inclusive prefix.  Publishing a value before its flag needs only the
+// value store to have completed (s_waitcnt vmcnt(0)), not the L2 write-back
+// of an agent-scope release fence, which would also flush every dirty output
+// line of the XCD; a reader asks for the value once it has the flag.  The
+// values are stored complemented: no sum then looks like a tag.
+//
+// Few tiles (WIDE): each word is the tag over 22 or 21 bits of the value, so
+// the writer waits for nothing and a reader takes all three in one round trip
+// and retries until their tags agree.  1M doubles as 245 tiles: 8.6 us with
+// flags, 5.8 us so and with the whole workgroup looking back.  At 2^28 this
+// costs more traffic than it saves waiting: 0.77 against 0.71 ms.
+struct TileWords {
+  unsigned long long *w0, *w1, *w2;  // [tile]
+};
+constexpr int kLowBits = 21;  // of words 1 and 2; word 0 holds the top 22
+constexpr unsigned long long kLowMask = (1ull << kLowBits) - 1;
+
+__device__ __forceinline__ unsigned long long tile_tag(unsigned long long epoch, unsigned status) {
+  return (epoch << 2 | status) << 22;
 }
-__device__ __forceinline__ void store_flag(unsigned long long* p, unsigned long long v) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // compiler ordering
-  __builtin_amdgcn_s_waitcnt(0x0F70);                      // vmcnt(0): value store complete
+__device__ __forceinline__ void store_word(unsigned long long* p, unsigned long long v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ double load_value(const double* p) {
-  unsigned long long bits =
-      __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return __longlong_as_double(static_cast<long long>(bits));
+__device__ __forceinline__ unsigned long long load_word(const unsigned long long* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void store_value(double* p, double v) {
-  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p),
-                     static_cast<unsigned long long>(__double_as_longlong(v)), __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ unsigned long long bits(double v) {
+  return static_cast<unsigned long long>(__double_as_longlong(v));
+}
+__device__ __forceinline__ double value(unsigned long long b) { return __longlong_as_double(static_cast<long long>(b)); }
+
+template <bool WIDE>
+__device__ __forceinline__ void publish(const TileWords& w, int64_t t, unsigned long long epoch, unsigned status,
+                                        double v) {
+  const unsigned long long b = bits(v), tag = tile_tag(epoch, status);
+  if constexpr (WIDE) {
+    store_word(&w.w0[t], tag | b >> (2 * kLowBits));
+    store_word(&w.w1[t], tag | (b >> kLowBits & kLowMask));
+    store_word(&w.w2[t], tag | (b & kLowMask));
+  } else {
+    store_word(status == 2 ? &w.w2[t] : &w.w1[t], ~b);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // compiler ordering
+    __builtin_amdgcn_s_waitcnt(0x0F70);                      // vmcnt(0): value store complete
+    store_word(&w.w0[t], tag);
+  }
+}
+// The status of tile k in this epoch, 0 if it has none yet (or, WIDE, is being
+// rewritten); WIDE: *v is its value.
+template <bool WIDE>
+__device__ __forceinline__ unsigned look(const TileWords& w, int64_t k, unsigned long long epoch, double* v) {
+  const unsigned long long a = load_word(&w.w0[k]), tag = a >> 22;
+  if constexpr (WIDE) {
+    const unsigned long long b = load_word(&w.w1[k]), c = load_word(&w.w2[k]);
+    if (b >> 22 != tag || c >> 22 != tag) return 0;
+    *v = value((a & 0x3FFFFFull) << (2 * kLowBits) | (b & kLowMask) << kLowBits | (c & kLowMask));
+  }
+  return tag >> 2 == epoch ? unsigned(tag & 3) : 0;
 }
 
 // Wavefront scans on DPP lane moves (VALU only, no LDS round trips).  A
@@ -120,6 +158,38 @@ __device__ __forceinline__ double lane_value(double v) {
 }
 __device__ __forceinline__ double last_lane(double v) { return lane_value<kWave - 1>(v); }
 
+// One wavefront's look at the 64 tiles top, top - 1, ... (tiles before `first`
+// count as an inclusive prefix of zero): the sum of their values back to and
+// with the nearest inclusive one, *done if there is one.
+template <bool WIDE>
+__device__ __forceinline__ double look_window(const TileWords& words, int64_t top, int64_t first,
+                                              unsigned long long epoch, int lane, bool* done, bool* expired) {
+  const int64_t k = top - lane;
+  double val = 0.0;
+  unsigned status = 2;
+  if (k >= first) {
+    unsigned spins = 0;
+    while ((status = look<WIDE>(words, k, epoch, &val)) == 0) {
+      if (++spins > kSpinLimit) {
+        *expired = true;
+        status = 2;
+        val = 0.0;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");  // value loads stay after the flag tests
+  const unsigned long long inc = __ballot(status == 2);
+  const int last = inc ? __ffsll(static_cast<long long>(inc)) - 1 : kWave;
+  *done = inc != 0;
+  if (!WIDE && k >= first && !*expired) {
+    if (lane < last) val = value(~load_word(&words.w1[k]));
+    else if (lane == last) val = value(~load_word(&words.w2[k]));
+  }
+  return wave_sum(lane <= last ? val : 0.0);
+}
+
 // Segment tables of a segmented scan: segment s covers [off[s], off[s+1])
 // and owns the global tiles [tile0[s], tile0[s+1]); tile t belongs to
 // segment tile_seg[t].  A segment's tiles start at even elements (the
@@ -132,22 +202,21 @@ struct SegTables {
   const int* tile_seg;
 };
 
-// SEG = false: one array of n elements, tile t covers [t*T, t*T + T), flags
+// SEG = false: one array of n elements, tile t covers [t*T, t*T + T), words
 // carry the epoch read from the header.  SEG = true: tiles come from the
 // segment tables, the look-back stops at the segment's first tile, and the
-// flags were cleared before the launch (epoch 0, no epoch advance).
-template <int BS, int ROWS, bool NT, bool SEG, bool INCL = false>  // 16-byte rows per lane: 128*ROWS doubles a wave
+// words were cleared before the launch (epoch 0, no epoch advance).
+template <int BS, int ROWS, bool NT, bool SEG, bool INCL, bool WIDE>  // 16-byte rows per lane: 128*ROWS doubles a wave
 __global__ __launch_bounds__(BS) void scan_kernel(const double* x, double* y, int64_t n, int64_t ntiles,
-                                                   ScanHeader* __restrict__ hdr,
-                                                   unsigned long long* __restrict__ flags,
-                                                   double* __restrict__ aggs, double* __restrict__ incls,
-                                                   int vec, SegTables seg) {
+                                                   ScanHeader* __restrict__ hdr, TileWords words, int vec,
+                                                   SegTables seg) {
   constexpr int kRowLen = 2 * kWave;            // doubles per wavefront row
   constexpr int kChunk = kRowLen * ROWS;        // doubles per wavefront
   constexpr int kTileN = kChunk * (BS / kWave);
   __shared__ double wave_tot[BS / kWave];
   __shared__ unsigned long long s_epoch;
-  __shared__ double s_prefix;
+  __shared__ double look_sum[2][BS / kWave];
+  __shared__ int look_done[2][BS / kWave];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -210,10 +279,10 @@ __global__ __launch_bounds__(BS) void scan_kernel(const double* x, double* y, in
   }
   if (lane == 0) wave_tot[wave] = carry;
   __syncthreads();
-  // Flag tag: 0 for the segmented form (its flags are cleared before every
-  // launch), epoch + 1 for the single-array form, so a single-array scan
-  // never accepts a flag a segmented call left in a shared scratch.
-  const unsigned long long E = SEG ? 0ull : s_epoch + 1;
+  // Epoch: 0 for the segmented form (its words are cleared before every
+  // launch), the header's + 1 for the single-array form, so a single-array scan
+  // never accepts a word a segmented call left in a shared scratch.
+  const unsigned long long E = SEG ? 0ull : (s_epoch + 1) & 0xFFFFFFFFFFull;
   double wave_off = 0.0, tile_agg = 0.0;
 #pragma unroll
   for (int w = 0; w < BS / kWave; ++w) {
@@ -221,65 +290,51 @@ __global__ __launch_bounds__(BS) void scan_kernel(const double* x, double* y, in
     if (w < wave) wave_off += wt;
     tile_agg += wt;
   }
+  if (tid == 0) publish<WIDE>(words, t, E, t == first ? 2 : 1, tile_agg);
 
-  // Publish the aggregate, then look back (wavefront 0).
-  if (wave == 0) {
-    if (t == first) {
+  // Look back.  Few tiles all publish at about the same time, so there the
+  // whole workgroup looks, BS predecessors per round; many tiles find an
+  // inclusive prefix close by, and wavefront 0 looks alone (looking BS back at
+  // 2^28 doubles waits for tiles it does not need, and took 1.00 ms).
+  double prefix = 0.0;
+  if (WIDE && t != first) {
+    bool expired = false;
+    int64_t top = t - 1;
+    for (int round = 0;; round ^= 1, top -= BS) {
+      bool done;
+      const double sum = look_window<true>(words, top - int64_t(wave) * kWave, first, E, lane, &done, &expired);
       if (lane == 0) {
-        store_value(&incls[t], tile_agg);
-        store_flag(&flags[t], (E << 2) | 2ull);
-        s_prefix = 0.0;
+        look_sum[round][wave] = sum;
+        look_done[round][wave] = done;
       }
-    } else {
-      if (lane == 0) {
-        store_value(&aggs[t], tile_agg);
-        store_flag(&flags[t], (E << 2) | 1ull);
+      __syncthreads();
+      done = false;
+#pragma unroll
+      for (int w = 0; w < BS / kWave; ++w) {
+        if (!done) prefix += look_sum[round][w];
+        done |= look_done[round][w] != 0;
       }
-      double excl = 0.0;
-      int64_t top = t - 1;
-      bool expired = false;
-      while (true) {
-        const int64_t k = top - lane;
-        unsigned status = 2;  // before the first tile: an inclusive prefix of zero
-        if (k >= first) {
-          unsigned spins = 0;
-          while (true) {
-            const unsigned long long f = load_flag(&flags[k]);
-            status = static_cast<unsigned>(f & 3ull);
-            if ((f >> 2) == E && status != 0) break;
-            if (++spins > kSpinLimit) {
-              expired = true;
-              status = 2;
-              break;
-            }
-            __builtin_amdgcn_s_sleep(1);
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");  // value loads stay after the flag tests
-        const unsigned long long inc_mask = __ballot(status == 2);
-        const int first_inc = inc_mask ? (__ffsll(static_cast<long long>(inc_mask)) - 1) : kWave;
-        double val = 0.0;
-        if (k >= first && !expired) {
-          if (lane < first_inc) val = load_value(&aggs[k]);
-          else if (lane == first_inc) val = load_value(&incls[k]);
-        }
-        excl += wave_sum(val);
-        if (inc_mask) break;
-        top -= kWave;
-      }
-      if (__ballot(expired) != 0 && lane == 0) atomicOr(&hdr->error, 1u);
-      if (lane == 0) {
-        store_value(&incls[t], excl + tile_agg);
-        store_flag(&flags[t], (E << 2) | 2ull);
-        s_prefix = excl;
-      }
+      if (done) break;
     }
-    // Every tile has read the epoch once the last tile's look-back is done.
-    if (!SEG && lane == 0 && t == ntiles - 1) atomicAdd(&hdr->epoch, 1ull);
+    if (tid == 0) publish<WIDE>(words, t, E, 2, prefix + tile_agg);
+    if (expired) atomicOr(&hdr->error, 1u);
+  } else if (t != first) {
+    if (wave == 0) {
+      bool expired = false, done = false;
+      for (int64_t top = t - 1; !done; top -= kWave) prefix += look_window<false>(words, top, first, E, lane, &done, &expired);
+      if (lane == 0) {
+        publish<WIDE>(words, t, E, 2, prefix + tile_agg);
+        look_sum[0][0] = prefix;
+      }
+      if (expired) atomicOr(&hdr->error, 1u);
+    }
+    __syncthreads();
+    prefix = look_sum[0][0];
   }
-  __syncthreads();
+  // Every tile has read the epoch once the last tile's look-back is done.
+  if (!SEG && tid == 0 && t == ntiles - 1) atomicAdd(&hdr->epoch, 1ull);
 
-  const double off = s_prefix + wave_off;
+  const double off = prefix + wave_off;
   // The inclusive value of an element is the exclusive value of the element
   // after it: for lane l's pair, its own second value and lane l+1's first
   // (for lane 63 the next row's first, after the last row the wavefront's
@@ -316,16 +371,16 @@ __global__ void zero_kernel(unsigned* p, int64_t nwords) {
   for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < nwords; i += stride) p[i] = 0u;
 }
 
-// Before a segmented scan: clears the flags and fills tile_seg from tile0
+// Before a segmented scan: clears the tiles' words and fills tile_seg from tile0
 // (the last segment whose first tile is <= t owns tile t; empty segments
 // share their first tile with the next segment and so are never chosen).
-__global__ __launch_bounds__(256) void seg_prep_kernel(unsigned* __restrict__ flag_words, int64_t nwords,
+__global__ __launch_bounds__(256) void seg_prep_kernel(unsigned* __restrict__ words, int64_t nwords,
                                                        const int64_t* __restrict__ tile0, int nseg,
                                                        int* __restrict__ tile_seg, int64_t ntiles) {
   const int64_t stride = int64_t(gridDim.x) * blockDim.x;
   const int64_t end = nwords > ntiles ? nwords : ntiles;
   for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < end; i += stride) {
-    if (i < nwords) flag_words[i] = 0u;
+    if (i < nwords) words[i] = 0u;
     if (i < ntiles) {
       int a = 0, b = nseg - 1;
       while (a < b) {
@@ -341,26 +396,50 @@ __global__ __launch_bounds__(256) void seg_prep_kernel(unsigned* __restrict__ fl
 inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
 struct Layout {
-  size_t flags_off, aggs_off, incls_off, total;
+  size_t words_off[3], total;
 };
 Layout layout_for(int64_t ntiles) {
   Layout l;
-  l.flags_off = kHeaderBytes;
-  l.aggs_off = l.flags_off + align256(size_t(ntiles) * 8);
-  l.incls_off = l.aggs_off + align256(size_t(ntiles) * 8);
-  l.total = l.incls_off + align256(size_t(ntiles) * 8);
+  l.total = kHeaderBytes;
+  for (size_t& off : l.words_off) {
+    off = l.total;
+    l.total += align256(size_t(ntiles) * 8);
+  }
   return l;
+}
+TileWords words_in(char* base, const Layout& l) {
+  auto at = [&](int i) { return reinterpret_cast<unsigned long long*>(base + l.words_off[i]); };
+  return {at(0), at(1), at(2)};
 }
 
 template <int ROWS, bool SEG, int BS = kBS, bool INCL = false>
 void launch_rows(bool nt, unsigned grid, const double* x, double* y, int64_t n, int64_t ntiles, ScanHeader* hdr,
-                 unsigned long long* flags, double* aggs, double* incls, int vec, SegTables seg, hipStream_t s) {
-  if (nt)
-    scan_kernel<BS, ROWS, true, SEG, INCL><<<dim3(grid), dim3(BS), 0, s>>>(x, y, n, ntiles, hdr, flags, aggs, incls,
-                                                                            vec, seg);
-  else
-    scan_kernel<BS, ROWS, false, SEG, INCL><<<dim3(grid), dim3(BS), 0, s>>>(x, y, n, ntiles, hdr, flags, aggs, incls,
-                                                                             vec, seg);
+                 TileWords words, int vec, SegTables seg, hipStream_t s) {
+  const bool wide = !SEG && ROWS <= 8 && ntiles <= kWideTiles;
+  auto go = [&](auto kernel) { kernel<<<dim3(grid), dim3(BS), 0, s>>>(x, y, n, ntiles, hdr, words, vec, seg); };
+  if constexpr (!SEG && ROWS <= 8) {
+    if (wide) return nt ? go(scan_kernel<BS, ROWS, true, SEG, INCL, true>) : go(scan_kernel<BS, ROWS, false, SEG, INCL, true>);
+  }
+  if (nt) go(scan_kernel<BS, ROWS, true, SEG, INCL, false>);
+  else go(scan_kernel<BS, ROWS, false, SEG, INCL, false>);
+}
+
+// Default tile: 64 doubles for each of 256 work-items, and smaller ones where
+// that would leave most CUs without a tile (and the scratch has their words):
+// 1M doubles take 11.3 us as 62 tiles of 16384 and 8.6 us as 245 of 4096; at
+// 4M tiles of 8192 (512 work-items) are the fastest, 15.3 us against 16.0 and
+// 18.4.
+constexpr int64_t kSmallScan = int64_t(1) << 20, kMediumScan = int64_t(1) << 22;
+struct ScanShape {
+  int bs, ipt;
+};
+ScanShape scan_shape(int64_t n, const rpx_tuning* tune, size_t scratch_bytes) {
+  const int bs = tune_or(tune, &rpx_tuning::block_size, 0), ipt = tune_or(tune, &rpx_tuning::items_per_thread, 0);
+  if (bs == 0 && ipt == 0 && n <= kMediumScan) {
+    const ScanShape d{n <= kSmallScan ? 256 : 512, 16};
+    if (layout_for(ceil_div(n, int64_t(d.bs) * d.ipt)).total <= scratch_bytes) return d;
+  }
+  return {bs ? bs : kBS, ipt ? ipt : kDefaultIPT};
 }
 
 template <bool INCL>
@@ -375,22 +454,20 @@ int scan_one(const double* x, double* y, int64_t n, int ipt, int bs, bool nt, vo
   if (scratch_bytes < l.total) return RPX_ERR_SCRATCH_TOO_SMALL;
   char* base = reinterpret_cast<char*>(scratch);
   auto* hdr = reinterpret_cast<ScanHeader*>(base);
-  auto* flags = reinterpret_cast<unsigned long long*>(base + l.flags_off);
-  auto* aggs = reinterpret_cast<double*>(base + l.aggs_off);
-  auto* incls = reinterpret_cast<double*>(base + l.incls_off);
+  const TileWords words = words_in(base, l);
   const int vec = aligned16(x) && aligned16(y);
   const unsigned grid = unsigned(ntiles);
   const SegTables none{nullptr, nullptr, nullptr};
   if (bs == 512) {
-    if (ipt == 16) launch_rows<8, false, 512, INCL>(nt, grid, x, y, n, ntiles, hdr, flags, aggs, incls, vec, none, s);
+    if (ipt == 16) launch_rows<8, false, 512, INCL>(nt, grid, x, y, n, ntiles, hdr, words, vec, none, s);
     else if (ipt == 32)
-      launch_rows<16, false, 512, INCL>(nt, grid, x, y, n, ntiles, hdr, flags, aggs, incls, vec, none, s);
-    else launch_rows<32, false, 512, INCL>(nt, grid, x, y, n, ntiles, hdr, flags, aggs, incls, vec, none, s);
+      launch_rows<16, false, 512, INCL>(nt, grid, x, y, n, ntiles, hdr, words, vec, none, s);
+    else launch_rows<32, false, 512, INCL>(nt, grid, x, y, n, ntiles, hdr, words, vec, none, s);
   } else {
-    if (ipt == 16) launch_rows<8, false, kBS, INCL>(nt, grid, x, y, n, ntiles, hdr, flags, aggs, incls, vec, none, s);
+    if (ipt == 16) launch_rows<8, false, kBS, INCL>(nt, grid, x, y, n, ntiles, hdr, words, vec, none, s);
     else if (ipt == 32)
-      launch_rows<16, false, kBS, INCL>(nt, grid, x, y, n, ntiles, hdr, flags, aggs, incls, vec, none, s);
-    else launch_rows<32, false, kBS, INCL>(nt, grid, x, y, n, ntiles, hdr, flags, aggs, incls, vec, none, s);
+      launch_rows<16, false, kBS, INCL>(nt, grid, x, y, n, ntiles, hdr, words, vec, none, s);
+    else launch_rows<32, false, kBS, INCL>(nt, grid, x, y, n, ntiles, hdr, words, vec, none, s);
   }
   return launch_status();
 }
@@ -434,19 +511,17 @@ size_t rpx_scan_scratch_bytes(int64_t n, const rpx_tuning* /*tune*/) {
 int rpx_scan_exclusive_f64(const double* x, double* y, int64_t n, void* scratch, size_t scratch_bytes,
                            const rpx_tuning* tune, void* stream) {
   if (n < 0 || (n > 0 && (!x || !y || !scratch))) return RPX_ERR_INVALID_ARGUMENT;
-  const int ipt = tune_or(tune, &rpx_tuning::items_per_thread, kDefaultIPT);
-  const int bs = tune_or(tune, &rpx_tuning::block_size, kDefaultScanBS);
+  const ScanShape d = scan_shape(n, tune, scratch_bytes);
   const bool nt = (tune_flags(tune) & RPX_TUNE_CACHED) == 0;
-  return scan_one<false>(x, y, n, ipt, bs, nt, scratch, scratch_bytes, as_stream(stream));
+  return scan_one<false>(x, y, n, d.ipt, d.bs, nt, scratch, scratch_bytes, as_stream(stream));
 }
 
 int rpx_scan_inclusive_f64(const double* x, double* y, int64_t n, void* scratch, size_t scratch_bytes,
                            const rpx_tuning* tune, void* stream) {
   if (n < 0 || (n > 0 && (!x || !y || !scratch))) return RPX_ERR_INVALID_ARGUMENT;
-  const int ipt = tune_or(tune, &rpx_tuning::items_per_thread, kDefaultIPT);
-  const int bs = tune_or(tune, &rpx_tuning::block_size, kDefaultScanBS);
+  const ScanShape d = scan_shape(n, tune, scratch_bytes);
   const bool nt = (tune_flags(tune) & RPX_TUNE_CACHED) == 0;
-  return scan_one<true>(x, y, n, ipt, bs, nt, scratch, scratch_bytes, as_stream(stream));
+  return scan_one<true>(x, y, n, d.ipt, d.bs, nt, scratch, scratch_bytes, as_stream(stream));
 }
 
 size_t rpx_scan_segmented_scratch_bytes(const int64_t* offsets_host, int64_t nseg) {
@@ -481,18 +556,17 @@ int rpx_scan_exclusive_segmented_f64(const double* x, double* y, const int64_t* 
   auto* d_tile_seg = reinterpret_cast<int*>(base + g.tile_seg_off);
   const HostChunk table{d_off, tab.data(), tab.size() * sizeof(int64_t)};
   if (const int rc = upload_async(&table, 1, st); rc != RPX_SUCCESS) return rc;
-  // Flags start at zero for every call (no epochs across segments).
-  auto* flags = reinterpret_cast<unsigned long long*>(base + g.l.flags_off);
-  const int64_t words = g.ntiles * 2;
+  // The tiles' words start at zero for every call (no epochs across segments).
+  char* const tiles = base + g.l.words_off[0];
+  const int64_t words = int64_t(g.l.total - g.l.words_off[0]) / 4;
   const int64_t work = words > g.ntiles ? words : g.ntiles;
   seg_prep_kernel<<<dim3(unsigned(ceil_div(work, 256) < 4096 ? ceil_div(work, 256) : 4096)), dim3(256), 0, st>>>(
-      reinterpret_cast<unsigned*>(flags), words, d_tile0, int(nseg), d_tile_seg, g.ntiles);
+      reinterpret_cast<unsigned*>(tiles), words, d_tile0, int(nseg), d_tile_seg, g.ntiles);
   if (const int rc = launch_status(); rc != RPX_SUCCESS) return rc;
   const SegTables seg{d_off, d_tile0, d_tile_seg};
   const int vec = aligned16(x) && aligned16(y);
   launch_rows<32, true>(true, unsigned(g.ntiles), x, y, offsets_host[nseg], g.ntiles,
-                        reinterpret_cast<ScanHeader*>(base), flags, reinterpret_cast<double*>(base + g.l.aggs_off),
-                        reinterpret_cast<double*>(base + g.l.incls_off), vec, seg, st);
+                        reinterpret_cast<ScanHeader*>(base), words_in(base, g.l), vec, seg, st);
   return launch_status();
 }
 
