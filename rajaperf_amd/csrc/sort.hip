@@ -9,9 +9,9 @@
 // order is numeric order with -0.0 before +0.0 and NaNs at the ends.  Equal
 // images are equal bit patterns, so the sort need not be stable.
 //
-// MI355X design: a sample sort.  A bucket of up to 4096 keys is sorted in
+// MI355X design: a sample sort.  A bucket of up to 7664 keys is sorted in
 // registers and LDS by one workgroup (bucket_kernel); a longer segment is
-// first cut into buckets of about 3000 keys by splitters taken from a sorted
+// first cut into buckets of about 4000 keys by splitters taken from a sorted
 // random sample of it:
 //   sample:  one workgroup per segment sorts a sample, writes the splitters;
 //   hist:    every key's bucket (search over the splitters in LDS), kept as
@@ -21,13 +21,13 @@
 //   bucket:  every bucket (and every short segment) sorted.
 // So a key moves twice and is read once more, where a least-significant-digit
 // radix sort of 8-bit digits, which this replaces, moves it eight times and
-// reads it eight times more: 41.6 M keys in 256 ragged segments 2.30 -> 0.83
-// ms, one segment of 10^6 keys (24 launches then, 6 now) 0.30 -> 0.12 ms.
+// reads it eight times more: 41.6 M keys in 256 ragged segments 2.30 -> 0.63
+// ms, one segment of 10^6 keys (24 launches then, 6 now) 0.30 -> 0.07 ms.
 // Segments above kOneLevel keys are cut twice, first into about
-// sqrt(n / 3072) parts.  Keys equal to a repeated splitter go round robin to
+// sqrt(n / 4096) parts.  Keys equal to a repeated splitter go round robin to
 // the buckets between its copies, which hold nothing else and are not sorted,
 // so equal keys cannot overfill a bucket.  A bucket that is overfull by bad
-// luck in the sample is sorted by big_kernel, of any length.
+// luck in the sample is sorted in pieces that are then merged (overfull_kernel).
 #include <algorithm>
 #include <vector>
 
@@ -42,14 +42,24 @@ typedef unsigned long long u64;
 constexpr int kBS = 256;
 constexpr int kRows = 16;
 constexpr int kTile = kBS * kRows;  // 4096 keys per tile of hist and scatter
-constexpr int kBucket = 4096;       // keys bucket_kernel sorts
-constexpr int kAim = 3072;          // mean keys per bucket
+constexpr int kAim = 4096;          // least mean of keys per bucket
 constexpr int kMaxK = 1024;         // buckets per segment and level
 constexpr int kCol = 64;            // buckets per workgroup of colscan
-constexpr int kBig = 8192;          // keys big_kernel sorts in one piece
 // Longest segment cut in one level: 512 buckets leave runs of 8 keys (64
 // bytes) per tile and bucket to write.
 constexpr long long kOneLevel = 512ll * kAim;
+
+// A bucket_kernel workgroup of 2^TB work-items: the keys it sorts, and its
+// LDS, of which sixteen wavefronts' fit on a CU (__syncthreads_or takes 256
+// bytes besides).
+template <int TB>
+struct Room {
+  static constexpr int kT = 1 << TB, kCap = 15 * kT - 16;
+  static constexpr int kBytes = 160 * kT - 256;
+};
+constexpr int kTB = 9;  // the workgroups of long segments
+typedef Room<kTB> Large;
+typedef Room<8> Small;
 
 // A segment at one level: keys [base, base + len) of x (src = 0) or of the
 // scratch copy (src = 1; both are indexed alike), cut into k buckets that
@@ -61,9 +71,9 @@ struct Seg {
 };
 
 // Number of rows, buckets and column groups of a level whose segments were
-// found on the device, and the list of overfull buckets.
+// found on the device, and of the overfull buckets.
 struct Header {
-  int rows, buckets, cols, nbig;
+  int rows, buckets, cols, over;
 };
 
 // One level.  segs = null: nseg segments of equal length from x[0], all
@@ -84,7 +94,7 @@ struct Level {
   unsigned* starts;  // first key of the bucket in its segment; top bit: pure
   unsigned short* ids;
   Header* header;
-  int* big;
+  int* over;  // overfull buckets
 };
 
 __device__ __forceinline__ u64 to_key(u64 b) { return (b >> 63) ? ~b : (b | 0x8000000000000000ull); }
@@ -101,11 +111,23 @@ __device__ __forceinline__ Seg get_seg(const Level& l, int s) {
   return g;
 }
 
+// Sampled keys for a cut into k buckets.  A bucket's share has a spread of
+// sqrt(k / samples) of its mean, and may be 4.5 of those above it before it is
+// overfull: with kAim in place of this rule, buckets of 41.6 M keys in 256
+// segments were half as full and took 237 us in
+// bucket_kernel instead of 212.
+__host__ __device__ constexpr int samples_for(int k) { return k <= 16 ? 2048 : 8192; }
 __host__ __device__ inline int buckets_for(long long len, bool whole) {
-  if (len <= kBucket) return 1;
+  if (len <= Large::kCap) return 1;
   if (whole || len <= kOneLevel) {
-    const long long k = (len + kAim - 1) / kAim;
-    return int(k < kMaxK ? k : kMaxK);
+    long long k = (len + kAim - 1) / kAim;
+    if (k >= kMaxK) return kMaxK;
+    for (int i = 0; i < 3; ++i) {
+      const float spread = sqrtf(float(k) / float(samples_for(int(k))));
+      const long long aim = (long long)(float(Large::kCap) / (1.0f + 4.5f * spread));
+      if (aim > kAim) k = (len + aim - 1) / aim;
+    }
+    return int(k < 2 ? 2 : k);
   }
   // Two levels: about sqrt(len / kAim) parts each.
   int k = 2;
@@ -115,9 +137,10 @@ __host__ __device__ inline int buckets_for(long long len, bool whole) {
 
 // ---- sorting network in registers and LDS ------------------------------------
 //
-// 256 work-items sort N = 2^M = 256 R keys (M = 8 + RB, R = 2^RB per
-// work-item) with a bitonic network whose merges begin with the mirrored
-// comparison (i with i ^ (2^k - 1)), so every comparison is ascending.  A
+// Where the linear map below does not do: 2^TB work-items sort N = 2^M keys
+// (M = TB + RB, R = 2^RB per work-item) with a bitonic network whose merges
+// begin with the mirrored comparison (i with i ^ (2^k - 1)), so every
+// comparison is ascending.  A
 // work-item holds the R keys whose indexes differ in bits [LO, LO + RB) and
 // runs up to RB strides on registers before the keys change places through
 // LDS; element i lives at LDS slot i + i/R, which spreads every layout over
@@ -165,10 +188,10 @@ struct AsImage {
 // A bit pattern that AsDouble cannot order: NaN or -inf.
 __device__ __forceinline__ bool unordered(u64 b) { return b >= 0xFFF0000000000000ull || (b << 1) > (0x7FF0000000000000ull << 1); }
 
-template <class C, int RB>
+template <class C, int TB, int RB>
 struct Net {
   typedef typename C::T T;
-  static constexpr int R = 1 << RB, M = 8 + RB, N = 1 << M;
+  static constexpr int kT = 1 << TB, R = 1 << RB, M = TB + RB, N = 1 << M;
   static constexpr int kSlots = N + N / R;
 
   // LDS slot of element (hi, r, lo) of layout LO is base + offset(r).
@@ -261,125 +284,51 @@ struct Net {
     T* lds = reinterpret_cast<T*>(mem);
     T v[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = (r * kBS + t < len) ? C::enter(b[r]) : C::last();
+    for (int r = 0; r < R; ++r) v[r] = (r * kT + t < len) ? C::enter(b[r]) : C::last();
     sort(v, lds, t);
     put<0, false>(v, lds, t);
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int i = r * kBS + t;
+      const int i = r * kT + t;
       if (i < len) dst[i] = C::leave(lds[i + (i >> RB)]);
     }
   }
 };
 
-constexpr int kBucketSlots = Net<AsDouble, 4>::kSlots;
-constexpr int kBigSlots = Net<AsDouble, 5>::kSlots;
-static_assert(Net<AsDouble, 4>::N == kBucket && Net<AsDouble, 5>::N == kBig, "network sizes");
-
-template <int RB>
-__device__ __forceinline__ bool load_keys(u64 (&b)[1 << RB], const u64* src, int len, int t) {
-  bool special = false;
+// ---- sorting by a linear map --------------------------------------------------
+//
+// The keys of a bucket lie between two neighbouring splitters, where most
+// inputs are close to evenly spread.  2^TB work-items map up to 16 keys each
+// onto 16 bins each, linearly from the least key to the greatest, count the
+// bins with LDS atomics (a counter's old value is the key's place in its bin)
+// and put the keys into their bins' slots.  The map is monotone in floating
+// point, so only keys of one bin can be out of order.  A work-item then sorts
+// 16 consecutive slots in registers and merges its upper eight with its
+// neighbour's lower eight, which sorts all if no bin holds more than nine
+// different keys; half a key per bin is usual.  Whether it did is read off the
+// neighbours of the merged sixteens.  If not, or with NaNs, infinities, or a
+// -0.0 (which equals +0.0 as a double), nothing has been written and the
+// network sorts the keys.
+//
+// What bounds it: about 50 vector instructions and 60 bytes of LDS traffic per
+// key, where the network spends 91 comparisons and 360 bytes; each takes 40% of
+// the time, as do the 16 bytes per key from and to memory, and the eight
+// barriers between them keep a workgroup waiting.  Buckets of 41.6 M keys: 407
+// us with the network alone (4096 keys at most, the overfull in a kernel of 52
+// us), 212 us here.  Ranking the keys of a bin by comparing each with all
+// others took 315 us.
+// Odd-even merges of sorted runs of P keys into longer ones, up to all 16.
+template <int P, int K = P>
+__device__ __forceinline__ void batcher(double (&v)[16]) {
 #pragma unroll
-  for (int r = 0; r < (1 << RB); ++r) {
-    const int i = r * kBS + t;
-    b[r] = i < len ? src[i] : 0ull;
-  }
-#pragma unroll
-  for (int r = 0; r < (1 << RB); ++r) special |= unordered(b[r]);
-  return special;
+  for (int i = 0; i < 16 - K; ++i)
+    if (i >= K % P && (i - K % P) / K % 2 == 0 && i / (2 * P) == (i + K) / (2 * P)) AsDouble::order(v[i], v[i + K]);
+  if constexpr (K > 1) batcher<P, K / 2>(v);
+  else if constexpr (P < 8) batcher<2 * P>(v);
 }
 
-// src[0..len) -> dst sorted, len <= 256 << RB, with the images if need be.
-template <int RB>
-__device__ __forceinline__ void sort_piece(const u64* src, u64* dst, int len, void* mem, int t) {
-  u64 b[1 << RB];
-  const bool special = load_keys<RB>(b, src, len, t);
-  if (__syncthreads_or(special)) Net<AsImage, RB>::sort_keys(b, dst, len, mem, t);
-  else Net<AsDouble, RB>::sort_keys(b, dst, len, mem, t);
-}
-
-// ---- splitters -----------------------------------------------------------------
-
-// Sample of segment s, sorted, and every k-quantile of it as a splitter.
-// S = 2^M keys from S equal strata at pseudo-random places in them; at least
-// 16 per bucket for the most buckets, 32 and more otherwise (the spread of the
-// bucket sizes is 1/sqrt of that).
-template <class C, int RB>
-__device__ __forceinline__ void make_splitters(const u64 (&b)[1 << RB], const Seg& g, u64* splitters, int* dup,
-                                               void* mem, int t) {
-  typedef Net<C, RB> W;
-  typename C::T* lds = reinterpret_cast<typename C::T*>(mem);
-  typename C::T v[W::R];
-#pragma unroll
-  for (int r = 0; r < W::R; ++r) v[r] = C::enter(b[r]);
-  W::sort(v, lds, t);
-  W::template put<0, false>(v, lds, t);
-  __syncthreads();
-  bool d = false;
-  for (int j = t + 1; j < g.k; j += kBS) {
-    auto quantile = [&](int q) {
-      const int i = q * W::N / g.k;  // q < 1024
-      return to_key(C::leave(lds[i + (i >> RB)]));
-    };
-    const u64 s = quantile(j);
-    splitters[j - 1] = s;
-    d |= j > 1 && s == quantile(j - 1);
-  }
-  const int any = __syncthreads_or(d);
-  if (t == 0) *dup = any;
-}
-
-template <int RB>
-__device__ __forceinline__ void sample_segment(const u64* src, const Seg& g, u64* splitters, int* dup, void* mem,
-                                               int t) {
-  constexpr int R = 1 << RB, S = 256 << RB;
-  u64 b[R];
-  bool special = false;
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const u64 i = u64(r * kBS + t);
-    const u64 jitter = mix64(i * kGamma + u64(g.len)) >> 48;
-    b[r] = src[(i << 16 | jitter) * u64(g.len) >> (16 + 8 + RB)];  // (i + jitter 2^-16) len / S
-  }
-#pragma unroll
-  for (int r = 0; r < R; ++r) special |= unordered(b[r]);
-  static_assert(S <= kBig, "sample fits the LDS");
-  if (__syncthreads_or(special)) make_splitters<AsImage, RB>(b, g, splitters, dup, mem, t);
-  else make_splitters<AsDouble, RB>(b, g, splitters, dup, mem, t);
-}
-
-// One workgroup per segment: its entries of the row, column and bucket maps,
-// and its splitters.
-__global__ __launch_bounds__(kBS) void sample_kernel(const u64* x, const u64* alt, Level l) {
-  __shared__ u64 mem[kBigSlots];
-  const int t = threadIdx.x, s = blockIdx.x;
-  if (s == 0 && t == 0) l.header->nbig = 0;
-  const Seg g = get_seg(l, s);
-  if (l.segs) {
-    for (int i = t; i < g.k; i += kBS) l.bucket_seg[g.first_bucket + i] = s;
-    if (g.k > 1) {
-      for (int i = t; i < g.rows; i += kBS) l.row_seg[g.first_row + i] = s;
-      for (int i = t; i < (g.k + kCol - 1) / kCol; i += kBS) l.col_seg[g.first_col + i] = s;
-    }
-  }
-  if (g.k <= 1) return;
-  const u64* src = (g.src ? alt : x) + g.base;
-  u64* sp = l.splitters + g.first_bucket;
-  // 2048 samples for up to 64 buckets, 8192 above.
-  if (g.k <= 64) sample_segment<3>(src, g, sp, l.dup + s, mem, t);
-  else sample_segment<5>(src, g, sp, l.dup + s, mem, t);
-}
-
-// ---- partition -----------------------------------------------------------------
-
-// Segment of row, column group or bucket i.
-__device__ __forceinline__ int seg_of(const Level& l, const int* map, int i, int per_seg) {
-  if (!l.segs) return i / per_seg;
-  return map ? map[i] : i;
-}
-
-// Exclusive scan over the 256 work-items of a workgroup (one value each).
+// Exclusive scan over the work-items of a workgroup (one value each).
 __device__ __forceinline__ unsigned block_exclusive_scan(unsigned v, unsigned* wsum) {
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   unsigned incl = v;
@@ -393,6 +342,275 @@ __device__ __forceinline__ unsigned block_exclusive_scan(unsigned v, unsigned* w
   unsigned run = incl - v;
   for (int w = 0; w < wave; ++w) run += wsum[w];
   return run;
+}
+
+// LDS of up to `keys` keys: 17 words per 16 of them (both a work-item's 16 and
+// adjacent work-items' keys then fall into different banks), and the bins.
+constexpr int linear_bytes(int tb, int keys) { return keys / 16 * 17 * 8 + (32 << tb); }
+static_assert(linear_bytes(kTB, Large::kCap) <= Large::kBytes && linear_bytes(8, Small::kCap) <= Small::kBytes &&
+                  Large::kCap % 16 == 0 && Small::kCap % 16 == 0,
+              "keys and bins fit");
+
+// get(i): the bits of key i, 0 <= i < len, 1 <= len <= kKeys <= 2^(TB+4).
+// Calls out(place, key) for every key, or returns false, by all work-items.
+template <int TB, int kKeys, class Get, class Out>
+__device__ __forceinline__ bool sort_linear(int len, char* lds, int t, Get get, Out out) {
+  constexpr int T = 1 << TB, R = 16, N = T * R, kWaves = T / kWave, W = R / 2;
+  static_assert(kKeys <= N && kKeys % 16 == 0 && N <= 65536, "16-bit counters");
+  double* keys = reinterpret_cast<double*>(lds);
+  unsigned* bins = reinterpret_cast<unsigned*>(lds + kKeys / 16 * 17 * 8);  // two 16-bit counters per word
+  double* ends = keys;                                                      // before any key is placed
+  unsigned* wsum = reinterpret_cast<unsigned*>(ends + 2 * kWaves);
+  const int lane = t & (kWave - 1), wave = t / kWave;
+  auto slot = [](int i) { return i + (i >> 4); };
+  double x[R];
+  unsigned widest = 0u;
+  bool special = false;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = (r << TB) + t;
+    if ((r << TB) < len) x[r] = __longlong_as_double((long long)get(i < len ? i : len - 1));
+  }
+#pragma unroll
+  for (int j = 0; j < W; ++j) bins[j * T + t] = 0u;
+  double lo = x[0], hi = x[0];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if ((r << TB) >= len) continue;
+    const u64 b = (u64)__double_as_longlong(x[r]);
+    const unsigned size = unsigned(b >> 32) & 0x7FFFFFFFu;
+    widest = size > widest ? size : widest;
+    special |= b == 0x8000000000000000ull;
+    asm("v_min_f64 %0, %0, %1" : "+v"(lo) : "v"(x[r]));
+    asm("v_max_f64 %0, %0, %1" : "+v"(hi) : "v"(x[r]));
+  }
+  special |= widest >= 0x7FF00000u;
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) {
+    const double l = __shfl_xor(lo, off, kWave), h = __shfl_xor(hi, off, kWave);
+    asm("v_min_f64 %0, %0, %1" : "+v"(lo) : "v"(l));
+    asm("v_max_f64 %0, %0, %1" : "+v"(hi) : "v"(h));
+  }
+  if (lane == 0) {
+    ends[wave] = lo;
+    ends[kWaves + wave] = hi;
+  }
+  if (__syncthreads_or(special)) return false;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    const double l = ends[w], h = ends[kWaves + w];
+    asm("v_min_f64 %0, %0, %1" : "+v"(lo) : "v"(l));
+    asm("v_max_f64 %0, %0, %1" : "+v"(hi) : "v"(h));
+  }
+  const double spread = hi - lo;
+  const double scale = double(N) / spread;
+  if (!(spread < 1e300 && scale < 1e300)) {
+    if (spread != 0.0) return false;
+#pragma unroll
+    for (int r = 0; r < R; ++r)  // all equal
+      if ((r << TB) + t < len) out((r << TB) + t, (u64)__double_as_longlong(x[r]));
+    return true;
+  }
+  unsigned at[R];  // the key's bin, and its place in it above
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if ((r << TB) >= len) continue;
+    int bin = int((x[r] - lo) * scale);
+    bin = bin < N - 1 ? bin : N - 1;
+    at[r] = unsigned(bin);
+    if ((r << TB) + t < len) {
+      const unsigned old = atomicAdd(&bins[bin >> 1], 1u << (bin << 4 & 31));
+      at[r] |= old >> (bin << 4 & 31) << 16;
+    }
+  }
+  __syncthreads();
+  {
+    unsigned c[W], sum = 0;
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+      c[j] = bins[t * W + j];
+      sum += (c[j] & 0xFFFFu) + (c[j] >> 16);
+    }
+    unsigned run = block_exclusive_scan(sum, wsum);
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+      const unsigned second = run + (c[j] & 0xFFFFu);
+      bins[t * W + j] = run | second << 16;
+      run = second + (c[j] >> 16);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if ((r << TB) + t < len) {
+      const unsigned bin = at[r] & 0xFFFFu;
+      keys[slot(int((bins[bin >> 1] >> (bin << 4 & 31) & 0xFFFFu) + (at[r] >> 16)))] = x[r];
+    }
+  }
+  __syncthreads();
+  const double none = __longlong_as_double(0x7FF0000000000000ll);
+  const int first = 16 * t;
+  double* own = keys + 17 * t;  // slots first .. first + 15; the next work-item's from own + 17
+  if (first < len) {
+#pragma unroll
+    for (int u = 0; u < 16; ++u) x[u] = own[u];
+    if (first + 16 > len) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u) x[u] = first + u < len ? x[u] : none;
+    }
+    batcher<1>(x);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) own[u] = x[u];
+  }
+  __syncthreads();
+  if (first + 8 < len) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = x[u + 8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u + 8] = first + 16 < len ? own[17 + u] : none;
+    batcher<8>(x);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) own[8 + u] = x[u];
+    if (first + 16 < len) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) own[17 + u] = x[u + 8];
+    }
+  }
+  __syncthreads();
+  bool bad = t == 0 && len > 8 && keys[7] > keys[8];
+  if (first + 24 < len) bad |= own[17 + 7] > own[17 + 8];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if ((r << TB) + t < len) x[r] = keys[slot((r << TB) + t)];
+  }
+  if (__syncthreads_or(bad)) return false;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if ((r << TB) + t < len) out((r << TB) + t, (u64)__double_as_longlong(x[r]));
+  }
+  return true;
+}
+
+template <int TB, int RB>
+__device__ __forceinline__ void sort_network(const u64* src, u64* dst, int len, char* lds, int t) {
+  u64 b[1 << RB];
+  bool special = false;
+#pragma unroll
+  for (int r = 0; r < (1 << RB); ++r) {
+    const int i = (r << TB) + t;
+    b[r] = i < len ? src[i] : 0ull;
+  }
+#pragma unroll
+  for (int r = 0; r < (1 << RB); ++r) special |= unordered(b[r]);
+  if (__syncthreads_or(special)) Net<AsImage, TB, RB>::sort_keys(b, dst, len, lds, t);
+  else Net<AsDouble, TB, RB>::sort_keys(b, dst, len, lds, t);
+}
+
+static_assert(Net<AsDouble, kTB, 4>::kSlots * 8 <= Large::kBytes && Net<AsDouble, 8, 4>::kSlots * 8 <= Small::kBytes,
+              "the networks fit too");
+
+// src[0..len) -> dst sorted (dst may be src), 1 <= len <= Room<TB>::kCap.
+template <int TB>
+__device__ __forceinline__ void sort_piece(const u64* src, u64* dst, int len, char* lds, int t) {
+  // 32-bit byte offsets from a uniform base
+  const auto get = [&](int i) {
+    return *reinterpret_cast<const u64*>(reinterpret_cast<const char*>(src) + unsigned(i) * 8u);
+  };
+  const auto put = [&](int i, u64 v) {
+    *reinterpret_cast<u64*>(reinterpret_cast<char*>(dst) + unsigned(i) * 8u) = v;
+  };
+  if (sort_linear<TB, Room<TB>::kCap>(len, lds, t, get, put)) return;
+  __syncthreads();
+  if (len <= 4 << TB) sort_network<TB, 2>(src, dst, len, lds, t);
+  else sort_network<TB, 4>(src, dst, len, lds, t);
+}
+
+// ---- splitters -----------------------------------------------------------------
+
+// Sample of segment s, sorted, and every k-quantile of it as a splitter.
+// S = 2^(kTB+RB) keys from S equal strata at pseudo-random places in them.
+template <class C, int RB>
+__device__ __forceinline__ void network_splitters(const u64 (&b)[1 << RB], int k, u64* sp, char* mem, int t) {
+  typedef Net<C, kTB, RB> W;
+  typename C::T* lds = reinterpret_cast<typename C::T*>(mem);
+  typename C::T v[W::R];
+#pragma unroll
+  for (int r = 0; r < W::R; ++r) v[r] = C::enter(b[r]);
+  W::sort(v, lds, t);
+  W::template put<0, false>(v, lds, t);
+  __syncthreads();
+  for (int j = t + 1; j < k; j += W::kT) {
+    const int i = j * W::N / k;  // j < 1024
+    sp[j - 1] = to_key(C::leave(lds[i + (i >> RB)]));
+  }
+}
+
+template <int RB>
+__device__ __forceinline__ void sample_segment(const u64* src, const Seg& g, u64* splitters, int* dup, u64* sp,
+                                               char* mem, int t) {
+  constexpr int R = 1 << RB, T = 1 << kTB, M = kTB + RB, S = 1 << M;
+  const auto sampled = [&](int at) {
+    const u64 i = u64(at);
+    const u64 jitter = mix64(i * kGamma + u64(g.len)) >> 48;
+    return src[(i << 16 | jitter) * u64(g.len) >> (16 + M)];  // (i + jitter 2^-16) len / S
+  };
+  // Quantile j is the key at place floor(j S / k).
+  const auto quantile = [&](int place, u64 b) {
+    const int j = int((unsigned(place) * unsigned(g.k) + unsigned(S - 1)) >> M);
+    if (j > 0 && j < g.k && (unsigned(j) << M) < unsigned(place + 1) * unsigned(g.k)) sp[j - 1] = to_key(b);
+  };
+  if (!sort_linear<kTB, S>(S, mem, t, sampled, quantile)) {
+    __syncthreads();
+    u64 b[R];
+    bool special = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) b[r] = sampled(r * T + t);
+#pragma unroll
+    for (int r = 0; r < R; ++r) special |= unordered(b[r]);
+    if (__syncthreads_or(special)) network_splitters<AsImage, RB>(b, g.k, sp, mem, t);
+    else network_splitters<AsDouble, RB>(b, g.k, sp, mem, t);
+  }
+  __syncthreads();
+  bool d = false;
+  for (int j = t; j < g.k - 1; j += T) {
+    splitters[j] = sp[j];
+    d |= j > 0 && sp[j] == sp[j - 1];
+  }
+  const int any = __syncthreads_or(d);
+  if (t == 0) *dup = any;
+}
+
+// One workgroup per segment: its entries of the row, column and bucket maps,
+// and its splitters.
+constexpr int kSampleBytes = linear_bytes(kTB, 8192);
+static_assert(kSampleBytes >= 8 * Net<AsDouble, kTB, 4>::kSlots, "the network fits too");
+__global__ __launch_bounds__(1 << kTB) void sample_kernel(const u64* x, const u64* alt, Level l) {
+  __shared__ __attribute__((aligned(16))) char mem[kSampleBytes];
+  __shared__ u64 sp[kMaxK];
+  constexpr int T = 1 << kTB;
+  const int t = threadIdx.x, s = blockIdx.x;
+  if (s == 0 && t == 0) l.header->over = 0;
+  const Seg g = get_seg(l, s);
+  if (l.segs) {
+    for (int i = t; i < g.k; i += T) l.bucket_seg[g.first_bucket + i] = s;
+    if (g.k > 1) {
+      for (int i = t; i < g.rows; i += T) l.row_seg[g.first_row + i] = s;
+      for (int i = t; i < (g.k + kCol - 1) / kCol; i += T) l.col_seg[g.first_col + i] = s;
+    }
+  }
+  if (g.k <= 1) return;
+  const u64* src = (g.src ? alt : x) + g.base;
+  u64* splitters = l.splitters + g.first_bucket;
+  if (samples_for(g.k) == 2048) sample_segment<2>(src, g, splitters, l.dup + s, sp, mem, t);
+  else sample_segment<4>(src, g, splitters, l.dup + s, sp, mem, t);
+}
+
+// ---- partition -----------------------------------------------------------------
+
+// Segment of row, column group or bucket i.
+__device__ __forceinline__ int seg_of(const Level& l, const int* map, int i, int per_seg) {
+  if (!l.segs) return i / per_seg;
+  return map ? map[i] : i;
 }
 
 // A row is `chunk` tiles.  The search runs over the splitters as a complete
@@ -646,48 +864,26 @@ __device__ __forceinline__ Piece get_piece(const Level& l, int i) {
   return Piece{g.base + (long long)(st & 0x7FFFFFFFu), int(l.totals[i]), 1 - g.src, (st >> 31) != 0};
 }
 
-// Every bucket of up to kBucket keys, by the smallest network that holds it.
-// Longer ones go on the list for big_kernel.
-__global__ __launch_bounds__(kBS) void bucket_kernel(u64* x, const u64* alt, Level l) {
-  __shared__ u64 mem[kBucketSlots];
-  const int t = threadIdx.x, i = blockIdx.x;
-  if (l.bound && i >= l.bound->buckets) return;
-  const Piece p = get_piece(l, i);
-  const u64* src = (p.src ? alt : x) + p.base;
-  u64* dst = x + p.base;
-  if (p.pure) {
-    if (p.src)
-      for (int j = t; j < p.len; j += kBS) dst[j] = src[j];
-    return;
-  }
-  if (p.len > kBucket) {
-    if (t == 0) l.big[atomicAdd(&l.header->nbig, 1)] = i;
-    return;
-  }
-  if (p.len <= 1 && !p.src) return;
-  if (p.len <= 1024) sort_piece<2>(src, dst, p.len, mem, t);
-  else if (p.len <= 2048) sort_piece<3>(src, dst, p.len, mem, t);
-  else sort_piece<4>(src, dst, p.len, mem, t);
-}
-
-// Any length: pieces of kBig keys, then merges of ever longer runs, every
-// key finding its place by a search in the other run.  The pieces start in x
-// or alt so that the last merge ends in x.
-__device__ void sort_any(u64* x, u64* alt, const Piece& p, void* mem, int t) {
+// Any length: parts of Room<TB>::kCap keys, then merges of ever longer runs,
+// every key finding its place by a search in the other run.  The parts start
+// in x or alt so that the last merge ends in x.
+template <int TB>
+__device__ __forceinline__ void sort_any(u64* x, u64* alt, const Piece& p, char* mem, int t) {
+  constexpr int kPiece = Room<TB>::kCap;
   u64* at[2] = {x + p.base, alt + p.base};
   const u64* src = at[p.src];
   int rounds = 0;
-  while (((long long)kBig << rounds) < p.len) ++rounds;
+  while (((long long)kPiece << rounds) < p.len) ++rounds;
   int cur = rounds & 1;
-  for (long long o = 0; o < p.len; o += kBig) {
-    const int n = int(p.len - o < kBig ? p.len - o : kBig);
-    sort_piece<5>(src + o, at[cur] + o, n, mem, t);
+  for (long long o = 0; o < p.len; o += kPiece) {
+    const int n = int(p.len - o < kPiece ? p.len - o : kPiece);
+    sort_piece<TB>(src + o, at[cur] + o, n, mem, t);
     __syncthreads();
   }
-  for (long long w = kBig; w < p.len; w *= 2) {
+  for (long long w = kPiece; w < p.len; w *= 2) {
     const u64* a = at[cur];
     u64* d = at[cur ^ 1];
-    for (long long i = t; i < p.len; i += kBS) {
+    for (long long i = t; i < p.len; i += 1 << TB) {
       const long long lo = i / (2 * w) * (2 * w);
       const long long mid = lo + w < p.len ? lo + w : p.len;
       const long long hi = lo + 2 * w < p.len ? lo + 2 * w : p.len;
@@ -708,11 +904,31 @@ __device__ void sort_any(u64* x, u64* alt, const Piece& p, void* mem, int t) {
   }
 }
 
-__global__ __launch_bounds__(kBS) void big_kernel(u64* x, u64* alt, Level l) {
-  __shared__ u64 mem[kBigSlots];
-  const int n = l.header->nbig;
+// Every bucket and uncut segment of up to Room<TB>::kCap keys.  Longer ones go
+// on the list for overfull_kernel (in this kernel its code would spill).
+template <int TB>
+__global__ __launch_bounds__(1 << TB, 4) void bucket_kernel(u64* x, const u64* alt, Level l) {
+  __shared__ __attribute__((aligned(16))) char mem[Room<TB>::kBytes];
+  const int t = threadIdx.x, i = blockIdx.x;
+  if (l.bound && i >= l.bound->buckets) return;
+  const Piece p = get_piece(l, i);
+  const u64* src = (p.src ? alt : x) + p.base;
+  u64* dst = x + p.base;
+  if (p.pure) {
+    if (p.src)
+      for (int j = t; j < p.len; j += 1 << TB) dst[j] = src[j];
+    return;
+  }
+  if (p.len == 0 || (p.len == 1 && !p.src)) return;
+  if (p.len <= Room<TB>::kCap) sort_piece<TB>(src, dst, p.len, mem, t);
+  else if (t == 0) l.over[atomicAdd(&l.header->over, 1)] = i;
+}
+
+__global__ __launch_bounds__(1 << kTB) void overfull_kernel(u64* x, u64* alt, Level l) {
+  __shared__ __attribute__((aligned(16))) char mem[Large::kBytes];
+  const int n = l.header->over;
   for (int i = blockIdx.x; i < n; i += gridDim.x) {
-    sort_any(x, alt, get_piece(l, l.big[i]), mem, threadIdx.x);
+    sort_any<kTB>(x, alt, get_piece(l, l.over[i]), mem, threadIdx.x);
     __syncthreads();
   }
 }
@@ -829,7 +1045,7 @@ Sizes measure(const int64_t* off, int64_t nseg) {
     }
   }
   s.l1.segs = s.nseg;
-  s.small = s.longest <= kBucket;
+  s.small = s.longest <= Large::kCap;
   s.two_levels = s.longest > kOneLevel;
   if (s.two_levels) {
     s.l2.segs = s.l1.buckets;
@@ -868,9 +1084,9 @@ Layout lay_out(const Sizes& s, void* scratch) {
   unsigned short* ids = a.take<unsigned short>(s.keys);
   Header* headers = a.take<Header>(2);  // overfull buckets; bounds of the second level
   o.bound = headers + 1;
+  int* over = a.take<int>(std::max(s.l1.buckets, s.l2.buckets));
   o.segs1 = a.take<Seg>(s.nseg);
   o.segs2 = a.take<Seg>(s.l2.segs);
-  int* big = a.take<int>(std::max(s.l1.buckets, s.l2.buckets));
   for (int i = 0; i < 2; ++i) {
     const LevelSize& z = i ? s.l2 : s.l1;
     Level& l = o.level[i];
@@ -885,14 +1101,14 @@ Layout lay_out(const Sizes& s, void* scratch) {
     l.starts = a.take<unsigned>(z.buckets);
     l.ids = ids;
     l.header = headers;
-    l.big = big;
+    l.over = over;
   }
   o.total = a.used;
   return o;
 }
 
 int partition(u64* x, u64* alt, const Level& l, const LevelSize& z, hipStream_t st) {
-  sample_kernel<<<dim3(unsigned(l.nseg)), dim3(kBS), 0, st>>>(x, alt, l);
+  sample_kernel<<<dim3(unsigned(l.nseg)), dim3(1 << kTB), 0, st>>>(x, alt, l);
   if (z.rows > 0) {
     hist_kernel<<<dim3(unsigned(z.rows)), dim3(kBS), 0, st>>>(x, alt, l);
     colscan_kernel<<<dim3(unsigned(z.cols)), dim3(kCol * kWalkers), 0, st>>>(l);
@@ -970,10 +1186,13 @@ int rpx_sort_segmented_f64(double* x, const int64_t* offsets_host, int64_t nseg,
     z = s.l2;
     if (const int rc = partition(xs, o.alt, *l, z, st); rc != RPX_SUCCESS) return rc;
   }
-  bucket_kernel<<<dim3(unsigned(z.buckets)), dim3(kBS), 0, st>>>(xs, o.alt, *l);
+  if (s.longest <= Small::kCap)
+    bucket_kernel<8><<<dim3(unsigned(z.buckets)), dim3(1 << 8), 0, st>>>(xs, o.alt, *l);
+  else
+    bucket_kernel<kTB><<<dim3(unsigned(z.buckets)), dim3(1 << kTB), 0, st>>>(xs, o.alt, *l);
   if (!s.small) {
-    const unsigned grid = unsigned(z.buckets < 512 ? z.buckets : 512);
-    big_kernel<<<dim3(grid), dim3(kBS), 0, st>>>(xs, o.alt, *l);
+    const unsigned grid = unsigned(z.buckets < 256 ? z.buckets : 256);
+    overfull_kernel<<<dim3(grid), dim3(1 << kTB), 0, st>>>(xs, o.alt, *l);
   }
   return launch_status();
 }
