@@ -37,7 +37,7 @@
 // and the residue bytes d_t ([t] then the GEMM's accumulator fragments).
 #include "rpx_common.hpp"
 
-#include <mutex>
+#include <algorithm>
 
 using namespace rpx;
 
@@ -61,8 +61,8 @@ inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 // Per-call constants of the modular scheme, passed by value to the kernels.
 struct CrtParams {
   int T, b;
-  double m[kMaxMods];    // moduli
-  double inv[kMaxMods];  // fl(1/m_t), used only to pick a quotient that is then corrected
+  double inv[kMaxMods];         // fl(1/m_t)
+  unsigned minus_m[kMaxMods];   // -m_t modulo 256
   double h[kMaxMods];    // floor(2^44 y_t/m_t) 2^-44, y_t = (M/m_t)^-1 mod m_t
   double l[kMaxMods];    // y_t/m_t - h_t, rounded
   double M_hi, M_lo;     // prod m_t = M_hi + M_lo, M_lo rounded (a 2^-106 relative error)
@@ -115,7 +115,7 @@ bool crt_setup(int64_t nk, int nmoduli, CrtParams* p) {
   p->M_lo = hiu >= M ? -double(static_cast<long double>(hiu - M)) : double(static_cast<long double>(M - hiu));
   for (int t = 0; t < kMaxMods; ++t) {
     const int64_t m = kMods[t];
-    p->m[t] = double(m);
+    p->minus_m[t] = unsigned(-m) & 0xFFu;
     p->inv[t] = 1.0 / double(m);
     int64_t mt = 1;  // (M / m_t) mod m_t
     for (int s = 0; s < T; ++s)
@@ -153,37 +153,58 @@ __device__ __forceinline__ int exponent_of(double m) {
 }
 
 // Symmetric residue of the integer-valued x modulo m, |x| <= 2^46 (or
-// |x| < 2^31): fl(x fl(1/m)) is within 2^-13 of x/m, and x/m is at least
-// 1/(2m) >= 2^-9 from a half-integer unless m = 256 and x = 128 (mod 256).
-// So q = rint(x/m) exactly, the fma is exact, and the result lies in
-// [-(m-1)/2, (m-1)/2], or in [-128, 128] for m = 256, where the byte kept
-// (r & 0xFF) makes 128 the same residue as -128.
-__device__ __forceinline__ int sym_mod(double x, double m, double inv) {
-  return int(fma(-rint(x * inv), m, x));
+// |x| < 2^31), in the low byte of the result; the other bytes are anything.
+// x fl(1/m) is within 2^-15 of x/m, and x/m is at least 1/(2m) >= 2^-9 from a
+// half-integer unless m = 256 and x = 128 (mod 256).  So the fma, rounded to
+// integers by the size of kInteger, has rint(x/m) in its low bits, and the
+// residue x - rint(x/m) m lies in [-(m-1)/2, (m-1)/2], or in [-128, 128] for
+// m = 256, where the byte kept makes 128 the same residue as -128.  Only its
+// low byte is wanted, so the low bytes of x, of the quotient and of -m do:
+// one FP64 instruction and one 24-bit multiply-add where the residue as a
+// double and its conversion took four FP64 instructions.
+constexpr double kInteger = 6755399441055744.0;  // 1.5 * 2^52
+__device__ __forceinline__ unsigned low_word(double x) { return unsigned(__double2loint(x + kInteger)); }
+__device__ __forceinline__ unsigned sym_mod(double x, unsigned x_low, double inv, unsigned minus_m) {
+  return __umul24(unsigned(__double2loint(fma(x, inv, kInteger))), minus_m) + x_low;
+}
+// The low bytes of four words.
+__device__ __forceinline__ unsigned pack4(unsigned a, unsigned b, unsigned c, unsigned d) {
+  return __builtin_amdgcn_perm(b, a, 0x0c0c0400u) | __builtin_amdgcn_perm(d, c, 0x04000c0cu);
 }
 
-// One workgroup per (padded) row of A: row exponent, then the residues.
-// Each work-item takes 16 consecutive k and writes one 16-byte chunk per
-// modulus.
-__global__ __launch_bounds__(256) void split_rows_kernel(const double* __restrict__ A, int64_t ni, int64_t nk,
-                                                         int64_t nkp, int64_t nip, signed char* __restrict__ As,
-                                                         int* __restrict__ ea, const CrtParams P) {
-  __shared__ double red[4];
-  const int64_t i = blockIdx.x;
+// Row i of A (padded rows too) by one workgroup: row exponent, then the
+// residues.  A work-item takes four consecutive k of every 1024, so that a
+// wavefront's loads and, per modulus, its stores are whole lines, and up to
+// 4096 k stay in registers between the two uses (with 16 consecutive k per
+// work-item a wavefront's load touched 64 lines, which had left the L1 before
+// the next load wanted them: 4096 rows of 4096 took 83 us, 66
+// here with the cheaper residues, 54 for its bytes).
+constexpr int kRowPasses = 4, kRowSpan = kRowPasses * 1024;
+__device__ __forceinline__ void split_row(const double* __restrict__ A, int64_t i, int64_t ni, int64_t nk, int64_t nkp,
+                                          int64_t nip, signed char* __restrict__ As, int* __restrict__ ea,
+                                          const CrtParams& P, double* red) {
   const int tid = threadIdx.x;
   const bool live = i < ni;
   const double* row = A + (live ? i * nk : 0);
-  double m = 0.0;
-  if (live) {
-    int64_t k = tid;
-    for (; k + 7 * 256 < nk; k += 8 * 256) {
-      double v[8];
+  double x[4 * kRowPasses];
+  auto load = [&](int64_t k0) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = row[k + u * 256];
+    for (int p = 0; p < kRowPasses; ++p) {
+      const int64_t k = k0 + 1024 * p + 4 * tid;
+      if (live && k + 4 <= nk) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) m = fmax(m, fabs(v[u]));
+        for (int c = 0; c < 4; ++c) x[4 * p + c] = row[k + c];
+      } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) x[4 * p + c] = live && k + c < nk ? row[k + c] : 0.0;
+      }
     }
-    for (; k < nk; k += 256) m = fmax(m, fabs(row[k]));
+  };
+  double m = 0.0;
+  for (int64_t k0 = 0; k0 < nkp; k0 += kRowSpan) {
+    load(k0);
+#pragma unroll
+    for (int u = 0; u < 4 * kRowPasses; ++u) m = fmax(m, fabs(x[u]));
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
@@ -192,47 +213,38 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const double* __restric
   m = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
   const int e = exponent_of(m);
   if (tid == 0) ea[i] = e;
-  for (int64_t k0 = int64_t(tid) * 16; k0 < nkp; k0 += 256 * 16) {
-    double x[16];
-    if (live && k0 + 16 <= nk) {
+  for (int64_t k0 = 0; k0 < nkp; k0 += kRowSpan) {
+    if (nkp > kRowSpan) load(k0);
 #pragma unroll
-      for (int u = 0; u < 16; ++u) x[u] = row[k0 + u];
-    } else {
-#pragma unroll
-      for (int u = 0; u < 16; ++u) x[u] = (live && k0 + u < nk) ? row[k0 + u] : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < 16; ++u) x[u] = rint(ldexp(x[u], P.b - e));
-    for (int t = 0; t < P.T; ++t) {
-      v4i w;
+    for (int p = 0; p < kRowPasses; ++p) {
+      const int64_t k = k0 + 1024 * p + 4 * tid;
+      if (k >= nkp) continue;
+      double v[4];
+      unsigned low[4];
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        int packed = 0;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int r = sym_mod(x[4 * c + q], P.m[t], P.inv[t]);
-          packed |= (r & 0xFF) << (8 * q);
-        }
-        w[c] = packed;
+        v[c] = rint(ldexp(x[4 * p + c], P.b - e));
+        low[c] = low_word(v[c]);
       }
-      *reinterpret_cast<v4i*>(As + (int64_t(t) * nip + i) * nkp + k0) = w;
+      signed char* out = As + i * nkp + k;
+      for (int t = 0; t < P.T; ++t, out += nip * nkp) {
+        unsigned r[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) r[c] = sym_mod(v[c], low[c], P.inv[t], P.minus_m[t]);
+        *reinterpret_cast<unsigned*>(out) = pack4(r[0], r[1], r[2], r[3]);
+      }
     }
   }
 }
 
-// Column maxima of B as exponents.  A workgroup takes 64 columns x
-// kColExpRows rows: wavefront w reads rows w, w + 4, ... (each load is 64
-// consecutive columns of one row, 16 loads in flight per work-item), the
-// four wavefronts' maxima meet in LDS, and one atomicMax per column and
-// workgroup (nk / 512 per column) publishes the exponent.
-constexpr int kColExpRows = 512;
-__global__ __launch_bounds__(256) void col_exponent_kernel(const double* __restrict__ B, int64_t nk, int64_t nj,
-                                                           int* __restrict__ fb) {
-  __shared__ double red[4][64];
+// Maxima of 64 columns of B over the rows [k0, ke), as exponents (INT32_MIN for
+// a column of zeros): wavefront w reads rows w, w + 4, ... (each load is 64
+// consecutive columns of one row, 16 loads in flight per work-item), and the
+// four wavefronts' maxima meet in LDS.
+__device__ __forceinline__ void column_exponents(const double* __restrict__ B, int64_t j0, int64_t k0, int64_t ke,
+                                                 int64_t nj, int* __restrict__ out, double* red) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t j = int64_t(blockIdx.x) * 64 + lane;
-  const int64_t k0 = int64_t(blockIdx.y) * kColExpRows;
-  const int64_t ke = (k0 + kColExpRows < nk) ? k0 + kColExpRows : nk;
+  const int64_t j = j0 + lane;
   double m = 0.0;
   if (j < nj) {
     int64_t k = k0 + w;
@@ -245,17 +257,34 @@ __global__ __launch_bounds__(256) void col_exponent_kernel(const double* __restr
     }
     for (; k < ke; k += 4) m = fmax(m, fabs(B[k * nj + j]));
   }
-  red[w][lane] = m;
+  red[w * 64 + lane] = m;
   __syncthreads();
   if (w == 0 && j < nj) {
-    m = fmax(fmax(red[0][lane], red[1][lane]), fmax(red[2][lane], red[3][lane]));
-    if (m != 0.0) atomicMax(&fb[j], exponent_of(m));
+    m = fmax(fmax(red[lane], red[64 + lane]), fmax(red[128 + lane], red[192 + lane]));
+    out[j] = m != 0.0 ? exponent_of(m) : INT32_MIN;
   }
 }
 
-__global__ void fill_int_kernel(int* p, int64_t n, int v) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
+constexpr int64_t kChunkRows = 512;
+
+// Both in one launch: B's column exponents need none of A's work, and neither
+// fills the memory by itself.  (On two streams, joined by events, they cost a
+// call 10 us more at 1000 x 1000 x 1200 and no less at 4096^3.)  `chunks` parts of B's rows leave their exponents
+// in part[chunk][njp] for split_cols_kernel.
+__global__ __launch_bounds__(256) void prepare_kernel(const double* __restrict__ A, const double* __restrict__ B,
+                                                      int64_t ni, int64_t nj, int64_t nk, int64_t nkp, int64_t nip,
+                                                      int64_t njp, int64_t chunk_rows, int64_t column_blocks,
+                                                      signed char* __restrict__ As, int* __restrict__ ea,
+                                                      int* __restrict__ part, const CrtParams P) {
+  __shared__ double red[256];
+  const int64_t b = blockIdx.x;
+  if (b < column_blocks) {
+    const int64_t groups = njp / 64, chunk = b / groups, k0 = chunk * chunk_rows;
+    const int64_t ke = k0 + chunk_rows < nk ? k0 + chunk_rows : nk;
+    column_exponents(B, b % groups * 64, k0, ke, nj, part + chunk * njp, red);
+  } else {
+    split_row(A, b - column_blocks, ni, nk, nkp, nip, As, ea, P, red);
+  }
 }
 
 // B -> Bs[t][j][k]: a workgroup owns 64 columns x 128 k; work-item (w, j)
@@ -267,7 +296,8 @@ __global__ void fill_int_kernel(int* p, int64_t n, int v) {
 // of Bs, so every store instruction writes eight whole lines.
 constexpr int kColPitch = 144;  // bytes per LDS row of the B transpose
 __global__ __launch_bounds__(512) void split_cols_kernel(const double* __restrict__ B, int64_t nk, int64_t nj,
-                                                         int64_t nkp, int64_t njp, const int* __restrict__ fb,
+                                                         int64_t nkp, int64_t njp, const int* __restrict__ part,
+                                                         int chunks, int* __restrict__ fb,
                                                          signed char* __restrict__ Bs, const CrtParams P) {
   __shared__ __attribute__((aligned(16))) signed char lds[2][64 * kColPitch];
   const int tid = threadIdx.x;
@@ -275,7 +305,14 @@ __global__ __launch_bounds__(512) void split_cols_kernel(const double* __restric
   const int64_t j = j0 + (tid & 63);
   const int64_t kb = int64_t(blockIdx.y) * 128;
   const int64_t k0 = kb + 16 * (tid >> 6);
-  const int f = (j < nj) ? fb[j] : 0;
+  int f = INT32_MIN;
+  if (j < nj) {
+    for (int c = 0; c < chunks; ++c) {
+      const int e = part[c * njp + j];
+      f = e > f ? e : f;
+    }
+    if (blockIdx.y == 0 && tid < 64) fb[j] = f;
+  }
   const int sh = P.b - (f == INT32_MIN ? 0 : f);
   double x[16];
   if (j < nj && k0 + 16 <= nk) {
@@ -285,21 +322,22 @@ __global__ __launch_bounds__(512) void split_cols_kernel(const double* __restric
 #pragma unroll
     for (int u = 0; u < 16; ++u) x[u] = (j < nj && k0 + u < nk) ? B[(k0 + u) * nj + j] : 0.0;
   }
+  unsigned low[16];
 #pragma unroll
-  for (int u = 0; u < 16; ++u) x[u] = rint(ldexp(x[u], sh));
+  for (int u = 0; u < 16; ++u) {
+    x[u] = rint(ldexp(x[u], sh));
+    low[u] = low_word(x[u]);
+  }
   const int jj = tid & 63, w16 = 16 * (tid >> 6);  // this work-item's LDS row and byte offset in it
   const int rrow = tid >> 3, rpart = 16 * (tid & 7);  // the row chunk it stores
   for (int t = 0; t < P.T; ++t) {
     v4i w;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      int packed = 0;
+      unsigned r[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int r = sym_mod(x[4 * c + q], P.m[t], P.inv[t]);
-        packed |= (r & 0xFF) << (8 * q);
-      }
-      w[c] = packed;
+      for (int q = 0; q < 4; ++q) r[q] = sym_mod(x[4 * c + q], low[4 * c + q], P.inv[t], P.minus_m[t]);
+      w[c] = int(pack4(r[0], r[1], r[2], r[3]));
     }
     signed char* buf = lds[t & 1];
     *reinterpret_cast<v4i*>(buf + jj * kColPitch + w16) = w;
@@ -351,7 +389,7 @@ typedef const __attribute__((address_space(1))) void global_void;
 __global__ __launch_bounds__(kThreads) void ozaki_gemm_kernel(unsigned* __restrict__ R,
                                                               const signed char* __restrict__ As,
                                                               const signed char* __restrict__ Bs, int64_t nip,
-                                                              int64_t njp, int64_t nkp, int tiles_n,
+                                                              int64_t njp, int64_t nkp, int tiles_n, int per_group,
                                                               const CrtParams P) {
   __shared__ v4i A0[kTM * kChunks], A1[kTM * kChunks];
   __shared__ v4i B0[kTN * kChunks], B1[kTN * kChunks];
@@ -361,7 +399,9 @@ __global__ __launch_bounds__(kThreads) void ozaki_gemm_kernel(unsigned* __restri
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = (wave >> 1) * kWaveM, wn = (wave & 1) * kWaveN;
   const int ksteps = int(nkp / kTK);  // even: nkp is a multiple of 2 kTK
-  const int total = P.T * ksteps;     // stages over all moduli
+  const int t_begin = int(blockIdx.y) * per_group;  // this workgroup's moduli
+  const int t_end = t_begin + per_group < P.T ? t_begin + per_group : P.T;
+  const int total = t_end * ksteps;  // the stage after its last
   const int fr = lane & 15, fk = lane >> 4;  // MFMA operand row and k quarter
   // This wavefront's fragments in the residue array: [tile][wave][i][j][lane].
   const int64_t frag0 = ((tm * tiles_n + tn) * (kThreads / kWave) + wave) * (kFm * kFn);
@@ -424,9 +464,9 @@ __global__ __launch_bounds__(kThreads) void ozaki_gemm_kernel(unsigned* __restri
     asm volatile("" ::: "memory");
   };
 
-  load_stage(0, A0, B0);
-  int g = 0;
-  for (int t = 0; t < P.T; ++t) {
+  int g = t_begin * ksteps;
+  load_stage(g, A0, B0);
+  for (int t = t_begin; t < t_end; ++t) {
 #pragma unroll
     for (int i = 0; i < kFm; ++i)
 #pragma unroll
@@ -441,24 +481,30 @@ __global__ __launch_bounds__(kThreads) void ozaki_gemm_kernel(unsigned* __restri
     }
     // d_t = the sum's symmetric residue modulo m_t (|sum| < 2^31, see
     // sym_mod); the four rows of a lane's accumulator go to one 32-bit word.
-    const double m = P.m[t], inv = P.inv[t];
+    const double inv = P.inv[t];
+    const unsigned minus_m = P.minus_m[t];
     unsigned* rt = R + int64_t(t) * per_mod + frag0 * kWave + lane;
 #pragma unroll
     for (int i = 0; i < kFm; ++i)
 #pragma unroll
       for (int j = 0; j < kFn; ++j) {
-        unsigned w = 0;
+        unsigned d[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) w |= unsigned(sym_mod(double(acc[i][j][r]), m, inv) & 0xFF) << (8 * r);
-        rt[(i * kFn + j) * kWave] = w;
+        for (int r = 0; r < 4; ++r) d[r] = sym_mod(double(acc[i][j][r]), unsigned(acc[i][j][r]), inv, minus_m);
+        rt[(i * kFn + j) * kWave] = pack4(d[0], d[1], d[2], d[3]);
       }
   }
 }
 
 // One work-item per (fragment, lane): the four outputs of that accumulator
 // slot.  X/M = sum_t d_t (h_t + l_t) mod 1; the h_t part is exact (every
-// term is a multiple of 2^-44 below 128 in magnitude and the sum is reduced
-// modulo 1 after each add).
+// term is a multiple of 2^-44 below 128 in magnitude, and the sum is reduced
+// modulo 1 after every three: below 385, it is a 53-bit multiple of 2^-44).
+// T is a template parameter: with it as a variable the loop over the moduli
+// was not unrolled and indexed the words through the index register (13 moduli,
+// 1000 x 1000: 8.0 us, 6.0 here; 4096 x 4096: 76 us both, 54 for the 13 bytes
+// in and 8 out of an element).
+template <int T>
 __global__ __launch_bounds__(256) void crt_combine_kernel(double* __restrict__ C, const unsigned* __restrict__ R,
                                                           const int* __restrict__ ea, const int* __restrict__ fb,
                                                           double alpha, double beta, int use_beta, int64_t ni,
@@ -474,20 +520,19 @@ __global__ __launch_bounds__(256) void crt_combine_kernel(double* __restrict__ C
   const int wave = f / (kFm * kFn), i = (f / kFn) % kFm, j = f % kFn;
   const int64_t row0 = (tile / tiles_n) * kTM + (wave >> 1) * kWaveM + i * 16 + 4 * (lane >> 4);
   const int64_t col = (tile % tiles_n) * kTN + (wave & 1) * kWaveN + j * 16 + (lane & 15);
-  // All residue words first (T <= 16), so their loads are in flight together.
-  unsigned wv[kMaxMods];
+  // All residue words first, so their loads are in flight together.
+  unsigned wv[T];
 #pragma unroll
-  for (int t = 0; t < kMaxMods; ++t) wv[t] = t < P.T ? R[int64_t(t) * per_mod + g] : 0u;
+  for (int t = 0; t < T; ++t) wv[t] = R[int64_t(t) * per_mod + g];
   double fh[4] = {0.0, 0.0, 0.0, 0.0}, fl[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int t = 0; t < kMaxMods; ++t) {
-    if (t >= P.T) break;
+  for (int t = 0; t < T; ++t) {
     const double h = P.h[t], l = P.l[t];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const double d = double(int(wv[t] << (24 - 8 * r)) >> 24);  // the signed byte r
-      const double s = fma(d, h, fh[r]);  // exact: multiples of 2^-44 below 129 in magnitude
-      fh[r] = s - floor(s);
+      fh[r] = fma(d, h, fh[r]);
+      if (t % 3 == 2) fh[r] = __builtin_amdgcn_fract(fh[r]);
       fl[r] = fma(d, l, fl[r]);
     }
   }
@@ -501,7 +546,8 @@ __global__ __launch_bounds__(256) void crt_combine_kernel(double* __restrict__ C
     // X = (fx + fl) M with fx = fh - nearest integer (exact, a multiple of
     // 2^-52 in [-1/2, 1/2]) and M = M_hi + M_lo: the product fx M_hi is
     // split exactly by an fma, the small terms are added to its error.
-    double fx = fh[r] - rint(fh[r]);
+    const double f1 = __builtin_amdgcn_fract(fh[r]);
+    double fx = f1 - rint(f1);
     if (fx + fl[r] > 0.5) fx -= 1.0;
     if (fx + fl[r] < -0.5) fx += 1.0;
     const double p = fx * P.M_hi;
@@ -513,32 +559,26 @@ __global__ __launch_bounds__(256) void crt_combine_kernel(double* __restrict__ C
   }
 }
 
-// A's row split does not depend on B's column exponents or B's split, so it
-// runs on a library-owned auxiliary stream (non-blocking, default
-// priority), forked from and joined back to the caller's stream with events;
-// stream capture follows the fork and join.  One auxiliary stream and event
-// pair per device, created on first use; the mutex keeps concurrent callers
-// from recording the shared events at the same time.
-struct AuxStream {
-  hipStream_t aux = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr;
-};
-constexpr int kMaxDevices = 64;
-std::mutex g_aux_mu;
-AuxStream g_aux[kMaxDevices];
+template <int T = 1, class... Args>
+void launch_combine(int moduli, dim3 grid, hipStream_t s, const Args&... args) {
+  if (moduli == T) crt_combine_kernel<T><<<grid, dim3(256), 0, s>>>(args...);
+  else if constexpr (T < kMaxMods) launch_combine<T + 1>(moduli, grid, s, args...);
+}
 
-int aux_for_device(AuxStream** out) {
-  int dev = -1;
-  RPX_TRY(hipGetDevice(&dev));
-  if (dev < 0 || dev >= kMaxDevices) return RPX_ERR_UNSUPPORTED;
-  AuxStream& a = g_aux[dev];
-  if (!a.aux) {
-    RPX_TRY(hipStreamCreateWithFlags(&a.aux, hipStreamNonBlocking));
-    RPX_TRY(hipEventCreateWithFlags(&a.fork, hipEventDisableTiming));
-    RPX_TRY(hipEventCreateWithFlags(&a.join, hipEventDisableTiming));
+// Moduli per workgroup.  With all T in one, the tiles of a small C leave most
+// CUs idle (512^3 on four workgroups: 135 us a call, 28 on 52; 2048^3 on 64:
+// 400 us, 178 on 256); each modulus is a GEMM of its own,
+// so they go to as many workgroups as make the fewest stages in a row.  A
+// workgroup costs about two stages besides (its first loads, its launch), and
+// more rounds of 256 workgroups are taken only for fewer stages.
+int moduli_per_group(int64_t tiles, int T, int64_t ksteps) {
+  int best = T;
+  int64_t least = INT64_MAX;
+  for (int per = T; per >= 1; --per) {
+    const int64_t stages = ceil_div(tiles * ceil_div(T, per), int64_t(256)) * (per * ksteps + 2);
+    if (stages < least) least = stages, best = per;
   }
-  *out = &a;
-  return RPX_SUCCESS;
+  return best;
 }
 
 }  // namespace
@@ -577,7 +617,7 @@ int rpx_gemm_mixed_tuned_f64(double* C, const double* A, const double* B, double
   const MixedLayout l = mixed_layout(ni, nj, nk, P.T);
   if (scratch_bytes < l.total) return RPX_ERR_SCRATCH_TOO_SMALL;
   const int64_t tm = l.nip / kTM, tn = l.njp / kTN;
-  if (l.nip > INT32_MAX || tm * tn > INT32_MAX || ceil_div(l.nip * l.njp / 4, 256) > INT32_MAX)
+  if (l.nip + l.njp > INT32_MAX || tm * tn > INT32_MAX || ceil_div(l.nip * l.njp / 4, 256) > INT32_MAX)
     return RPX_ERR_UNSUPPORTED;
   char* base = reinterpret_cast<char*>(scratch);
   signed char* As = reinterpret_cast<signed char*>(base + l.a_off);
@@ -586,25 +626,20 @@ int rpx_gemm_mixed_tuned_f64(double* C, const double* A, const double* B, double
   int* fb = reinterpret_cast<int*>(base + l.fb_off);
   unsigned* R = reinterpret_cast<unsigned*>(base + l.r_off);
   hipStream_t s = as_stream(stream);
-  std::lock_guard<std::mutex> lock(g_aux_mu);
-  AuxStream* ax = nullptr;
-  if (const int st = aux_for_device(&ax); st != RPX_SUCCESS) return st;
-  RPX_TRY(hipEventRecord(ax->fork, s));
-  RPX_TRY(hipStreamWaitEvent(ax->aux, ax->fork, 0));
-  split_rows_kernel<<<dim3(unsigned(l.nip)), dim3(256), 0, ax->aux>>>(A, ni, nk, l.nkp, l.nip, As, ea, P);
-  if (const int st = launch_status(); st != RPX_SUCCESS) return st;
-  RPX_TRY(hipEventRecord(ax->join, ax->aux));
-  fill_int_kernel<<<dim3(unsigned(ceil_div(l.njp, 256))), dim3(256), 0, s>>>(fb, l.njp, INT32_MIN);
-  if (nk > 0)
-    col_exponent_kernel<<<dim3(unsigned(ceil_div(nj, 64)), unsigned(ceil_div(nk, kColExpRows))), dim3(256), 0, s>>>(
-        B, nk, nj, fb);
-  split_cols_kernel<<<dim3(unsigned(l.njp / 64), unsigned(l.nkp / 128)), dim3(512), 0, s>>>(B, nk, nj, l.nkp, l.njp,
-                                                                                           fb, Bs, P);
-  RPX_TRY(hipStreamWaitEvent(s, ax->join, 0));
-  ozaki_gemm_kernel<<<dim3(unsigned(tm * tn)), dim3(kThreads), 0, s>>>(R, As, Bs, l.nip, l.njp, l.nkp, int(tn), P);
+  // The column exponents' parts lie where the residue bytes d_t go later.
+  int* part = reinterpret_cast<int*>(base + l.r_off);
+  const int64_t chunks = nk > 0 ? std::min(ceil_div(nk, kChunkRows), int64_t(kTM / 4)) : 0;
+  const int64_t chunk_rows = chunks > 0 ? ceil_div(nk, chunks) : 0, column_blocks = chunks * (l.njp / 64);
+  prepare_kernel<<<dim3(unsigned(column_blocks + l.nip)), dim3(256), 0, s>>>(
+      A, B, ni, nj, nk, l.nkp, l.nip, l.njp, chunk_rows, column_blocks, As, ea, part, P);
+  split_cols_kernel<<<dim3(unsigned(l.njp / 64), unsigned(l.nkp / 128)), dim3(512), 0, s>>>(
+      B, nk, nj, l.nkp, l.njp, part, int(chunks), fb, Bs, P);
+  const int per_group = moduli_per_group(tm * tn, P.T, l.nkp / kTK);
+  ozaki_gemm_kernel<<<dim3(unsigned(tm * tn), unsigned(ceil_div(P.T, per_group))), dim3(kThreads), 0, s>>>(
+      R, As, Bs, l.nip, l.njp, l.nkp, int(tn), per_group, P);
   const int use_beta = (tune_flags(tune) & RPX_TUNE_GEMM_BETA) != 0;
-  crt_combine_kernel<<<dim3(unsigned(ceil_div(l.nip * l.njp / 4, 256))), dim3(256), 0, s>>>(
-      C, R, ea, fb, alpha, beta, use_beta, ni, nj, l.nip, l.njp, int(tn), P);
+  const dim3 combine(unsigned(ceil_div(l.nip * l.njp / 4, 256)));
+  launch_combine(P.T, combine, s, C, R, ea, fb, alpha, beta, use_beta, ni, nj, l.nip, l.njp, int(tn), P);
   return launch_status();
 }
 
