@@ -696,7 +696,7 @@ int rpx_jacobi2d_fused_f64(double* A, double* B, int64_t N, int64_t tsteps, void
   // Without a requested tile or depth the register-resident tiles take every
   // grid, odd N too, that they have room for: all tested N from 131 to 8192
   // are faster on them (N = 1002, 40 steps: 82 against 374 us; N = 8192, 50
-  // steps: 2.99 against 3.98 ms).  One time step stays with the two in-place
+  // steps: 2.61 against 3.98 ms).  One time step stays with the two in-place
   // sweeps, which a tile launch and a copy back would not beat.
   const bool untuned = tune_or(tune, &rpx_tuning::items_per_thread, 0) == 0 && tune_or(tune, &rpx_tuning::depth, 0) == 0;
   if (untuned && N <= kJacobiOneTileN) return jacobi_one_tile(A, B, N, tsteps, s);

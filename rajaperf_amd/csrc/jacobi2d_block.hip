@@ -4,7 +4,8 @@
 // Reference: src/polybench/POLYBENCH_JACOBI_2D-Seq.cpp:30-54 (tsteps x two
 // sweeps over the interior).
 //
-// A workgroup of W wavefronts holds W*RW rows of 128 columns: a lane holds
+// Two forms of tile.  In the narrow one a workgroup of W wavefronts holds W*RW
+// rows of 128 columns: a lane holds
 // the column pair 2*lane of RW consecutive rows, twice (the A and the B of the
 // time step).  A sweep computes one array from the other; west and east
 // neighbours come from the adjacent lanes (DPP moves), the rows above and
@@ -23,8 +24,11 @@
 // N = 1002, 40 time steps: 374 us with the 16-row wavefront tiles of
 // jacobi_fused_kernel (13 launches of 27 us, each one wavefront's serial
 // chain of 28 rows x 6 levels), 82 us here (7 launches).  N = 8192, 50 time
-// steps: 3.98 ms with streaming chunks, 2.99 ms here.
+// steps: 3.98 ms with streaming chunks, 2.96 ms on narrow tiles of 88 rows,
+// 2.61 ms on wide ones (below).
 #include "jacobi2d.hpp"
+
+#include <cmath>
 
 using namespace rpx;
 
@@ -189,6 +193,204 @@ __global__ __launch_bounds__(W* kWave, 4) void jacobi_block_kernel(const BlockAr
     block_tile<W, RW, kInner>(g, edge, rbase, j0, wave, lane, r_begin, r_end, c_begin, c_end);
 }
 
+// ---- wide tiles --------------------------------------------------------------
+//
+// 256 columns: a lane holds four columns of RW rows, once, and a sweep replaces
+// them in place: half the registers per point, so twice the columns and less
+// halo, and four DPP moves for 20 FP64 instructions instead of 10 (a row and
+// sweep of 256 columns takes 127 clocks, two of 128 columns 128, but 64 of 100
+// points of an 88-row tile are kept at six steps and not 54).  N = 8192: 326 us
+// per launch of 6.25 steps, 165 of which the memory needs and about 225 the
+// FP64 units, in part one after the other: two workgroups per CU are all that
+// the registers hold.  From N = 2000 or so; smaller grids have too few of them.
+// The grid's boundary cells, which the A and the B level have of their own,
+// wait in LDS for the tiles that hold any.
+constexpr int kWideCols = 256;
+
+template <int W, int RW>
+struct WideRoom {
+  v2d edge[2][W][2][2][kWave];   // [parity][wavefront][first or last row][pair]
+  v2d row[2][2][2][kWave];       // the grid's first or last row, [A or B][pair]
+  double column[2][W * RW];      // its first or last column, [A or B]
+};
+
+typedef double Quad[4];
+__device__ __forceinline__ void put_quad(v2d (*to)[kWave], int lane, const Quad& q) {
+  to[0][lane] = v2d{q[0], q[1]};
+  to[1][lane] = v2d{q[2], q[3]};
+}
+__device__ __forceinline__ void get_quad(Quad& q, const v2d (*from)[kWave], int lane) {
+  const v2d l = from[0][lane], r = from[1][lane];
+  q[0] = l.x, q[1] = l.y, q[2] = r.x, q[3] = r.y;
+}
+__device__ __forceinline__ void load_quad(Quad& q, const double* from) {
+  const v2d l = *reinterpret_cast<const v2d_u*>(from), r = *reinterpret_cast<const v2d_u*>(from + 2);
+  q[0] = l.x, q[1] = l.y, q[2] = r.x, q[3] = r.y;
+}
+
+// One sweep.  q[RW + 1] holds the A level's row i in q[i + 1] and the B level's
+// in q[i]: the sweep from A to B (LEVEL = 1) goes down and puts each new row
+// where the old row above it was, the sweep back goes up and puts it where the
+// old row below it was.
+template <int W, int RW, int SIDE, int LEVEL>
+__device__ __forceinline__ void wide_sweep(Quad (&q)[RW + 1], WideRoom<W, RW>& m, int wave, int lane, bool first,
+                                           bool last) {
+  // Row i, with its old neighbours up and dn.
+  auto row = [&](int i, const Quad& up, const Quad& dn) {
+    const Quad& c = q[i + LEVEL];
+    Quad r;
+    const double w = from_west(c[3]), e = from_east(c[0]);
+    r[0] = point(c[0], w, c[1], dn[0], up[0]);
+    r[1] = point(c[1], c[0], c[2], dn[1], up[1]);
+    r[2] = point(c[2], c[1], c[3], dn[2], up[2]);
+    r[3] = point(c[3], c[2], e, dn[3], up[3]);
+    if (SIDE == kWest) r[0] = lane == 0 ? m.column[LEVEL][wave * RW + i] : r[0];
+    if (SIDE == kEast) r[3] = lane == kWave - 1 ? m.column[LEVEL][wave * RW + i] : r[3];
+    // Pinned: the optimiser otherwise moves the rows' last steps behind the
+    // branches below, old rows and all, and spills.
+    asm volatile("" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]));
+    __builtin_amdgcn_sched_barrier(0);  // one row at a time
+#pragma unroll
+    for (int k = 0; k < 4; ++k) q[i + 1 - LEVEL][k] = r[k];
+  };
+  auto top = [&] {
+    if (first) {
+      get_quad(q[1 - LEVEL], m.row[0][LEVEL], lane);
+    } else {
+      Quad up;
+      get_quad(up, m.edge[1 - LEVEL][wave > 0 ? wave - 1 : 0][1], lane);
+      row(0, up, q[1 + LEVEL]);
+    }
+    put_quad(m.edge[LEVEL][wave][0], lane, q[1 - LEVEL]);
+  };
+  auto bottom = [&] {
+    if (last) {
+      get_quad(q[RW - LEVEL], m.row[1][LEVEL], lane);
+    } else {
+      Quad dn;
+      get_quad(dn, m.edge[1 - LEVEL][wave < W - 1 ? wave + 1 : wave][0], lane);
+      row(RW - 1, q[RW - 2 + LEVEL], dn);
+    }
+    put_quad(m.edge[LEVEL][wave][1], lane, q[RW - LEVEL]);
+  };
+  if (LEVEL == 1) {
+    top();
+#pragma unroll
+    for (int i = 1; i < RW - 1; ++i) row(i, q[i], q[i + 2]);
+    bottom();
+  } else {
+    bottom();
+#pragma unroll
+    for (int i = RW - 2; i > 0; --i) row(i, q[i - 1], q[i + 1]);
+    top();
+  }
+  __syncthreads();
+}
+
+// LAST: the launch that stores the last B as well.
+template <int W, int RW, int SIDE, bool LAST>
+__device__ __forceinline__ void wide_tile(const BlockArgs& g, WideRoom<W, RW>& m, int64_t rbase, int64_t j0, int wave,
+                                          int lane, int r_begin, int r_end, int c_begin, int c_end) {
+  const int64_t N = g.N, row0 = rbase + wave * RW, at0 = row0 * N + j0 + 4 * lane;
+  const int first = row0 == 0, last = row0 + RW == N;
+  Quad q[RW + 1];  // A's row i in q[i + 1]
+#pragma unroll
+  for (int i = 0; i < RW; ++i) load_quad(q[i + 1], g.Ain + at0 + i * N);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) q[0][k] = 0.0;
+  auto boundary_row = [&](Quad& r, int64_t at, v2d (*room)[2][kWave]) {
+    load_quad(r, g.B + at);
+    put_quad(room[1], lane, r);
+    load_quad(r, g.Abnd + at);
+    put_quad(room[0], lane, r);
+  };
+  if (first) boundary_row(q[1], at0, m.row[0]);
+  if (last) boundary_row(q[RW], at0 + (RW - 1) * N, m.row[1]);
+  if (SIDE != kInner) {
+    const int64_t edge_col = SIDE == kWest ? 0 : N - 1;
+    if (lane < RW) {
+      m.column[0][wave * RW + lane] = g.Abnd[(row0 + lane) * N + edge_col];
+      m.column[1][wave * RW + lane] = g.B[(row0 + lane) * N + edge_col];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+      const double b = m.column[0][wave * RW + i];
+      if (SIDE == kWest) q[i + 1][0] = lane == 0 ? b : q[i + 1][0];
+      else q[i + 1][3] = lane == kWave - 1 ? b : q[i + 1][3];
+    }
+  }
+  put_quad(m.edge[0][wave][0], lane, q[1]);
+  put_quad(m.edge[0][wave][1], lane, q[RW]);
+  __syncthreads();
+  auto store = [&](double* out, int slot) {
+    int64_t base = at0;  // opaque, or the addresses of all rows are kept through the time steps
+    asm volatile("" : "+v"(base));
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+      const int k = wave * RW + i;
+      if (k < r_begin || k >= r_end) continue;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int c = 4 * lane + 2 * h;
+        const bool x_own = c >= c_begin && c < c_end, y_own = c + 1 >= c_begin && c + 1 < c_end;
+        double* at = out + base + i * N + 2 * h;
+        if (x_own && y_own) *reinterpret_cast<v2d_u*>(at) = v2d{q[i + slot][2 * h], q[i + slot][2 * h + 1]};
+        if (SIDE == kInner) continue;  // whole pairs
+        if (x_own && !y_own) at[0] = q[i + slot][2 * h];
+        if (y_own && !x_own) at[1] = q[i + slot][2 * h + 1];
+      }
+    }
+  };
+  // Opaque to the optimiser, which otherwise makes copies of the loop.
+  int is_first, is_last;
+  auto opaque = [&] {
+    is_first = __builtin_amdgcn_readfirstlane(first), is_last = __builtin_amdgcn_readfirstlane(last);
+    asm volatile("" : "+s"(is_first), "+s"(is_last));
+  };
+  for (int64_t t = LAST; t < g.steps; ++t) {
+    opaque();
+    wide_sweep<W, RW, SIDE, 1>(q, m, wave, lane, is_first, is_last);
+    wide_sweep<W, RW, SIDE, 0>(q, m, wave, lane, is_first, is_last);
+  }
+  if (LAST) {
+    opaque();
+    wide_sweep<W, RW, SIDE, 1>(q, m, wave, lane, is_first, is_last);
+    store(g.B, 0);
+    wide_sweep<W, RW, SIDE, 0>(q, m, wave, lane, is_first, is_last);
+  }
+  store(g.Aout, 1);
+}
+
+template <int W, int RW, bool LAST>
+__global__ __launch_bounds__(W* kWave, 4) void jacobi_wide_kernel(const BlockArgs g) {
+  __shared__ WideRoom<W, RW> room;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const unsigned tile = xcd_major(blockIdx.x, gridDim.x);
+  const int strip = int(tile % unsigned(g.strips)), chunk = int(tile / unsigned(g.strips));
+  const int halo = 2 * int(g.steps);
+  int64_t j0 = int64_t(strip) * g.own_c, rbase = int64_t(chunk) * g.own_r;
+  int c_begin = strip == 0 ? 1 : halo, c_end = halo + g.own_c;
+  int r_begin = chunk == 0 ? 1 : halo, r_end = halo + g.own_r;
+  if (strip == g.strips - 1) {
+    c_begin += int(j0 - (g.N - kWideCols));
+    j0 = g.N - kWideCols;
+    c_end = kWideCols - 1;
+  }
+  if (chunk == g.chunks - 1) {
+    r_begin += int(rbase - (g.N - W * RW));
+    rbase = g.N - W * RW;
+    r_end = W * RW - 1;
+  }
+  if (strip == 0)
+    wide_tile<W, RW, kWest, LAST>(g, room, rbase, j0, wave, lane, r_begin, r_end, c_begin, c_end);
+  else if (strip == g.strips - 1)
+    wide_tile<W, RW, kEast, LAST>(g, room, rbase, j0, wave, lane, r_begin, r_end, c_begin, c_end);
+  else
+    wide_tile<W, RW, kInner, LAST>(g, room, rbase, j0, wave, lane, r_begin, r_end, c_begin, c_end);
+}
+
 // A whole grid of N <= 128 in one workgroup's registers.
 template <int W, int RW>
 __global__ __launch_bounds__(W* kWave) void jacobi_grid_kernel(const BlockArgs g) {
@@ -201,9 +403,21 @@ __global__ __launch_bounds__(W* kWave) void jacobi_grid_kernel(const BlockArgs g
 // Tiles: W wavefronts of RW rows.  Few rows leave small grids enough tiles
 // for 256 CUs; many rows recompute less halo on large ones.
 struct TileShape {
-  int waves, rows;
+  int waves, rows, cols;
+  double sweep_us;  // one sweep of a tile on a CU that has as many as it holds, per tile
+  double tbps;      // rate of a launch of few steps, which the memory bounds
 };
-constexpr TileShape kShapes[] = {{8, 4}, {8, 5}, {16, 4}, {16, 5}, {8, 10}, {8, 11}};
+constexpr TileShape kShapes[] = {{8, 4, kTileCols, 0.23, 4.75},  {8, 5, kTileCols, 0.295, 4.7},
+                                 {16, 4, kTileCols, 0.48, 4.65}, {16, 5, kTileCols, 0.78, 4.5},
+                                 {8, 10, kWideCols, 1.05, 4.1},  {8, 11, kWideCols, 1.145, 4.1}};
+
+template <int W, int RW>
+int launch_wide(const BlockArgs& g, hipStream_t s) {
+  const dim3 grid(unsigned(g.strips) * unsigned(g.chunks)), block(W * kWave);
+  if (g.store_b) jacobi_wide_kernel<W, RW, true><<<grid, block, 0, s>>>(g);
+  else jacobi_wide_kernel<W, RW, false><<<grid, block, 0, s>>>(g);
+  return launch_status();
+}
 
 template <int W, int RW>
 int launch_block(const BlockArgs& g, hipStream_t s) {
@@ -214,28 +428,31 @@ int launch_block(const BlockArgs& g, hipStream_t s) {
 // The tile counts of a launch; false where the shape does not fit.
 bool layout(BlockArgs& g, const TileShape& t) {
   const int rows = t.waves * t.rows;
-  g.own_c = int(kTileCols - 4 * g.steps);
+  g.own_c = int(t.cols - 4 * g.steps);
   g.own_r = int(rows - 4 * g.steps);
-  if (g.own_c <= 0 || g.own_r <= 0 || g.N < kTileCols || g.N < rows) return false;
-  const int64_t strips = 1 + ceil_div(g.N - kTileCols, g.own_c), chunks = 1 + ceil_div(g.N - rows, g.own_r);
+  if (g.own_c <= 0 || g.own_r <= 0 || g.N <= t.cols || g.N < rows) return false;
+  const int64_t strips = 1 + ceil_div(g.N - t.cols, g.own_c), chunks = 1 + ceil_div(g.N - rows, g.own_r);
   if (strips * chunks > INT32_MAX) return false;
   g.strips = int(strips);
   g.chunks = int(chunks);
   return true;
 }
 
-// Time of a launch in microseconds, a fit to launches of all shapes and
-// depths at N = 131 to 8192 (within about 15%): 4 us, and the larger of the
-// sweeps' issue time and one read and write of the grid at 5 TB/s.  A sweep
-// of a tile takes 0.03 us + 0.033 us per row and SIMD; beyond 256 tiles a CU
-// runs several, and the last round is 0.4 full on average.
+// Time of a launch in microseconds, a fit to launches of all shapes and depths
+// at 16 grids from N = 300 to 8192 (the shape and depth that it picks are
+// within 3% of the fastest at all of them): 4.6 us, the sweeps' issue time, and
+// one read and write of the grid (slowest with wide tiles, whose lanes read and
+// write every other 16 bytes), which overlap in part.  A CU works on two
+// tiles at a time; an odd one out is alone, and its wavefronts then wait for
+// each other's edge rows.  Beyond four tiles per CU this evens out.
 double launch_us(BlockArgs g, const TileShape& t) {
   if (!layout(g, t)) return 1e30;
-  const double tiles = double(g.strips) * g.chunks / 256.0;
-  const double sweep = 0.03 + 0.033 * t.waves * t.rows / 4;
-  const double compute = (tiles <= 1 ? 1.0 : tiles + 0.4) * 2 * double(g.steps) * sweep;
-  const double memory = 16e-6 * double(g.N) * double(g.N) / 5.0;
-  return 4.0 + (compute > memory ? compute : memory);
+  const bool wide = t.cols == kWideCols;
+  const double tiles = double(g.strips) * g.chunks / 256.0, n = std::ceil(tiles), alone = wide ? 1.36 : 1.07;
+  const double rounds = n > 4 ? tiles : std::fmod(n, 2.0) == 1.0 ? n - 1 + alone : n;
+  const double sweeps = rounds * 2 * double(g.steps) * t.sweep_us;
+  const double memory = 16e-6 * double(g.N) * double(g.N) / t.tbps;
+  return 4.6 + std::cbrt(sweeps * sweeps * sweeps + memory * memory * memory);
 }
 
 int launch_shape(BlockArgs g, int shape, hipStream_t s) {
@@ -245,8 +462,8 @@ int launch_shape(BlockArgs g, int shape, hipStream_t s) {
     case 1: return launch_block<8, 5>(g, s);
     case 2: return launch_block<16, 4>(g, s);
     case 3: return launch_block<16, 5>(g, s);
-    case 4: return launch_block<8, 10>(g, s);
-    default: return launch_block<8, 11>(g, s);
+    case 4: return launch_wide<8, 10>(g, s);
+    default: return launch_wide<8, 11>(g, s);
   }
 }
 
