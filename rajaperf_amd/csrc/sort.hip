@@ -21,8 +21,8 @@
 //   bucket:  every bucket (and every short segment) sorted.
 // So a key moves twice and is read once more, where a least-significant-digit
 // radix sort of 8-bit digits, which this replaces, moves it eight times and
-// reads it eight times more: 41.6 M keys in 256 ragged segments 2.30 -> 0.63
-// ms, one segment of 10^6 keys (24 launches then, 6 now) 0.30 -> 0.07 ms.
+// reads it eight times more: 41.6 M keys in 256 ragged segments 2.30 -> 0.58
+// ms, one segment of 10^6 keys (24 launches then, 7 now) 0.30 -> 0.054 ms.
 // Segments above kOneLevel keys are cut twice, first into about
 // sqrt(n / 4096) parts.  Keys equal to a repeated splitter go round robin to
 // the buckets between its copies, which hold nothing else and are not sorted,
@@ -39,8 +39,11 @@ namespace {
 
 typedef unsigned long long u64;
 
-constexpr int kBS = 256;
-constexpr int kRows = 16;
+// Work-items of hist and scatter, eight keys each.  What bounds both is the
+// latency of their LDS phases and loads; with 256 work-items of 16 keys half as
+// many wavefronts fit on a CU, and hist took 150 us instead of 101 (41.6 M keys).
+constexpr int kBS = 512;
+constexpr int kRows = 8;
 constexpr int kTile = kBS * kRows;  // 4096 keys per tile of hist and scatter
 constexpr int kAim = 4096;          // least mean of keys per bucket
 constexpr int kMaxK = 1024;         // buckets per segment and level
@@ -545,15 +548,32 @@ __device__ __forceinline__ void network_splitters(const u64 (&b)[1 << RB], int k
   }
 }
 
+// Key i of the 2^m sampled from len at src: that at (i + jitter 2^-16) len / 2^m.
+__device__ __forceinline__ u64 sampled_key(const u64* src, int len, int i, int m) {
+  const u64 jitter = mix64(u64(i) * kGamma + u64(len)) >> 48;
+  return src[(u64(i) << 16 | jitter) * u64(len) >> (16 + m)];
+}
+
+// A CU takes about 20 us to read 8192 keys from as many lines.  Where the
+// segments leave CUs free, kGather of them read a segment's sample and leave it
+// side by side where the segment's keys will go (10^6 keys: 28 us -> 5 and 10).
+constexpr int kGather = 8, kGatherSegs = 128;
+__global__ __launch_bounds__(256) void gather_kernel(u64* x, u64* alt, Level l) {
+  const int s = blockIdx.x / kGather;
+  const Seg g = get_seg(l, s);
+  if (g.k <= 1) return;
+  const u64* src = (g.src ? alt : x) + g.base;
+  u64* dst = (g.src ? x : alt) + g.base;
+  const int m = samples_for(g.k) == 2048 ? 11 : 13;
+  for (int i = int(blockIdx.x) % kGather * 256 + int(threadIdx.x); i < 1 << m; i += kGather * 256)
+    dst[i] = sampled_key(src, g.len, i, m);
+}
+
 template <int RB>
-__device__ __forceinline__ void sample_segment(const u64* src, const Seg& g, u64* splitters, int* dup, u64* sp,
-                                               char* mem, int t) {
+__device__ __forceinline__ void sample_segment(const u64* src, bool gathered, const Seg& g, u64* splitters, int* dup,
+                                               u64* sp, char* mem, int t) {
   constexpr int R = 1 << RB, T = 1 << kTB, M = kTB + RB, S = 1 << M;
-  const auto sampled = [&](int at) {
-    const u64 i = u64(at);
-    const u64 jitter = mix64(i * kGamma + u64(g.len)) >> 48;
-    return src[(i << 16 | jitter) * u64(g.len) >> (16 + M)];  // (i + jitter 2^-16) len / S
-  };
+  const auto sampled = [&](int i) { return gathered ? src[i] : sampled_key(src, g.len, i, M); };
   // Quantile j is the key at place floor(j S / k).
   const auto quantile = [&](int place, u64 b) {
     const int j = int((unsigned(place) * unsigned(g.k) + unsigned(S - 1)) >> M);
@@ -584,7 +604,7 @@ __device__ __forceinline__ void sample_segment(const u64* src, const Seg& g, u64
 // and its splitters.
 constexpr int kSampleBytes = linear_bytes(kTB, 8192);
 static_assert(kSampleBytes >= 8 * Net<AsDouble, kTB, 4>::kSlots, "the network fits too");
-__global__ __launch_bounds__(1 << kTB) void sample_kernel(const u64* x, const u64* alt, Level l) {
+__global__ __launch_bounds__(1 << kTB) void sample_kernel(const u64* x, const u64* alt, Level l, bool gathered) {
   __shared__ __attribute__((aligned(16))) char mem[kSampleBytes];
   __shared__ u64 sp[kMaxK];
   constexpr int T = 1 << kTB;
@@ -599,10 +619,10 @@ __global__ __launch_bounds__(1 << kTB) void sample_kernel(const u64* x, const u6
     }
   }
   if (g.k <= 1) return;
-  const u64* src = (g.src ? alt : x) + g.base;
+  const u64* src = ((g.src != 0) != gathered ? alt : x) + g.base;
   u64* splitters = l.splitters + g.first_bucket;
-  if (samples_for(g.k) == 2048) sample_segment<2>(src, g, splitters, l.dup + s, sp, mem, t);
-  else sample_segment<4>(src, g, splitters, l.dup + s, sp, mem, t);
+  if (samples_for(g.k) == 2048) sample_segment<2>(src, gathered, g, splitters, l.dup + s, sp, mem, t);
+  else sample_segment<4>(src, gathered, g, splitters, l.dup + s, sp, mem, t);
 }
 
 // ---- partition -----------------------------------------------------------------
@@ -1108,7 +1128,9 @@ Layout lay_out(const Sizes& s, void* scratch) {
 }
 
 int partition(u64* x, u64* alt, const Level& l, const LevelSize& z, hipStream_t st) {
-  sample_kernel<<<dim3(unsigned(l.nseg)), dim3(1 << kTB), 0, st>>>(x, alt, l);
+  const bool gathered = l.nseg <= kGatherSegs;
+  if (gathered) gather_kernel<<<dim3(unsigned(l.nseg * kGather)), dim3(256), 0, st>>>(x, alt, l);
+  sample_kernel<<<dim3(unsigned(l.nseg)), dim3(1 << kTB), 0, st>>>(x, alt, l, gathered);
   if (z.rows > 0) {
     hist_kernel<<<dim3(unsigned(z.rows)), dim3(kBS), 0, st>>>(x, alt, l);
     colscan_kernel<<<dim3(unsigned(z.cols)), dim3(kCol * kWalkers), 0, st>>>(l);

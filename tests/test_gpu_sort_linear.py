@@ -43,3 +43,12 @@ def test_both_workgroup_sizes(rpx, kind):
     for lens in ([1, 3824, 16, 0, 2000], [1, 3824, 16, 0, 2000, 7664, 5]):
         offs = [3] + [int(v) for v in 3 + np.cumsum(lens)]
         check(rpx, values(kind, offs[-1] + 4, rng), offs)
+
+
+@pytest.mark.parametrize("nseg", [128, 129])
+def test_gathered_and_own_samples(rpx, nseg):
+    # Up to 128 segments' samples are gathered by a kernel of their own.
+    rng = np.random.default_rng(nseg)
+    offs = [0] + [int(v) for v in np.cumsum(rng.integers(7000, 9000, nseg))]
+    check(rpx, values("uniform", offs[-1], rng), offs)
+    check(rpx, values("uniform", nseg * 8192, rng), [8192 * i for i in range(nseg + 1)])
