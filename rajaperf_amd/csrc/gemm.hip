@@ -213,23 +213,37 @@ __global__ __launch_bounds__(S::T, 2) void gemm_mfma_f64_kernel(double* __restri
     buf ^= 1;
   }
 
-  auto put = [&](int64_t gi, int64_t gj, double v) {
-    if (gi < ni && gj < nj) {
-      double* c = C + gi * nj + gj;
-      *c = use_beta ? fma(beta, *c, v) : v;
-    }
+  // With beta the old values of a batch of elements are loaded before the first
+  // of them is stored: each load would otherwise wait for the store before it
+  // (500^3 with beta and the copy of C: 14.9 us, 13.9 here).
+  auto old = [&](int64_t gi, int64_t gj) { return use_beta && gi < ni && gj < nj ? C[gi * nj + gj] : 0.0; };
+  auto put = [&](int64_t gi, int64_t gj, double v, double c) {
+    if (gi < ni && gj < nj) C[gi * nj + gj] = use_beta ? fma(beta, c, v) : v;
   };
   // v_mfma_f64_16x16x4f64 accumulator layout (measured on gfx950): element r
   // of lane l is row 4*r + l/16, column l%16.
   if constexpr (S::WK == 1) {
+    const int64_t row0 = m0 + wm + (lane >> 4), col0 = n0 + wn + fr;
 #pragma unroll
-    for (int i = 0; i < S::MF; ++i)
+    for (int i = 0; i < S::MF; ++i) {
+      double c[S::NF][4];
 #pragma unroll
       for (int j = 0; j < S::NF; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          put(m0 + wm + i * 16 + 4 * r + (lane >> 4), n0 + wn + j * 16 + fr, acc[i][j][r]);
+        for (int r = 0; r < 4; ++r) c[j][r] = old(row0 + i * 16 + 4 * r, col0 + j * 16);
+#pragma unroll
+      for (int j = 0; j < S::NF; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) put(row0 + i * 16 + 4 * r, col0 + j * 16, acc[i][j][r], c[j][r]);
+    }
   } else {
+    constexpr int kPer = (S::TM * S::TN + S::T - 1) / S::T;  // elements per work-item
+    double c[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int e = tid + u * S::T;
+      c[u] = e < S::TM * S::TN ? old(m0 + e / S::TN, n0 + e % S::TN) : 0.0;
+    }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < S::MF; ++i)
@@ -239,11 +253,14 @@ __global__ __launch_bounds__(S::T, 2) void gemm_mfma_f64_kernel(double* __restri
         for (int r = 0; r < 4; ++r)
           lds[(wk * S::TM + wm + i * 16 + 4 * r + (lane >> 4)) * S::TN + wn + j * 16 + fr] = acc[i][j][r];
     __syncthreads();
-    for (int e = tid; e < S::TM * S::TN; e += S::T) {
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int e = tid + u * S::T;
+      if (e >= S::TM * S::TN) continue;
       double v = lds[e];
 #pragma unroll
       for (int k = 1; k < S::WK; ++k) v += lds[k * S::TM * S::TN + e];
-      put(m0 + e / S::TN, n0 + e % S::TN, v);
+      put(m0 + e / S::TN, n0 + e % S::TN, v, c[u]);
     }
   }
 }
@@ -263,22 +280,27 @@ int launch_mfma(double* C, const double* A, const double* B, double alpha, doubl
 // split K over their wavefronts instead, so that few of them still fill the
 // matrix cores.
 //
-// What bounds them: FP64 MFMA issue, 64 clocks each (77 TF/s, measured).
-// 4096^3 runs at 65 TF/s (2.10 ms; 2.24 ms when A was scaled, and so waited
-// for, as it was loaded), its matrix cores busy 86% of the time; the rest is
-// LDS writes and the barrier between slabs.  1000 x 1000 x 1200 took 261 us as
-// 64 tiles of 128 x 128 on 256 CUs and takes 58 us as 256 tiles of 64 x 64
-// (31 us of MFMAs, 10 us of launch, first loads and epilogue, 8 us of LDS
-// writes, 6 us of loads).
-using Big = Shape<4, 4, 2, 2, 1, 16, 1>;     // 128 x 128, four wavefronts
+// What bounds them: FP64 MFMA issue, 64 clocks each (77 TF/s, measured), and
+// how evenly the tiles go over 256 CUs.  4096^3 runs at 66.7 TF/s (2.06 ms) on
+// sixteen wavefronts of 32 x 32 with slabs 32 deep; four wavefronts of 64 x 64,
+// slabs of 16 and two workgroups per CU took 2.14 ms, and as a lone tile kept
+// half of a SIMD's time: 2048^2 x 4096 612 -> 517 us, 4000 x 3000 x 2000
+// 1054 -> 785.  1000 x 1000 x 1200 took 261 us as 64 tiles of 128 x 128 on 256
+// CUs and takes 54 us as 256 tiles of 64 x 64 (31 us of MFMAs, 10 us of launch,
+// first loads and epilogue, the rest LDS writes and loads).  Tiles of 96 x 96
+// and 96 x 64 are for the sizes between: 1500^3 178 -> 129 us, 1100 x 1100 x
+// 4000 268 -> 244.
+using Big = Shape<2, 2, 4, 4, 1, 32, 2>;     // 128 x 128, sixteen wavefronts
+using Square = Shape<3, 2, 2, 3, 2, 16, 2>;  // 96 x 96, K in two, twelve wavefronts
+using Tall = Shape<3, 2, 2, 2, 2, 16, 2>;    // 96 x 64, K in two, eight wavefronts
 using Mid = Shape<2, 2, 2, 2, 2, 16, 2>;     // 64 x 64, K in two, two workgroups per CU
-using MidDeep = Shape<2, 2, 2, 2, 2, 32, 2>; // 64 x 64, K in two, one workgroup per CU
+using MidDeep = Shape<2, 2, 2, 2, 4, 16, 2>; // 64 x 64, K in four, one workgroup per CU
 using Small = Shape<2, 2, 1, 1, 4, 8, 1>;    // 32 x 32, K in four
 using SmallDeep = Shape<2, 2, 1, 1, 8, 8, 1>;// 32 x 32, K in eight
 using Tiny = Shape<1, 1, 1, 1, 8, 16, 1>;    // 16 x 16, K in eight
 
 // Time of a product without the launch, in microseconds: a tile alone on a CU
-// takes `alone` per unit of K, a CU's n-th tile `shared` (both fitted to 12
+// takes `alone` per unit of K, a CU's n-th tile `shared` (both fitted to 24
 // sizes from 64^3 to 4096^3, within about 15%).
 template <typename S>
 double mfma_us(int64_t ni, int64_t nj, int64_t nk, double alone, double shared) {
@@ -289,18 +311,21 @@ double mfma_us(int64_t ni, int64_t nj, int64_t nk, double alone, double shared) 
 
 int gemm_mfma(double* C, const double* A, const double* B, double alpha, double beta, int use_beta, int64_t ni,
               int64_t nj, int64_t nk, hipStream_t s) {
-  const double us[] = {mfma_us<Big>(ni, nj, nk, 0.145, 0.131),        mfma_us<Mid>(ni, nj, nk, 0.0435, 0.0365),
-                       mfma_us<MidDeep>(ni, nj, nk, 0.041, 0.041),    mfma_us<Small>(ni, nj, nk, 0.0163, 0.0122),
+  const double us[] = {mfma_us<Big>(ni, nj, nk, 0.126, 0.1255),        mfma_us<Square>(ni, nj, nk, 0.0845, 0.0835),
+                       mfma_us<Tall>(ni, nj, nk, 0.0605, 0.0595),      mfma_us<Mid>(ni, nj, nk, 0.0435, 0.0365),
+                       mfma_us<MidDeep>(ni, nj, nk, 0.0405, 0.039),    mfma_us<Small>(ni, nj, nk, 0.0163, 0.0122),
                        mfma_us<SmallDeep>(ni, nj, nk, 0.0138, 0.0122), mfma_us<Tiny>(ni, nj, nk, 0.0049, 0.0047)};
   int best = 0;
-  for (int i = 1; i < 6; ++i)
+  for (int i = 1; i < 8; ++i)
     if (us[i] < us[best]) best = i;
   switch (best) {
     case 0: return launch_mfma<Big>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
-    case 1: return launch_mfma<Mid>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
-    case 2: return launch_mfma<MidDeep>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
-    case 3: return launch_mfma<Small>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
-    case 4: return launch_mfma<SmallDeep>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
+    case 1: return launch_mfma<Square>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
+    case 2: return launch_mfma<Tall>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
+    case 3: return launch_mfma<Mid>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
+    case 4: return launch_mfma<MidDeep>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
+    case 5: return launch_mfma<Small>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
+    case 6: return launch_mfma<SmallDeep>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
     default: return launch_mfma<Tiny>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
   }
 }
