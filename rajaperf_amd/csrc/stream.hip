@@ -8,11 +8,13 @@
 // (global_load_dwordx4 / global_store_dwordx4); the U vectors of one
 // work-item are a workgroup-width apart, so every vector instruction of a
 // wavefront covers 1 KiB of contiguous memory.  All loads of a work-item
-// are issued before any arithmetic.  Loads and stores are nontemporal by
-// default: no operand is touched twice, and streaming them past L2/MALL
+// are issued before any arithmetic.  Loads and stores of long arrays are
+// nontemporal: no operand is touched twice, and streaming them past L2/MALL
 // measured 6.4 TB/s for TRIAD at 2^28 against 5.6 TB/s with regular
 // accesses (block 256, one vector per work-item; larger U measured slower).
-// RPX_TUNE_CACHED selects regular accesses.  Arithmetic follows
+// Arrays that the 256 MB MALL holds with a few others are often in it when the
+// next kernel wants them (kStreamFrom).  RPX_TUNE_CACHED selects regular
+// accesses for all.  Arithmetic follows
 // the Base_Seq association with no contraction (TRIAD is b + (alpha*c)
 // rounded twice), so results are bit-identical to Base_Seq.
 #include "rpx_common.hpp"
@@ -138,6 +140,12 @@ int dispatch_u(int items, double* out, const double* x, const double* y, double 
 constexpr int kDefaultBlock = 256;
 constexpr int kDefaultItems = 2;
 
+// Elements from which accesses are nontemporal.  COPY, MUL, ADD and TRIAD in
+// turn on the same arrays, regular against nontemporal: 15.0 / 16.5 us at 10^6
+// elements (launches), 47.7 / 49.3 at 4 10^6, 91.4 / 98.4 at 8 10^6, 208 / 196
+// at 16 10^6.
+constexpr int64_t kStreamFrom = int64_t(12) << 20;
+
 template <int OP>
 int run_stream(double* out, const double* x, const double* y, double alpha, int64_t n,
                const rpx_tuning* tune, void* stream) {
@@ -148,7 +156,7 @@ int run_stream(double* out, const double* x, const double* y, double alpha, int6
   hipStream_t s = as_stream(stream);
   const int bs = tune_or(tune, &rpx_tuning::block_size, kDefaultBlock);
   const int items = tune_or(tune, &rpx_tuning::items_per_thread, kDefaultItems);
-  const bool nt = (tune_flags(tune) & RPX_TUNE_CACHED) == 0;
+  const bool nt = n >= kStreamFrom && (tune_flags(tune) & RPX_TUNE_CACHED) == 0;
   const bool vec_ok = aligned16(out) && aligned16(x) && (!kTwoInputs || aligned16(y));
   if (!vec_ok) {
     int64_t grid = ceil_div(n, 256);
