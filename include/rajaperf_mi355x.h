@@ -209,8 +209,8 @@ size_t rpx_scan_scratch_bytes(int64_t n, const rpx_tuning* tune);
 /* Zeroes a scan scratch buffer; required once before its first use.  Each
  * call then leaves the buffer ready for the next (epoch-tagged flags).  A
  * scratch may be shared with the segmented form below (sized for the larger
- * of the two): the segmented form's flags carry a tag the single-array form
- * never accepts. */
+ * of the two): neither the segmented form's flags nor its tables read as a
+ * flag that the single-array form accepts. */
 int rpx_scan_scratch_init(void* scratch, size_t scratch_bytes, void* stream);
 /* Synchronously reads the scratch's error word: RPX_ERR_WAIT_EXPIRED if a
  * look-back wait of an earlier call gave up, else RPX_SUCCESS. */

@@ -30,6 +30,7 @@
 //  * every spin is bounded; a wait that expires records RPX_ERR_WAIT_EXPIRED
 //    in the scratch header and the kernel still runs to completion.
 #include "rpx_common.hpp"
+#include "scan_words.hpp"
 
 #include <vector>
 
@@ -75,9 +76,6 @@ struct TileWords {
 constexpr int kLowBits = 21;  // of words 1 and 2; word 0 holds the top 22
 constexpr unsigned long long kLowMask = (1ull << kLowBits) - 1;
 
-__device__ __forceinline__ unsigned long long tile_tag(unsigned long long epoch, unsigned status) {
-  return (epoch << 2 | status) << 22;
-}
 __device__ __forceinline__ void store_word(unsigned long long* p, unsigned long long v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -108,13 +106,13 @@ __device__ __forceinline__ void publish(const TileWords& w, int64_t t, unsigned 
 // rewritten); WIDE: *v is its value.
 template <bool WIDE>
 __device__ __forceinline__ unsigned look(const TileWords& w, int64_t k, unsigned long long epoch, double* v) {
-  const unsigned long long a = load_word(&w.w0[k]), tag = a >> 22;
+  const unsigned long long a = load_word(&w.w0[k]);
   if constexpr (WIDE) {
-    const unsigned long long b = load_word(&w.w1[k]), c = load_word(&w.w2[k]);
+    const unsigned long long b = load_word(&w.w1[k]), c = load_word(&w.w2[k]), tag = a >> 22;
     if (b >> 22 != tag || c >> 22 != tag) return 0;
     *v = value((a & 0x3FFFFFull) << (2 * kLowBits) | (b & kLowMask) << kLowBits | (c & kLowMask));
   }
-  return tag >> 2 == epoch ? unsigned(tag & 3) : 0;
+  return tile_status(a, epoch);
 }
 
 // Wavefront scans on DPP lane moves (VALU only, no LDS round trips).  A
@@ -197,9 +195,9 @@ __device__ __forceinline__ double look_window(const TileWords& words, int64_t to
 // after its first reads and writes 16-byte rows; the first tile skips the
 // element before an odd start.
 struct SegTables {
-  const int64_t* off;
-  const int64_t* tile0;
-  const int* tile_seg;
+  const uint64_t* off;       // table_entry
+  const uint64_t* tile0;     // table_entry
+  const uint32_t* tile_seg;  // segment_entry
 };
 
 // SEG = false: one array of n elements, tile t covers [t*T, t*T + T), words
@@ -228,9 +226,9 @@ __global__ __launch_bounds__(BS) void scan_kernel(const double* x, double* y, in
   // elements [lo, tend) of it; first is its segment's first tile.
   int64_t tal, lo, tend, first;
   if (SEG) {
-    const int sg = seg.tile_seg[t];
-    first = seg.tile0[sg];
-    const int64_t sbeg = seg.off[sg], send = seg.off[sg + 1];
+    const int sg = segment_value(seg.tile_seg[t]);
+    first = table_value(seg.tile0[sg]);
+    const int64_t sbeg = table_value(seg.off[sg]), send = table_value(seg.off[sg + 1]);
     tal = (sbeg & ~int64_t(1)) + (t - first) * kTileN;
     lo = sbeg > tal ? sbeg : tal;
     tend = (tal + kTileN < send) ? tal + kTileN : send;
@@ -281,7 +279,8 @@ __global__ __launch_bounds__(BS) void scan_kernel(const double* x, double* y, in
   __syncthreads();
   // Epoch: 0 for the segmented form (its words are cleared before every
   // launch), the header's + 1 for the single-array form, so a single-array scan
-  // never accepts a word a segmented call left in a shared scratch.
+  // never accepts a word or table entry a segmented call left in a shared
+  // scratch.
   const unsigned long long E = SEG ? 0ull : (s_epoch + 1) & 0xFFFFFFFFFFull;
   double wave_off = 0.0, tile_agg = 0.0;
 #pragma unroll
@@ -375,20 +374,21 @@ __global__ void zero_kernel(unsigned* p, int64_t nwords) {
 // (the last segment whose first tile is <= t owns tile t; empty segments
 // share their first tile with the next segment and so are never chosen).
 __global__ __launch_bounds__(256) void seg_prep_kernel(unsigned* __restrict__ words, int64_t nwords,
-                                                       const int64_t* __restrict__ tile0, int nseg,
-                                                       int* __restrict__ tile_seg, int64_t ntiles) {
+                                                       const uint64_t* __restrict__ tile0, int nseg,
+                                                       uint32_t* __restrict__ tile_seg, int64_t ntiles) {
   const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-  const int64_t end = nwords > ntiles ? nwords : ntiles;
+  const int64_t entries = ntiles + (ntiles & 1);  // whole 64 bits
+  const int64_t end = nwords > entries ? nwords : entries;
   for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < end; i += stride) {
     if (i < nwords) words[i] = 0u;
-    if (i < ntiles) {
+    if (i < entries) {
       int a = 0, b = nseg - 1;
       while (a < b) {
         const int mid = (a + b + 1) >> 1;
-        if (tile0[mid] <= i) a = mid;
+        if (table_value(tile0[mid]) <= i) a = mid;
         else b = mid - 1;
       }
-      tile_seg[i] = a;
+      tile_seg[i] = segment_entry(a);
     }
   }
 }
@@ -495,7 +495,7 @@ SegLayout seg_layout(const int64_t* offsets_host, int64_t nseg) {
   g.l = layout_for(g.ntiles > 0 ? g.ntiles : 1);
   g.tab_off = g.l.total;
   g.tile_seg_off = g.tab_off + align256(size_t(2 * (nseg + 1)) * sizeof(int64_t));
-  g.total = g.tile_seg_off + align256(size_t(g.ntiles) * sizeof(int));
+  g.total = g.tile_seg_off + align256(size_t(g.ntiles) * sizeof(uint32_t));
   return g;
 }
 
@@ -544,17 +544,17 @@ int rpx_scan_exclusive_segmented_f64(const double* x, double* y, const int64_t* 
   hipStream_t st = as_stream(stream);
   char* base = reinterpret_cast<char*>(scratch);
   // Tables: the offsets, then each segment's first tile (one copy).
-  std::vector<int64_t> tab(size_t(2 * (nseg + 1)));
+  std::vector<uint64_t> tab(size_t(2 * (nseg + 1)));
   int64_t t = 0;
   for (int64_t s = 0; s <= nseg; ++s) {
-    tab[size_t(s)] = offsets_host[s];
-    tab[size_t(nseg + 1 + s)] = t;
+    tab[size_t(s)] = table_entry(offsets_host[s]);
+    tab[size_t(nseg + 1 + s)] = table_entry(t);
     if (s < nseg) t += seg_tiles(offsets_host[s], offsets_host[s + 1]);
   }
-  auto* d_off = reinterpret_cast<int64_t*>(base + g.tab_off);
+  auto* d_off = reinterpret_cast<uint64_t*>(base + g.tab_off);
   auto* d_tile0 = d_off + (nseg + 1);
-  auto* d_tile_seg = reinterpret_cast<int*>(base + g.tile_seg_off);
-  const HostChunk table{d_off, tab.data(), tab.size() * sizeof(int64_t)};
+  auto* d_tile_seg = reinterpret_cast<uint32_t*>(base + g.tile_seg_off);
+  const HostChunk table{d_off, tab.data(), tab.size() * sizeof(uint64_t)};
   if (const int rc = upload_async(&table, 1, st); rc != RPX_SUCCESS) return rc;
   // The tiles' words start at zero for every call (no epochs across segments).
   char* const tiles = base + g.l.words_off[0];
