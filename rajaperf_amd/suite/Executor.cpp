@@ -108,12 +108,16 @@ const std::map<std::string, std::vector<std::string>>& device_kernels() {
       {"Stream_MUL", {"stream_vec_kernel<1,"}},
       {"Stream_ADD", {"stream_vec_kernel<2,"}},
       {"Stream_TRIAD", {"stream_vec_kernel<3,"}},
-      {"Stream_DOT", {"reduce_kernel<true,"}},
-      {"Algorithm_REDUCE_SUM", {"reduce_kernel<false,"}},
+      {"Stream_DOT", {"reduce_kernel<true,", "small_reduce_kernel<true>"}},
+      {"Algorithm_REDUCE_SUM", {"reduce_kernel<false,", "small_reduce_kernel<false>"}},
       {"Algorithm_SCAN", {"scan_kernel<"}},
-      {"Algorithm_SORT", {"hist_kernel(", "offsets_kernel(", "scatter_kernel("}},
-      {"Polybench_GEMM", {"gemm_mfma_f64_kernel(", "gemm_naive_kernel("}},
-      {"Polybench_JACOBI_2D", {"jacobi_fused_kernel<", "jacobi_vec_kernel<", "jacobi_scalar_kernel("}},
+      {"Algorithm_SORT",
+       {"gather_kernel(", "sample_kernel(", "hist_kernel(", "colscan_kernel(", "scatter_kernel(",
+        "second_level_kernel(", "bucket_kernel<", "overfull_kernel("}},
+      {"Polybench_GEMM", {"gemm_mfma_f64_kernel<", "gemm_naive_kernel("}},
+      {"Polybench_JACOBI_2D",
+       {"jacobi_block_kernel<", "jacobi_wide_kernel<", "jacobi_grid_kernel<", "jacobi_fused_kernel<",
+        "jacobi_stream_kernel<", "jacobi_vec_kernel<", "jacobi_scalar_kernel("}},
       {"Apps_MASS3DPA", {"mass3dpa_kernel<", "mass3dpa_naive_kernel<"}},
       {"Apps_DIFFUSION3DPA", {"diffusion3dpa_kernel<"}},
   };
