@@ -22,6 +22,7 @@
 // complete call leaves all the scratch it used zero: the ticket slots of a
 // later call with another n or tuning (a larger layout reaches into what
 // were partials) start at zero.
+#include "reduce_slots.hpp"
 #include "rpx_common.hpp"
 
 #include <mutex>
@@ -203,11 +204,10 @@ __global__ __launch_bounds__(BS) void reduce_kernel(const double* __restrict__ a
 // ---- short reductions ----------------------------------------------------------
 //
 // Up to kSmallReduce elements: one chunk of 4096 per workgroup, one step, and
-// no tickets.  Every workgroup but the last leaves its partial in a slot of
-// two 64-bit words, each 32 bits of it under a mark, and the last one waits for
-// the marks, takes the words, zeroes them and adds the partials in fixed
-// order.  The others depend on nothing, so the wait ends; it is bounded all
-// the same, and a wait that expired makes the result NaN.  What bounds these
+// no tickets.  Every workgroup but the last leaves its partial in a slot, and
+// the last one waits for them, takes them and adds them in fixed order.  The
+// others depend on nothing, so the wait ends; it is bounded all the same, and a
+// wait that expired makes the result NaN.  What bounds these
 // sizes is the chain after the loads: through the two ticket levels it was
 // two atomics, each queueing behind up to 63 others on its line, and two
 // round trips; here it is one round trip.  DOT of 1M: 9.6 us as 62 workgroups
@@ -216,8 +216,20 @@ __global__ __launch_bounds__(BS) void reduce_kernel(const double* __restrict__ a
 constexpr int kSmallBS = 512, kSmallU = 4;
 constexpr int64_t kSmallChunk = 2 * kSmallBS * kSmallU;  // doubles per workgroup
 constexpr int64_t kSmallReduce = int64_t(1) << 23;
-constexpr unsigned long long kMark = 1ull << 32;
 constexpr unsigned kSpinLimit = 1u << 22;
+
+struct AgentMemory {
+  static __device__ __forceinline__ unsigned long long load(unsigned long long* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  static __device__ __forceinline__ void store(unsigned long long* p, unsigned long long v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  static __device__ __forceinline__ unsigned long long exchange(unsigned long long* p, unsigned long long v) {
+    return __hip_atomic_exchange(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  static __device__ __forceinline__ void pause() { __builtin_amdgcn_s_sleep(1); }
+};
 
 size_t small_bytes(int64_t n) {
   const int64_t m = n < kSmallReduce ? n : kSmallReduce;
@@ -252,32 +264,15 @@ __global__ __launch_bounds__(kSmallBS) void small_reduce_kernel(const double* __
   if ((n & 1) && int(blockIdx.x) == last && threadIdx.x == 0) t += DOT ? a[n - 1] * b[n - 1] : a[n - 1];
   double sum = block_sum<kSmallBS>(t, lds);
   if (int(blockIdx.x) != last) {
-    if (threadIdx.x == 0) {
-      const unsigned long long v = static_cast<unsigned long long>(__double_as_longlong(sum));
-      unsigned long long* s = slots + 2 * int64_t(blockIdx.x);
-      __hip_atomic_store(s, kMark | v >> 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(s + 1, kMark | (v & 0xFFFFFFFFull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (threadIdx.x == 0)
+      slot_leave<AgentMemory>(slots + 2 * int64_t(blockIdx.x), static_cast<unsigned long long>(__double_as_longlong(sum)));
     return;
   }
   double mine = 0.0;
   for (int i = threadIdx.x; i < last; i += kSmallBS) {
-    unsigned long long* s = slots + 2 * int64_t(i);
-    unsigned long long hi, lo;
-    unsigned spins = 0;
-    while (true) {
-      hi = __hip_atomic_load(s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      lo = __hip_atomic_load(s + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if ((hi & lo & kMark) != 0) break;
-      if (++spins > kSpinLimit) {
-        hi = lo = ~0ull;  // a NaN
-        break;
-      }
-      __builtin_amdgcn_s_sleep(1);
-    }
-    __hip_atomic_store(s, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(s + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    mine += __longlong_as_double(static_cast<long long>(hi << 32 | (lo & 0xFFFFFFFFull)));
+    unsigned long long bits;
+    if (!slot_take<AgentMemory>(slots + 2 * int64_t(i), kSpinLimit, &bits)) bits = ~0ull;  // a NaN
+    mine += __longlong_as_double(static_cast<long long>(bits));
   }
   __syncthreads();  // lds
   if (threadIdx.x == 0) mine += sum;
