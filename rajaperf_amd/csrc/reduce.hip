@@ -358,6 +358,11 @@ int run_reduce(const double* a, const double* b, int64_t n, double* result, int 
   if (n < 0 || !result || (n > 0 && (!a || (DOT && !b)))) return RPX_ERR_INVALID_ARGUMENT;
   if (!scratch) return RPX_ERR_INVALID_ARGUMENT;
   if (!aligned16(a) || (DOT && !aligned16(b))) return RPX_ERR_INVALID_ARGUMENT;
+  const int bs = tune_or(tune, &rpx_tuning::block_size, kDefaultBlock);
+  const int items = tune_or(tune, &rpx_tuning::items_per_thread, kDefaultItems);
+  ReduceLayout l;
+  if (!layout_for(n, bs, items, tune, &l)) return RPX_ERR_UNSUPPORTED;
+  if (scratch_bytes < l.total) return RPX_ERR_SCRATCH_TOO_SMALL;
   // A scratch too small for the slots (but not for the tickets) keeps the tickets.
   if (n > 0 && n <= kSmallReduce && untuned(tune) && scratch_bytes >= small_bytes(n)) {
     auto* slots = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(scratch) + kHeaderBytes);
@@ -365,11 +370,6 @@ int run_reduce(const double* a, const double* b, int64_t n, double* result, int 
         a, b, n, slots, result, accumulate);
     return launch_status();
   }
-  const int bs = tune_or(tune, &rpx_tuning::block_size, kDefaultBlock);
-  const int items = tune_or(tune, &rpx_tuning::items_per_thread, kDefaultItems);
-  ReduceLayout l;
-  if (!layout_for(n, bs, items, tune, &l)) return RPX_ERR_UNSUPPORTED;
-  if (scratch_bytes < l.total) return RPX_ERR_SCRATCH_TOO_SMALL;
   const bool nt = (tune_flags(tune) & RPX_TUNE_CACHED) == 0;
   const int u = vec_per_step(items);
   char* base = reinterpret_cast<char*>(scratch);
