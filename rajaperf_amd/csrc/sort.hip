@@ -1050,6 +1050,7 @@ Sizes measure(const int64_t* off, int64_t nseg) {
   s.keys = off[nseg] - off[0];
   s.chunk = chunk_for(s.keys);
   s.uniform = off[0] == 0 && s.keys > 0;
+  long long cut_keys = 0, cut_buckets = 0;  // of the segments that are cut at all
   for (int64_t i = 0; i < nseg; ++i) {
     const long long len = off[i + 1] - off[i];
     if (len != off[1] - off[0]) s.uniform = false;
@@ -1062,16 +1063,23 @@ Sizes measure(const int64_t* off, int64_t nseg) {
     if (g.k > 1) {
       s.l1.cols += ceil_div(g.k, kCol);
       s.l1.counts += (long long)g.rows * g.k;
+      cut_keys += len;
+      cut_buckets += g.k;
     }
   }
   s.l1.segs = s.nseg;
   s.small = s.longest <= Large::kCap;
   s.two_levels = s.longest > kOneLevel;
   if (s.two_levels) {
+    // Only a bucket of more keys than one workgroup sorts is cut again, and
+    // there are few of them: uncut segments and usual buckets have no rows.
+    // (One segment of 3 10^6 keys beside 10^6 of 10: 1100 rows and 0.28 GB of
+    // scratch, where a row for every segment made 10^6 and 3.2 GB.)
+    const long long again = std::min(cut_buckets, cut_keys / (Large::kCap + 1));
     s.l2.segs = s.l1.buckets;
-    s.l2.rows = s.keys / ((long long)s.chunk * kTile) + s.l2.segs;
-    s.l2.buckets = s.keys / kAim + s.l2.segs;
-    s.l2.cols = s.l2.buckets / kCol + s.l2.segs;
+    s.l2.rows = cut_keys / ((long long)s.chunk * kTile) + again;
+    s.l2.buckets = cut_keys / kAim + s.l2.segs;
+    s.l2.cols = (cut_keys / kAim + again) / kCol + again;
     s.l2.counts = s.l2.rows * buckets_for(s.longest, true);
   }
   return s;
