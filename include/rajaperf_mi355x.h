@@ -272,7 +272,7 @@ int rpx_jacobi2d_f64(double* A, double* B, int64_t N, int64_t tsteps,
  * B and the new A, the new A going to `scratch` (an N x N grid) and back, so
  * no launch overwrites values a neighbouring tile still reads.  Ends with the
  * result in A and B, bit-equal to rpx_jacobi2d_f64.  Without a requested shape
- * tile and depth are chosen by N and tsteps, for odd N too.  With
+ * tile (or chunk) and depth are chosen by N and tsteps, for odd N too.  With
  * tune->items_per_thread or tune->depth (1..4, default 3) it runs
  * rpx_jacobi2d_fused_launch_f64's launches of that shape, and the two-sweep
  * path for odd N or pointers that are not 16-byte aligned.  The two-sweep

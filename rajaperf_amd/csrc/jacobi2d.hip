@@ -650,6 +650,19 @@ int sweep(double* dst, const double* src, int64_t N, const rpx_tuning* tune, hip
   }
 }
 
+// Two to six time steps are two launches either way, and on a large grid the
+// memory bounds both: then the streaming chunks, which read a row once on its
+// way down, pass the tiles, which read a halo of 4 x steps rows each, as long as
+// their rows are whole 64-byte lines.  Chunks / tiles in us at 2, 4, 5 and 6
+// steps: N = 8192 543/523, 555/526, 555/545, 571/534; 9472 719/718, 729/728,
+// 732/751, 746/719; 10240 829/841, 845/868, 843/869, 861/831; 16000 1947/2073,
+// 1957/2145, 1949/2134, 1967/2033; 20000 3009/3355, 3029/3278, 3025/3323,
+// 3052/3165.  Other even N: 15500 2040/1936, 10002 912/788.
+bool chunks_are_faster(int64_t N, int64_t tsteps) {
+  if (N % 8 != 0 || tsteps > 6) return false;
+  return N >= (tsteps == 6 ? 15872 : tsteps == 5 ? 8832 : 9856);
+}
+
 }  // namespace
 
 extern "C" {
@@ -694,13 +707,13 @@ int rpx_jacobi2d_fused_f64(double* A, double* B, int64_t N, int64_t tsteps, void
     if (scratch_bytes < rpx_jacobi2d_fused_scratch_bytes(N)) return RPX_ERR_SCRATCH_TOO_SMALL;
   }
   // Without a requested tile or depth the register-resident tiles take every
-  // grid, odd N too, that they have room for: all tested N from 131 to 8192
-  // are faster on them (N = 1002, 40 steps: 82 against 374 us; N = 8192, 50
-  // steps: 2.61 against 3.98 ms).  One time step stays with the two in-place
+  // grid, odd N too, that they have room for (N = 1002, 40 steps: 82 against
+  // 374 us; N = 8192, 50 steps: 2.61 against 3.98 ms), but for few steps on a
+  // large grid (chunks_are_faster).  One time step stays with the two in-place
   // sweeps, which a tile launch and a copy back would not beat.
   const bool untuned = tune_or(tune, &rpx_tuning::items_per_thread, 0) == 0 && tune_or(tune, &rpx_tuning::depth, 0) == 0;
   if (untuned && N <= kJacobiOneTileN) return jacobi_one_tile(A, B, N, tsteps, s);
-  if (untuned && tsteps > 1 && N <= kMaxFusedN && usable)
+  if (untuned && tsteps > 1 && N <= kMaxFusedN && usable && !(vec && chunks_are_faster(N, tsteps)))
     return jacobi_blocks(A, B, reinterpret_cast<double*>(scratch), N, tsteps, s);
   if (!vec) return rpx_jacobi2d_f64(A, B, N, tsteps, tune, stream);
   const int rows_req = tune_or(tune, &rpx_tuning::items_per_thread, 0);
