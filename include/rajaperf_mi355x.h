@@ -62,7 +62,8 @@ typedef struct rpx_tuning {
 #define RPX_TUNE_CACHED            0x1 /* stream/DOT/REDUCE_SUM/SCAN: regular cached
                                            loads and stores instead of the default
                                            nontemporal (streaming) ones, which the
-                                           stream kernels take from 12 Mi elements */
+                                           stream kernels take from 7.5 Mi elements
+                                           and DOT/REDUCE_SUM above 8 Mi */
 #define RPX_TUNE_NAIVE             0x2 /* plain FP64 comparators in the suite's Base_HIP
                                            shape: GEMM one work-item per C element,
                                            MASS3DPA one element per Q x Q workgroup */
@@ -76,6 +77,9 @@ typedef struct rpx_tuning {
                                            textbook C = alpha*A*B + beta*C (each C
                                            read once before it is written) instead of
                                            the suite's C = alpha*A*B */
+#define RPX_TUNE_NONTEMPORAL       0x20 /* stream: nontemporal loads and stores at every
+                                           length, for operands that no cache holds and
+                                           no kernel reads soon; RPX_TUNE_CACHED wins */
 
 /* ---- library / runtime support ---------------------------------------- *
  * Counterparts of the suite's HIP data utilities

@@ -33,6 +33,7 @@ RPX_TUNE_NAIVE = 0x2
 RPX_TUNE_JACOBI_SKIP_B = 0x4
 RPX_TUNE_MASS_SINGLE_LAUNCH = 0x8
 RPX_TUNE_GEMM_BETA = 0x10
+RPX_TUNE_NONTEMPORAL = 0x20
 
 
 class ExtensionMissing(RuntimeError):

@@ -13,8 +13,8 @@
 // measured 6.4 TB/s for TRIAD at 2^28 against 5.6 TB/s with regular
 // accesses (block 256, one vector per work-item; larger U measured slower).
 // Arrays that the 256 MB MALL holds with a few others are often in it when the
-// next kernel wants them (kStreamFrom).  RPX_TUNE_CACHED selects regular
-// accesses for all.  Arithmetic follows
+// next kernel wants them (kStreamFrom).  RPX_TUNE_CACHED selects regular and
+// RPX_TUNE_NONTEMPORAL nontemporal accesses for all.  Arithmetic follows
 // the Base_Seq association with no contraction (TRIAD is b + (alpha*c)
 // rounded twice), so results are bit-identical to Base_Seq.
 #include "rpx_common.hpp"
@@ -140,11 +140,16 @@ int dispatch_u(int items, double* out, const double* x, const double* y, double 
 constexpr int kDefaultBlock = 256;
 constexpr int kDefaultItems = 2;
 
-// Elements from which accesses are nontemporal.  COPY, MUL, ADD and TRIAD in
-// turn on the same arrays, regular against nontemporal: 15.0 / 16.5 us at 10^6
-// elements (launches), 47.7 / 49.3 at 4 10^6, 91.4 / 98.4 at 8 10^6, 208 / 196
-// at 16 10^6.
-constexpr int64_t kStreamFrom = int64_t(12) << 20;
+// Elements from which accesses are nontemporal.  Below, a program's next kernel
+// usually finds these arrays in the caches if they went through them.  Regular
+// against nontemporal, us: the four kernels in turn, each on the last one's
+// output, 14.3 / 16.7 at 10^6 elements, 25.6 / 30.9 at 2 Mi, 50.2 / 58.1 at 4
+// Mi, 107 / 112 at 8 Mi; the four and DOT on the same inputs 25.2 / 29.1 at
+// 10^6, 70.4 / 75.5 at 4 Mi, 140 / 140 at 8 Mi; TRIAD, DOT, REDUCE_SUM and SCAN
+// 55.5 / 59.2 at 4 Mi, 89.3 / 89.5 at 7 Mi, 102 / 98.8 at 8 Mi.  A kernel whose
+// operands no cache holds, and whose output nothing reads soon, pays for it
+// (TRIAD 6.2 / 5.4 at 1 Mi, 19.9 / 17.2 at 4 Mi): RPX_TUNE_NONTEMPORAL is for that.
+constexpr int64_t kStreamFrom = int64_t(15) << 19;
 
 template <int OP>
 int run_stream(double* out, const double* x, const double* y, double alpha, int64_t n,
@@ -156,7 +161,8 @@ int run_stream(double* out, const double* x, const double* y, double alpha, int6
   hipStream_t s = as_stream(stream);
   const int bs = tune_or(tune, &rpx_tuning::block_size, kDefaultBlock);
   const int items = tune_or(tune, &rpx_tuning::items_per_thread, kDefaultItems);
-  const bool nt = n >= kStreamFrom && (tune_flags(tune) & RPX_TUNE_CACHED) == 0;
+  const int flags = tune_flags(tune);
+  const bool nt = (flags & RPX_TUNE_CACHED) == 0 && (n >= kStreamFrom || (flags & RPX_TUNE_NONTEMPORAL) != 0);
   const bool vec_ok = aligned16(out) && aligned16(x) && (!kTwoInputs || aligned16(y));
   if (!vec_ok) {
     int64_t grid = ceil_div(n, 256);
