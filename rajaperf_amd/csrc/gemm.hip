@@ -13,6 +13,7 @@
 //  * gemm_mfma_f64_kernel: v_mfma_f64_16x16x4f64 on workgroup tiles from
 //    128 x 128 to 16 x 16, by size; tiles are mapped XCD-major so neighbouring
 //    tiles that share A rows / B columns run on the same XCD's L2.
+#include <cmath>
 #include <type_traits>
 
 #include "rpx_common.hpp"
@@ -233,6 +234,32 @@ __global__ __launch_bounds__(S::T, 2) void gemm_mfma_f64_kernel(double* __restri
   // of lane l is row 4*r + l/16, column l%16.
   if constexpr (S::WK == 1) {
     const int64_t row0 = m0 + wm + (lane >> 4), col0 = n0 + wn + fr;
+    // A tile inside C of a shape for short K, which the stores bound: without
+    // a test for each element.  (Big has no registers left for it: 4096^2 x
+    // 1024 539 -> 566 us.)
+    if (S::FB == 1 && m0 + S::TM <= ni && n_inside) {
+      double* to = C + row0 * nj + col0;
+#pragma unroll
+      for (int i = 0; i < S::MF; ++i) {
+        double c[S::NF][4];
+        if (use_beta) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int j = 0; j < S::NF; ++j) c[j][r] = to[(i * 16 + 4 * r) * nj + j * 16];
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int j = 0; j < S::NF; ++j) to[(i * 16 + 4 * r) * nj + j * 16] = fma(beta, c[j][r], acc[i][j][r]);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int j = 0; j < S::NF; ++j) to[(i * 16 + 4 * r) * nj + j * 16] = acc[i][j][r];
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < S::MF; ++i) {
       double c[S::NF][4];
@@ -300,6 +327,7 @@ int launch_mfma(double* C, const double* A, const double* B, double alpha, doubl
 // and 96 x 64 are for the sizes between: 1500^3 178 -> 129 us, 1100 x 1100 x
 // 4000 268 -> 244.
 using Big = Shape<2, 2, 4, 4, 1, 32, 2>;     // 128 x 128, sixteen wavefronts
+using Short = Shape<1, 4, 4, 2, 1, 16, 1>;   // 64 x 128, eight wavefronts, two workgroups per CU, for short K
 using Square = Shape<3, 2, 2, 3, 2, 16, 2>;  // 96 x 96, K in two, twelve wavefronts
 using Tall = Shape<3, 2, 2, 2, 2, 16, 2>;    // 96 x 64, K in two, eight wavefronts
 using Mid = Shape<2, 2, 2, 2, 2, 16, 2>;     // 64 x 64, K in two, two workgroups per CU
@@ -318,6 +346,12 @@ double mfma_us(int64_t ni, int64_t nj, int64_t nk, double alone, double shared) 
   return double(ceil_div(nk, S::KS) * S::KS) * (per_k > alone ? per_k : alone);
 }
 
+// The same with what a tile costs besides: its first loads, its stores.
+template <typename S>
+double tiles_us(int64_t ni, int64_t nj, double tile) {
+  return tile * double(ceil_div(ni, S::TM)) * double(ceil_div(nj, S::TN)) / 256.0;
+}
+
 int gemm_mfma(double* C, const double* A, const double* B, double alpha, double beta, int use_beta, int64_t ni,
               int64_t nj, int64_t nk, hipStream_t s) {
   if (__builtin_isinf(alpha)) return launch_mfma<Mid, true>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
@@ -328,6 +362,19 @@ int gemm_mfma(double* C, const double* A, const double* B, double alpha, double 
   int best = 0;
   for (int i = 1; i < 8; ++i)
     if (us[i] < us[best]) best = i;
+  // Short tiles for a C of at least one per CU and K up to 300 or so, where a
+  // tile costs 1.8 us besides its products and one of 128 x 128, alone on its
+  // CU, 7 us: 4096^2 x 64 60.1 -> 51.7 us, x 128 91.5 -> 85.7, 8192^2 x 16
+  // 166 -> 97, 1024 x 2048 x 16 9.5 -> 6.7.
+  const double besides[] = {tiles_us<Big>(ni, nj, 7.0),     tiles_us<Square>(ni, nj, 5.0),
+                            tiles_us<Tall>(ni, nj, 4.1),    tiles_us<Mid>(ni, nj, 2.1),
+                            tiles_us<MidDeep>(ni, nj, 3.7), tiles_us<Small>(ni, nj, 0.54),
+                            tiles_us<SmallDeep>(ni, nj, 0.9), tiles_us<Tiny>(ni, nj, 1.1)};
+  const double n = tiles_us<Short>(ni, nj, 1.0);  // per CU
+  const double rounds = n < 4 ? std::ceil(n) : n < 8 ? n + 0.25 : n;
+  const double short_us = rounds * (double(ceil_div(nk, Short::KS) * Short::KS) * 0.0695 + 1.8);
+  if (ni >= Short::TM && n >= 1 && short_us < 0.98 * (us[best] + besides[best]))
+    return launch_mfma<Short>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
   switch (best) {
     case 0: return launch_mfma<Big>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
     case 1: return launch_mfma<Square>(C, A, B, alpha, beta, use_beta, ni, nj, nk, s);
