@@ -654,13 +654,14 @@ int sweep(double* dst, const double* src, int64_t N, const rpx_tuning* tune, hip
 // memory bounds both: then the streaming chunks, which read a row once on its
 // way down, pass the tiles, which read a halo of 4 x steps rows each, as long as
 // their rows are whole 64-byte lines.  Chunks / tiles in us at 2, 4, 5 and 6
-// steps: N = 8192 543/523, 555/526, 555/545, 571/534; 9472 719/718, 729/728,
-// 732/751, 746/719; 10240 829/841, 845/868, 843/869, 861/831; 16000 1947/2073,
-// 1957/2145, 1949/2134, 1967/2033; 20000 3009/3355, 3029/3278, 3025/3323,
-// 3052/3165.  Other even N: 15500 2040/1936, 10002 912/788.
+// steps, a copy of A before them at N = 8000 and 8192 (675/675, 690/677, 688/701,
+// 698/691; 701/697, 714/700, 714/717, 728/709), none at 9472 (719/718, 729/728,
+// 732/751, 746/719), 10240 (829/841, 845/868, 843/869, 861/831), 16000 (1947/2073,
+// 1957/2145, 1949/2134, 1967/2033) and 20000 (3009/3355, 3029/3278, 3025/3323,
+// 3052/3165).  Other even N: 15500 2040/1936, 10002 912/788.
 bool chunks_are_faster(int64_t N, int64_t tsteps) {
   if (N % 8 != 0 || tsteps > 6) return false;
-  return N >= (tsteps == 6 ? 15872 : tsteps == 5 ? 8832 : 9856);
+  return N >= (tsteps == 6 ? 15872 : tsteps == 5 ? 7680 : 9856);
 }
 
 }  // namespace

@@ -7,7 +7,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("N,tsteps", [(8824, 5), (8832, 5), (9848, 2), (9856, 2), (9856, 3), (9856, 4), (9860, 4),
+@pytest.mark.parametrize("N,tsteps", [(7672, 5), (7680, 5), (8824, 5), (8832, 5), (9848, 2), (9856, 2), (9856, 3), (9856, 4), (9860, 4),
                                       (15872, 6)])
 def test_few_steps_on_a_large_grid(rpx, N, tsteps):
     L, grids = rpx.lib(), []
