@@ -69,7 +69,7 @@ SCAN::SCAN(const RunParams& params) : KernelBase(Algorithm_SCAN, params) {
   setVariantDefined(MI355X_Native);
 }
 void SCAN::setMI355XTuningDefinitions(VariantID vid) {
-  addVariantTuningName(vid, "default");  // 64 doubles per work-item
+  addVariantTuningName(vid, "default");  // 16 doubles per work-item up to 2^22 elements, 64 above
   addVariantTuningName(vid, "items_16");
   addVariantTuningName(vid, "items_32");
   addVariantTuningName(vid, "auto");
@@ -101,7 +101,10 @@ void SCAN::runMI355XVariant(VariantID, size_t tune_idx) {
   if (tune_idx == 3)  // trials write the same y the timed reps will
     tune = Autotuner::instance()
                .choose(getName(), "n=" + std::to_string(n),
-                       {{"default", with_items(64)}, {"items_16", with_items(16)}, {"items_32", with_items(32)}},
+                       {{"default", defaultTuning()},
+                        {"items_16", with_items(16)},
+                        {"items_32", with_items(32)},
+                        {"items_64", with_items(64)}},
                        [&](const rpx_tuning& t) {
                          rpxCheck(rpx_scan_exclusive_f64(m_x, m_y, n, scratch, sb, &t, nullptr), "SCAN");
                        })

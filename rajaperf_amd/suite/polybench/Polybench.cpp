@@ -96,12 +96,12 @@ POLYBENCH_JACOBI_2D::POLYBENCH_JACOBI_2D(const RunParams& params) : KernelBase(P
   setVariantDefined(MI355X_Native);
 }
 void POLYBENCH_JACOBI_2D::setMI355XTuningDefinitions(VariantID vid) {
-  addVariantTuningName(vid, "default");    // three time steps per fused launch (99-row chunks from N = 3072)
+  addVariantTuningName(vid, "default");    // tile or chunk, and time steps per fused launch, by N and tsteps
   addVariantTuningName(vid, "depth_2");    // two time steps per fused launch
   addVariantTuningName(vid, "depth_1");    // one time step per fused launch
   addVariantTuningName(vid, "two_sweep");  // one launch per sweep, as the suite's kernels
   addVariantTuningName(vid, "two_sweep_rows_32");
-  addVariantTuningName(vid, "auto");       // fused depth x tile rows, measured
+  addVariantTuningName(vid, "auto");       // the default and fused depth x tile rows, measured
 }
 void POLYBENCH_JACOBI_2D::setUp(VariantID, size_t) {
   const Size_type nn = Size_type(m_N * m_N);
@@ -143,7 +143,7 @@ void POLYBENCH_JACOBI_2D::runMI355XVariant(VariantID, size_t tune_idx) {
   if (tune_idx == 5) {
     // Trials advance copies of the initial grids, so A and B still start
     // from DATA_SETUP's values when the timed reps begin.
-    std::vector<TuneCandidate> cands;
+    std::vector<TuneCandidate> cands{{"default", defaultTuning()}};
     for (int depth = 1; depth <= 4; ++depth)
       for (int rows : {8, 16, 54, 99, 144}) {
         if (depth == 4 && rows < 54) continue;  // depth 4 runs streaming chunks only
