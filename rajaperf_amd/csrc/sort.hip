@@ -1101,13 +1101,14 @@ Sizes measure(const int64_t* off, int64_t nseg) {
   s.chunk = chunk_for(s.keys);
   s.uniform = off[0] == 0 && s.keys > 0;
   long long cut_keys = 0, cut_buckets = 0;  // of the segments that are cut at all
+  Seg g{};  // the last segment's, which the next usually equals
   for (int64_t i = 0; i < nseg; ++i) {
     const long long len = off[i + 1] - off[i];
     if (len != off[1] - off[0]) s.uniform = false;
     if (len <= 0) continue;
     ++s.nseg;
     s.longest = std::max(s.longest, len);
-    const Seg g = describe(0, len, s.chunk);
+    if (len != g.len) g = describe(0, len, s.chunk);
     s.l1.rows += g.rows;
     s.l1.buckets += g.k;
     if (g.k > 1) {
