@@ -166,11 +166,17 @@ int rpx_triad_f64(double* a, const double* b, const double* c, double alpha,
  * tune->grid_size, when set, caps the workgroup count by lengthening the
  * chunks) and writes one FP64 partial into `scratch`; partials are combined
  * in index order through two ticket levels (groups of 64 workgroups, then
- * the groups).  Results are identical from run to run for a fixed
- * (n, tune).  x (and b for DOT) must be 16-byte aligned.  `scratch` must be
- * zeroed once before its first use (rpx_reduce_scratch_init); every
- * complete call leaves it zero again, so one scratch serves later calls of
- * any n and tuning that fit it. */
+ * the groups).  Without a block_size, items_per_thread or grid_size, up to
+ * 2^23 elements go in chunks of 4096 instead, through regular loads whatever
+ * the flags, and the last workgroup adds the others' partials in a fixed
+ * order as they come; should it wait for one for seconds, the result is a
+ * NaN.  A scratch of less than rpx_reduce_scratch_bytes(n, tune) that fits
+ * the two levels takes them at these lengths too.  Results are identical from
+ * run to run for a fixed (n, tune) and a scratch of at least the queried size
+ * (or always less).  x (and b for DOT) must be 16-byte aligned.  `scratch`
+ * must be zeroed once before its first use (rpx_reduce_scratch_init); every
+ * call leaves it zero again, so one scratch serves later calls of any n and
+ * tuning that fit it. */
 size_t rpx_reduce_scratch_bytes(int64_t n, const rpx_tuning* tune);
 int rpx_reduce_scratch_init(void* scratch, size_t scratch_bytes,
                             void* stream);
@@ -205,9 +211,11 @@ int rpx_reduce_sum_f64(const double* x, int64_t n, double* result,
 /* ---- scan -------------------------------------------------------------- *
  * Exclusive prefix sum y[i] = x[0]+...+x[i-1], y[0] = 0
  * (src/algorithm/SCAN.hpp:27-32, SCAN-Seq.cpp:31-45, SCAN-Hip.cpp:39-326).
- * Single pass with decoupled look-back over tiles of 256 x
- * tune->items_per_thread doubles (16, 32 or 64; default 64); a tile only
- * waits on tiles with lower workgroup ids, which are dispatched before it.
+ * Single pass with decoupled look-back over tiles of tune->block_size x
+ * tune->items_per_thread doubles (256 or 512 by 16, 32 or 64; default 256 x
+ * 16 up to 2^20 elements, 512 x 16 up to 2^22 and 256 x 64 above, where the
+ * scratch has room for so many tiles); a tile only waits on tiles with lower
+ * workgroup ids, which are dispatched before it.
  * The scratch size does not depend on the tuning.  x and y may alias. */
 size_t rpx_scan_scratch_bytes(int64_t n, const rpx_tuning* tune);
 /* Zeroes a scan scratch buffer; required once before its first use.  Each

@@ -117,11 +117,10 @@ __device__ __forceinline__ void mass3dpa_elements(gcdouble* __restrict__ Bg, gcd
 
   // D (P3), X (P1) and Y (P6) pencils go to registers early: D and X before
   // P1, Y at the start of P4 (when D's registers are free), so none of these
-  // loads waits at the head of its stage.  X and Y only for D1D up to 8, and
-  // not at Q = D + 2 from D = 5 nor in the persistent loops (the single-launch
-  // batch kernel and the per-order loop), where the extra live registers cost
-  // a wavefront per SIMD.
-  constexpr bool kPreXY = kEarlyXY && D <= 8 && !(D >= 5 && Q >= D + 2);
+  // loads waits at the head of its stage.  X and Y not at Q = D + 2 from D = 5
+  // nor in the persistent loops (the single-launch batch kernel and the
+  // per-order loop), where the extra live registers cost a wavefront per SIMD.
+  constexpr bool kPreXY = kEarlyXY && !(D >= 5 && Q >= D + 2);
   gcdouble* const xp = Xg + (e0 + w / D2) * D3 + w % D2 * D;  // X[e][dz][dy][:]
   gdouble* const yp = Yg + (e0 + w / D2) * D3 + w % D2;       // Y[e][:][dy][dx]
   double x[D], y[D], dq[Q];
@@ -240,17 +239,17 @@ __global__ __launch_bounds__(kBS) void mass3dpa_kernel(const double* __restrict_
 // chunk0[batch].  A grid of a few workgroups per CU strides over the chunks;
 // each chunk dispatches on its batch's order to the same element code as the
 // single-order kernel, so results are bit-identical to it.
-constexpr int kBatchLds = MassShape<8, 9>::kLds > MassShape<7, 8>::kLds ? MassShape<8, 9>::kLds : MassShape<7, 8>::kLds;  // doubles: the largest kLds over the orders
+// Doubles: the largest kLds over the orders.
+constexpr int kBatchLds = MassShape<8, 9>::kLds > MassShape<7, 8>::kLds ? MassShape<8, 9>::kLds : MassShape<7, 8>::kLds;
 
 typedef __attribute__((address_space(3))) double lds_double;
 
 // One chunk of a batch of order D.  Not inlined: each order's element code
-// keeps its own register allocation (inlined into one kernel the eight
-// orders together needed 256 VGPRs, one wavefront per SIMD); the kernel is
-// bounded to three wavefronts per SIMD, which the LDS allows.  The LDS
-// pointer keeps its address space across the call so its accesses stay LDS
-// instructions.  Measured on 64 batches of orders 2..8 (1.0 M elements):
-// 3.3 ms, against 2.3 ms for one single-order launch per batch.
+// keeps its own register allocation.  The LDS pointer keeps its address space
+// across the call so its accesses stay LDS instructions.  64 batches of orders
+// 2..8 (1.08 M elements): 1.57 ms in this one launch, 1.52 with a
+// single-order launch per batch and 1.28 with a launch per order
+// (mass3dpa_order_chunk_kernel), the default.
 template <int D>
 __device__ __attribute__((noinline)) void mass_batch_chunk(rpx_mass_batch b, int64_t e0, lds_double* lds) {
   using S = MassShape<D, D + 1>;
@@ -372,9 +371,10 @@ __global__ __launch_bounds__(kBS) void mass3dpa_order_kernel(const char* __restr
 
 // The batches of one order with one workgroup per chunk, for a grid of the
 // order's chunk count.  Without the persistent loop around it the element
-// code compiles as in the single-order kernel (164 against 118 VGPRs at
-// D1D = 8, where the looped form waits on each LDS basis read of its last
-// stages and runs 12-15% slower at D1D = 7, 8).
+// code compiles as in the single-order kernel (at D1D = 8 62 VGPRs against 126,
+// eight wavefronts per SIMD against four), and a chunk does not wait for the
+// LDS reads of the one before: 64 batches of D1D = 7 / 8 (0.70 M elements) 1.60
+// / 2.42 ms, 1.80 / 2.66 in the loop on 1024 workgroups.
 template <int D>
 __global__ __launch_bounds__(kBS) void mass3dpa_order_chunk_kernel(const char* __restrict__ plan) {
   using S = MassShape<D, D + 1>;

@@ -269,8 +269,8 @@ constexpr int64_t kChunkRows = 512;
 
 // Both in one launch: B's column exponents need none of A's work, and neither
 // fills the memory by itself.  (On two streams, joined by events, they cost a
-// call 10 us more at 1000 x 1000 x 1200 and no less at 4096^3.)  `chunks` parts of B's rows leave their exponents
-// in part[chunk][njp] for split_cols_kernel.
+// call 10 us more at 1000 x 1000 x 1200 and no less at 4096^3.)  `chunks` parts
+// of B's rows leave their exponents in part[chunk][njp] for split_cols_kernel.
 __global__ __launch_bounds__(256) void prepare_kernel(const double* __restrict__ A, const double* __restrict__ B,
                                                       int64_t ni, int64_t nj, int64_t nk, int64_t nkp, int64_t nip,
                                                       int64_t njp, int64_t chunk_rows, int64_t column_blocks,

@@ -198,11 +198,12 @@ __global__ __launch_bounds__(W* kWave, 4) void jacobi_block_kernel(const BlockAr
 // 256 columns: a lane holds four columns of RW rows, once, and a sweep replaces
 // them in place: half the registers per point, so twice the columns and less
 // halo, and four DPP moves for 20 FP64 instructions instead of 10 (a row and
-// sweep of 256 columns takes 127 clocks, two of 128 columns 128, but 64 of 100
-// points of an 88-row tile are kept at six steps and not 54).  N = 8192: 326 us
-// per launch of 6.25 steps, 165 of which the memory needs and about 225 the
-// FP64 units, in part one after the other: two workgroups per CU are all that
-// the registers hold.  From N = 2000 or so; smaller grids have too few of them.
+// sweep of 256 columns takes 127 clocks, two of 128 columns 128, but 61 of 100
+// points of an 88-row tile are kept at seven steps, 51 of an 80-row narrow one).
+// N = 8192, 50 steps: seven launches of seven or eight steps, about 370 us each,
+// 165 of which the memory needs and about 310 the instructions, in part one
+// after the other: two workgroups per CU are all that the registers hold.  From
+// N = 2000 or so; smaller grids have too few of them.
 // The grid's boundary cells, which the A and the B level have of their own,
 // wait in LDS for the tiles that hold any.
 constexpr int kWideCols = 256;

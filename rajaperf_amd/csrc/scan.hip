@@ -7,8 +7,8 @@
 // ready flags every rep and spins on predecessors indexed by blockIdx.x.
 //
 // MI355X design:
-//  * a tile is 256 work-items x IPT doubles (IPT 16, 32 or 64: 32-128 KiB).
-//    Each wavefront owns a contiguous quarter of the tile and reads it as
+//  * a tile is 256 or 512 work-items x IPT doubles (IPT 16, 32 or 64: 32-256 KiB).
+//    Each wavefront owns a contiguous part of the tile and reads it as
 //    IPT/2 rows of 1 KiB (one 16-byte load per lane per row); it scans the
 //    rows in order in registers -- lane pair sum, a 64-lane scan on DPP row
 //    shifts and row broadcasts, and a running row carry -- so no LDS buffer
@@ -23,10 +23,10 @@
 //    atomic per tile serialises on its single address -- measured 5.5 ms
 //    against 0.8 ms for 2^28 doubles on MI355X.)
 //  * the look-back is done by the whole workgroup where there are few tiles
-//    and by one wavefront where there are many; a tile's words carry a tag (header epoch + 1) so the scratch
-//    needs no clearing between calls.  The last tile advances the epoch after
-//    its look-back: by then every tile has published, so every tile has read
-//    the epoch;
+//    and by one wavefront where there are many; a tile's words carry a tag
+//    (header epoch + 1) so the scratch needs no clearing between calls.  The
+//    last tile advances the epoch after its look-back: by then every tile has
+//    published, so every tile has read the epoch;
 //  * every spin is bounded; a wait that expires records RPX_ERR_WAIT_EXPIRED
 //    in the scratch header and the kernel still runs to completion.
 #include "rpx_common.hpp"
