@@ -62,8 +62,9 @@ typedef struct rpx_tuning {
 #define RPX_TUNE_CACHED            0x1 /* stream/DOT/REDUCE_SUM/SCAN: regular cached
                                            loads and stores instead of the default
                                            nontemporal (streaming) ones, which the
-                                           stream kernels take from 7.5 Mi elements
-                                           and DOT/REDUCE_SUM above 8 Mi */
+                                           stream kernels take from 12 Mi elements
+                                           (ADD and TRIAD from 7.5 Mi) and
+                                           DOT/REDUCE_SUM above 8 Mi */
 #define RPX_TUNE_NAIVE             0x2 /* plain FP64 comparators in the suite's Base_HIP
                                            shape: GEMM one work-item per C element,
                                            MASS3DPA one element per Q x Q workgroup */

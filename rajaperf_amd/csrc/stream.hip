@@ -13,7 +13,7 @@
 // measured 6.4 TB/s for TRIAD at 2^28 against 5.6 TB/s with regular
 // accesses (block 256, one vector per work-item; larger U measured slower).
 // Arrays that the 256 MB MALL holds with a few others are often in it when the
-// next kernel wants them (kStreamFrom).  RPX_TUNE_CACHED selects regular and
+// next kernel wants them (stream_from).  RPX_TUNE_CACHED selects regular and
 // RPX_TUNE_NONTEMPORAL nontemporal accesses for all.  Arithmetic follows
 // the Base_Seq association with no contraction (TRIAD is b + (alpha*c)
 // rounded twice), so results are bit-identical to Base_Seq.
@@ -145,11 +145,13 @@ constexpr int kDefaultItems = 2;
 // against nontemporal, us: the four kernels in turn, each on the last one's
 // output, 14.3 / 16.7 at 10^6 elements, 25.6 / 30.9 at 2 Mi, 50.2 / 58.1 at 4
 // Mi, 107 / 112 at 8 Mi; the four and DOT on the same inputs 25.2 / 29.1 at
-// 10^6, 70.4 / 75.5 at 4 Mi, 140 / 140 at 8 Mi; TRIAD, DOT, REDUCE_SUM and SCAN
-// 55.5 / 59.2 at 4 Mi, 89.3 / 89.5 at 7 Mi, 102 / 98.8 at 8 Mi.  A kernel whose
-// operands no cache holds, and whose output nothing reads soon, pays for it
-// (TRIAD 6.2 / 5.4 at 1 Mi, 19.9 / 17.2 at 4 Mi): RPX_TUNE_NONTEMPORAL is for that.
-constexpr int64_t kStreamFrom = int64_t(15) << 19;
+// 10^6, 70.4 / 75.5 at 4 Mi, 140 / 140 at 8 Mi.  With two inputs the caches hold
+// less of the next kernel's: TRIAD, DOT, REDUCE_SUM and SCAN 55.5 / 59.2 at 4
+// Mi, 89.3 / 89.5 at 7 Mi, 102 / 98.8 at 8 Mi.  COPY and a kernel that reads the
+// copy: JACOBI_2D, two steps of 9 10^6 points, 93 / 106.  A kernel whose operands
+// no cache holds, and whose output nothing reads soon, pays for it (TRIAD 6.2 /
+// 5.4 at 1 Mi, 19.9 / 17.2 at 4 Mi): RPX_TUNE_NONTEMPORAL is for that.
+constexpr int64_t stream_from(bool two_inputs) { return two_inputs ? int64_t(15) << 19 : int64_t(12) << 20; }
 
 template <int OP>
 int run_stream(double* out, const double* x, const double* y, double alpha, int64_t n,
@@ -162,7 +164,7 @@ int run_stream(double* out, const double* x, const double* y, double alpha, int6
   const int bs = tune_or(tune, &rpx_tuning::block_size, kDefaultBlock);
   const int items = tune_or(tune, &rpx_tuning::items_per_thread, kDefaultItems);
   const int flags = tune_flags(tune);
-  const bool nt = (flags & RPX_TUNE_CACHED) == 0 && (n >= kStreamFrom || (flags & RPX_TUNE_NONTEMPORAL) != 0);
+  const bool nt = (flags & RPX_TUNE_CACHED) == 0 && (n >= stream_from(kTwoInputs) || (flags & RPX_TUNE_NONTEMPORAL) != 0);
   const bool vec_ok = aligned16(out) && aligned16(x) && (!kTwoInputs || aligned16(y));
   if (!vec_ok) {
     int64_t grid = ceil_div(n, 256);

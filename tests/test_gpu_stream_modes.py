@@ -9,10 +9,11 @@ from rajaperf_amd.suite import run_suite
 
 pytestmark = pytest.mark.gpu
 
-FROM = 15 << 19
+FROM = 15 << 19   # two inputs
+FROM1 = 12 << 20  # one
 
 
-@pytest.mark.parametrize("n", [1, 513, 100_003, FROM - 1, FROM, FROM + 1])
+@pytest.mark.parametrize("n", [1, 513, 100_003, FROM - 1, FROM, FROM + 1, FROM1 - 1, FROM1])
 def test_streams_in_every_mode(rpx, rng, n):
     L = rpx.lib()
     a, b = rng.random(n), rng.random(n)
